@@ -188,12 +188,59 @@ __device__ __forceinline__ uint64_t near_mask(const Ed* L, int base, int n, doub
   return cand;
 }
 
+// The geography distances of the reported rows, put off to a kernel of their own. A pair's distance is the minimum of
+// the geography distances of the edge pairs that could hold it: a few of them per pair, each thousands of FP64
+// operations. Evaluated where they are found, one or two lanes of a group worked while its others waited; queued, they
+// fill whole waves (k_geog_items), and the pair kernels are left with the frame tests (300k parcels, 5 m self dwithin
+// with distances: the pair kernels 20.0 -> 4.7 ms and 1.1 ms for the items). The minimum does not depend on the
+// order, so the distances are the same bits. The queue is cut into segments, one counter each, so that the blocks do
+// not all append through one address; items that find their segment full are evaluated in place.
+struct DistQueue {
+  double* c = nullptr;        // [8][nseg * seg] the item's arc a0, a1 and arc b0, b1 (x, y each, degrees)
+  uint32_t* pair = nullptr;   // [nseg * seg] its candidate
+  uint32_t* count = nullptr;  // [nseg] items appended (may exceed seg: the rest were evaluated in place)
+  uint32_t nseg = 0, seg = 0;
+};
+__device__ __forceinline__ bool dq_push(const DistQueue& q, uint32_t p, double a0x, double a0y, double a1x, double a1y, double b0x, double b0y,
+                                        double b1x, double b1y) {
+  const uint32_t s = blockIdx.x % q.nseg, k = atomicAdd(&q.count[s], 1u);
+  if (k >= q.seg) return false;
+  const uint64_t n = (uint64_t)q.nseg * q.seg, i = (uint64_t)s * q.seg + k;
+  q.c[i] = a0x; q.c[n + i] = a0y; q.c[2 * n + i] = a1x; q.c[3 * n + i] = a1y;
+  q.c[4 * n + i] = b0x; q.c[5 * n + i] = b0y; q.c[6 * n + i] = b1x; q.c[7 * n + i] = b1y;
+  q.pair[i] = p;
+  return true;
+}
+
+__global__ void k_dq_clear(uint32_t* count) { count[threadIdx.x] = 0u; }
+
+// a thread per queued item: dist[pair] = min(dist[pair], its geography distance). Distances are not negative, so their
+// bit patterns compare as they do (a NaN compares above every number and is left out, as fmin does).
+__global__ void __launch_bounds__(256) k_geog_items(const DistQueue q, int b_is_point, double* __restrict__ dist) {
+  const uint32_t s = blockIdx.x % q.nseg, per = gridDim.x / q.nseg;   // the grid is a multiple of the segments
+  const uint64_t n = (uint64_t)q.nseg * q.seg, first = (uint64_t)s * q.seg;
+  const uint32_t m = min(q.count[s], q.seg);
+  for (uint32_t k = (blockIdx.x / q.nseg) * blockDim.x + threadIdx.x; k < m; k += per * blockDim.x) {
+    const uint64_t i = first + k;
+    const double v = geo::geog_dist_of(q.c[i], q.c[n + i], q.c[2 * n + i], q.c[3 * n + i], q.c[4 * n + i], q.c[5 * n + i], q.c[6 * n + i],
+                                       q.c[7 * n + i], b_is_point != 0);
+    atomicMin(reinterpret_cast<unsigned long long*>(dist) + q.pair[i], (unsigned long long)__double_as_longlong(v));
+  }
+}
+
 // One piece pair on a lane group (buffer.cuh:185-237). Returns 1 / 0, or -1 when a side has more than cap edges in
-// the window (need = edges required). With report and a hit, dist = the pair's distance (see the file comment).
+// the window (need = edges required). With report and a hit, dist = the pair's distance (see the file comment), before
+// the items queued for candidate p are taken into it.
 // REC: both pieces have packed records with at most PER * G stored vertices, read instead of the layer's arrays.
-template <int G, bool REC, int PER = 1>
-__device__ int dw_eval(const DPolys& P, const DPolys& R, uint32_t a, uint32_t b, double d, bool report, Ed* LA, Ed* LB, int cap, int gl,
-                       double& dist, int& need) {
+// GEO false: the pair is left undecided (-2) where an edge pair inside the error band would decide it, or where the
+// item queue is full; the caller sends it to a GEO kernel. Inside the band are the edge pairs within a fraction of a
+// millimetre of d for edges of some 100 m, so few pairs go, and a kernel without the call of geog_dist needs half the
+// registers.
+// sel (or null): a word per A edge and 64 B edges where the first pass leaves the edge pairs that can still hold the
+// minimum, so that the second looks at those alone (the box tests of the lists and most distances are not repeated).
+template <int G, bool REC, bool GEO, int PER = 1>
+__device__ int dw_eval(const DPolys& P, const DPolys& R, uint32_t a, uint32_t b, double d, bool report, const DistQueue& dq, uint32_t p, Ed* LA,
+                       Ed* LB, int cap, uint64_t* sel, int gl, double& dist, int& need) {
   RecView VA{}, VB{};
   if constexpr (REC) { VA = rec_view(P, a); VB = rec_view(R, b); }
   const double2 oa = REC ? VA.o : P.origin[a], ob = REC ? VB.o : R.origin[b], ea = REC ? VA.e : P.ext[a], eb = REC ? VB.e : R.ext[b];
@@ -210,7 +257,8 @@ __device__ int dw_eval(const DPolys& P, const DPolys& R, uint32_t a, uint32_t b,
   wave_lds_sync();
   const geo::Frame F = geo::frame_of(oa.y + ov.y0, oa.y + ov.y1);   // metric frame of the pair's window
   const double kx = F.kx, ky = F.ky;
-  bool hit = false, cross = false;
+  const int words = (cap + 63) / 64;   // of sel, per A edge
+  bool hit = false, cross = false, open = false;   // open: an edge pair inside the band was left undecided
   double m_up = INFINITY;
   // A's edges G at a time, the group stopping together once the pair is settled: a hit anywhere settles "within" (and,
   // without report, the row); with report, a crossing anywhere settles the distance (0), so the remaining edge pairs
@@ -223,7 +271,7 @@ __device__ int dw_eval(const DPolys& P, const DPolys& R, uint32_t a, uint32_t b,
       const double bx0 = fmin(e.x0, e.x1) - gx, bx1 = fmax(e.x0, e.x1) + gx, by0 = fmin(e.y0, e.y1) - gy, by1 = fmax(e.y0, e.y1) + gy;
       const double ux = (e.x1 - e.x0) * kx, uy = (e.y1 - e.y0) * ky, La2 = ux * ux + uy * uy;
       for (int base = 0; base < nb && !cross && (report || !hit); base += 64) {
-        uint64_t cand = near_mask(LB, base, nb, bx0, bx1, by0, by1);
+        uint64_t cand = near_mask(LB, base, nb, bx0, bx1, by0, by1), keep = 0;
         while (cand != 0) {
           const int j = base + __builtin_ctzll(cand);
           cand &= cand - 1;
@@ -237,18 +285,27 @@ __device__ int dw_eval(const DPolys& P, const DPolys& R, uint32_t a, uint32_t b,
           const double band = geo::geog_band(d, F, La2, vx * vx + vy * vy);
           const double dlo = d - band, dhi = d + band;
           if (d2 <= dlo * dlo) hit = true;
-          else if (!hit && d2 <= dhi * dhi &&   // (with report, a lane already within d needs no geography distance here)
-                   geo::geog_dist(oa.x + e.x0, oa.y + e.y0, oa.x + e.x1, oa.y + e.y1, oa.x + f.x0, oa.y + f.y0, oa.x + f.x1, oa.y + f.y1, false) <= d)
-            hit = true;
-          if (report) m_up = fmin(m_up, sqrt(d2) + band);
-          else if (hit) break;
+          else if (!hit && d2 <= dhi * dhi) {   // (with report, a lane already within d needs no geography distance here)
+            if constexpr (GEO)
+              hit = geo::geog_dist(oa.x + e.x0, oa.y + e.y0, oa.x + e.x1, oa.y + e.y1, oa.x + f.x0, oa.y + f.y0, oa.x + f.x1, oa.y + f.y1, false) <= d;
+            else open = true;
+          }
+          if (report) {
+            const double df = sqrt(d2);
+            m_up = fmin(m_up, df + band);
+            if (!(df - band > m_up)) keep |= 1ull << (j - base);   // m_up only falls: what is left out here stays out
+          } else if (hit) break;
         }
+        if (report && sel) sel[i * words + base / 64] = keep;
       }
+    } else if (report && sel && i < na) {
+      for (int base = 0; base < nb; base += 64) sel[i * words + base / 64] = 0;   // a synthetic edge holds nothing
     }
     if (gany<G>(report ? cross : hit)) break;
   }
   hit = gany<G>(hit);
   cross = gany<G>(cross);
+  if (!GEO && !hit && gany<G>(open)) return -2;
   bool contained = false;
   if (!hit || report) {
     // no boundary within d: within d iff one contains the other (a real vertex of one inside the other piece)
@@ -290,13 +347,14 @@ __device__ int dw_eval(const DPolys& P, const DPolys& R, uint32_t a, uint32_t b,
       // minimum geography distance over the edge pairs whose frame distance could hold it
       const double m = group_min<G>(m_up);
       double best = INFINITY;
+      open = false;
       for (int i = gl; i < na; i += G) {
         const Ed e = LA[i];
         if (e.syn) continue;
-        const double bx0 = fmin(e.x0, e.x1) - gx, bx1 = fmax(e.x0, e.x1) + gx, by0 = fmin(e.y0, e.y1) - gy, by1 = fmax(e.y0, e.y1) + gy;
         const double ux = (e.x1 - e.x0) * kx, uy = (e.y1 - e.y0) * ky, La2 = ux * ux + uy * uy;
         for (int base = 0; base < nb; base += 64) {
-          uint64_t cand = near_mask(LB, base, nb, bx0, bx1, by0, by1);
+          uint64_t cand = sel ? sel[i * words + base / 64]
+                              : near_mask(LB, base, nb, fmin(e.x0, e.x1) - gx, fmax(e.x0, e.x1) + gx, fmin(e.y0, e.y1) - gy, fmax(e.y0, e.y1) + gy);
           while (cand != 0) {
             const int j = base + __builtin_ctzll(cand);
             cand &= cand - 1;
@@ -305,11 +363,17 @@ __device__ int dw_eval(const DPolys& P, const DPolys& R, uint32_t a, uint32_t b,
             const double vx = (f.x1 - f.x0) * kx, vy = (f.y1 - f.y0) * ky;
             const double band = geo::geog_band(d, F, La2, vx * vx + vy * vy);
             if (sqrt(d2) - band > m) continue;
-            best = fmin(best, geo::geog_dist(oa.x + e.x0, oa.y + e.y0, oa.x + e.x1, oa.y + e.y1, oa.x + f.x0, oa.y + f.y0, oa.x + f.x1, oa.y + f.y1,
-                                             false));
+            if (!dq_push(dq, p, oa.x + e.x0, oa.y + e.y0, oa.x + e.x1, oa.y + e.y1, oa.x + f.x0, oa.y + f.y0, oa.x + f.x1, oa.y + f.y1)) {
+              if constexpr (GEO)
+                best = fmin(best, geo::geog_dist(oa.x + e.x0, oa.y + e.y0, oa.x + e.x1, oa.y + e.y1, oa.x + f.x0, oa.y + f.y0, oa.x + f.x1, oa.y + f.y1,
+                                                 false));
+              else open = true;
+            }
           }
         }
       }
+      // (items queued before the queue was full stay: the GEO kernel finds the same distances and takes the minimum)
+      if (!GEO && gany<G>(open)) return -2;
       dist = group_min<G>(best);
     }
   }
@@ -327,6 +391,7 @@ struct DwArgs {
   // batched requests: candidate p belongs to request r when seg[r] <= p < seg[r + 1], distance ds.d[r]
   const uint64_t* seg;
   DistSet ds;
+  DistQueue dq;   // with report
 };
 __device__ __forceinline__ double pair_distance(const DwArgs& A, uint32_t p) {
   if (!A.seg) return A.d;
@@ -344,17 +409,20 @@ __device__ __forceinline__ bool self_piece_pair(const DwArgs& A, uint32_t a, uin
 
 // list classes: a G-lane group per pair, CAP-edge LDS lists per side; class `which` (PairClass) of the partition;
 // pairs whose lists overflow are queued. REC: the class's pieces have packed records (tiny, small, medium: at most CAP
-// stored vertices each), read instead of the layer's arrays.
-template <int G, int CAP, bool REC>
-__global__ void __launch_bounds__(256) k_dw_lists(const DwArgs A, const uint32_t* __restrict__ list, const uint32_t* __restrict__ counts, int which,
-                                                  uint32_t* __restrict__ ovf_list, OverflowCtl* ctl) {
+// stored vertices each), read instead of the layer's arrays. Pairs left undecided go to `open_list`; with GEO the kernel
+// decides those (list = the open pairs, open_ctl their number).
+template <int G, int CAP, bool REC, bool GEO>
+__global__ void __launch_bounds__(256, GEO ? 2 : 3) k_dw_lists(const DwArgs A, const uint32_t* __restrict__ list, const uint32_t* __restrict__ counts, int which,
+                                                  uint32_t* __restrict__ ovf_list, OverflowCtl* ctl, uint32_t* __restrict__ open_list,
+                                                  OverflowCtl* open_ctl) {
   __shared__ Ed lds[256 / G][2 * CAP];
+  __shared__ uint64_t sels[256 / G][CAP * ((CAP + 63) / 64)];
   const int gpb = blockDim.x / G;
   const int gib = threadIdx.x / G, gl = threadIdx.x % G;
   Ed* LA = lds[gib];
   Ed* LB = LA + CAP;
-  const uint32_t n = counts[which];
-  const uint32_t* L = list + class_first(counts, which);
+  const uint32_t n = GEO ? open_ctl->count : counts[which];
+  const uint32_t* L = GEO ? list : list + class_first(counts, which);
   PairStream ps(L, A.pa, A.pb, n, blockIdx.x * gpb + gib, gridDim.x * gpb);
   for (; ps.k < n; ps.advance()) {
     ps.prefetch();
@@ -365,9 +433,11 @@ __global__ void __launch_bounds__(256) k_dw_lists(const DwArgs A, const uint32_t
     }
     double dist = NAN;
     int need = 0;
-    const int r = dw_eval<G, REC, CAP / G>(A.P, A.R, a, b, pair_distance(A, p), A.report != 0, LA, LB, CAP, gl, dist, need);
+    const int r = dw_eval<G, REC, GEO, CAP / G>(A.P, A.R, a, b, pair_distance(A, p), A.report != 0, A.dq, p, LA, LB, CAP, sels[gib], gl,
+                                                dist, need);
     if (gl == 0) {
-      if (r < 0) queue_overflow(p, need, ovf_list, ctl);
+      if (r == -2) queue_overflow(p, 0, open_list, open_ctl);
+      else if (r < 0) queue_overflow(p, need, ovf_list, ctl);
       else {
         A.hit[p] = (uint8_t)r;
         if (A.dist) A.dist[p] = r ? dist : NAN;
@@ -377,86 +447,190 @@ __global__ void __launch_bounds__(256) k_dw_lists(const DwArgs A, const uint32_t
   }
 }
 
-// overflow: a wave per pair, lists in a per-wave slab of global memory
-__global__ void __launch_bounds__(256) k_dw_overflow(const DwArgs A, const uint32_t* __restrict__ list, uint32_t n, int cap, Ed* __restrict__ slab) {
+// overflow: a wave per pair. IN_LDS: lists of up to cap edges in LDS, the queue's length read on the device (a launch
+// right behind the kernels that fill it, on their stream, so that the long pairs run beside the other classes: 300k
+// parcels, 5 m: 0.76 ms that followed them); pairs with longer lists are handed on to `defer` (counted in ctl->pad0).
+// Otherwise the lists are in a per-wave slab of global memory.
+constexpr int DW_OVF_CAP = 448;   // 35 KiB of lists: four waves per CU
+template <bool IN_LDS>
+__global__ void __launch_bounds__(IN_LDS ? 64 : 256) k_dw_overflow(const DwArgs A, const uint32_t* __restrict__ list, uint32_t n, int cap,
+                                                                   Ed* __restrict__ slab, OverflowCtl* ctl, uint32_t* __restrict__ defer_list,
+                                                                   OverflowCtl* defer) {
+  extern __shared__ __align__(16) unsigned char smem[];
   const int wpb = blockDim.x / 64;
   const int wib = threadIdx.x / 64, gl = threadIdx.x % 64;
   const uint64_t wave = (uint64_t)blockIdx.x * wpb + wib;
-  Ed* LA = slab + wave * 2 * (uint64_t)cap;
+  Ed* LA = IN_LDS ? reinterpret_cast<Ed*>(smem) : slab + wave * 2 * (uint64_t)cap;
   Ed* LB = LA + cap;
+  if (IN_LDS) n = ctl->count;
   for (uint32_t k = (uint32_t)wave; k < n; k += gridDim.x * wpb) {
     const uint32_t p = list[k];
     double dist = NAN;
     int need = 0;
-    const int r = dw_eval<64, false>(A.P, A.R, A.pa[p], A.pb[p], pair_distance(A, p), A.report != 0, LA, LB, cap, gl, dist, need);
+    const int r = dw_eval<64, false, true>(A.P, A.R, A.pa[p], A.pb[p], pair_distance(A, p), A.report != 0, A.dq, p, LA, LB, cap, nullptr, gl, dist, need);
     if (gl == 0) {
-      A.hit[p] = r > 0 ? 1 : 0;
-      if (A.dist) A.dist[p] = r > 0 ? dist : NAN;
+      if (r < 0) { queue_overflow(p, need, defer_list, defer); atomicAdd(&ctl->pad0, 1u); }   // (the slab's lists hold what was needed)
+      else {
+        A.hit[p] = r > 0 ? 1 : 0;
+        if (A.dist) A.dist[p] = r > 0 ? dist : NAN;
+      }
     }
     wave_lds_sync();
   }
 }
 
-// thread per (point, piece): inside the piece, or within d of its real boundary (buffer.cuh:1018-1049); with report,
-// the distance (0 inside, else the minimum geography distance over the edges that could hold it)
+// (point, piece) candidates of the point dwithin: inside the piece, or within d of its real boundary (buffer.cuh:
+// 1018-1049); with report, the distance (0 inside, else the minimum geography distance over the edges that could hold
+// it, queued). PtFrame: the candidate's frame, and the box around the point outside which an edge can neither be within
+// d nor hold the minimum: it is farther than d and four times the widest band of the piece (the band of an edge as long
+// as its extent's diagonal), while the distance of a row is at most d, and m_up at most d and two bands. Only the edges
+// near the point pay for the distance (a division each).
+struct PtFrame {
+  double2 pt, o;
+  double px, py, ox, bx0, bx1, by0, by1;
+  geo::Frame F;
+  __device__ __forceinline__ PtFrame(const double2 p, const double2 origin, const double2 ext, double d) : pt(p), o(origin) {
+    px = pt.x - o.x; py = pt.y - o.y;
+    const double reach = d / geo::KY_MIN;   // latitude the closest boundary point can be from the point
+    F = geo::frame_of(pt.y - reach, pt.y + reach);
+    ox = (o.x - o.x) - 1.0;
+    const double exm = ext.x * F.kx, eym = ext.y * F.ky, far = d + 4.0 * geo::geog_band(d, F, exm * exm + eym * eym, 0.0);
+    const double nx = far / fabs(F.kx), ny = far / fabs(F.ky);
+    bx0 = px - nx; bx1 = px + nx; by0 = py - ny; by1 = py + ny;
+  }
+  __device__ __forceinline__ bool near(const double2 u, const double2 v) const {
+    return !(fmax(u.x, v.x) < bx0 || fmin(u.x, v.x) > bx1 || fmax(u.y, v.y) < by0 || fmin(u.y, v.y) > by1);
+  }
+  __device__ __forceinline__ void dist2(const double2 u, const double2 v, double d, double& d2, double& band) const {
+    d2 = geo::pt_seg_d2(px * F.kx, py * F.ky, u.x * F.kx, u.y * F.ky, v.x * F.kx, v.y * F.ky);
+    const double ex = (v.x - u.x) * F.kx, ey = (v.y - u.y) * F.ky;
+    band = geo::geog_band(d, F, ex * ex + ey * ey, 0.0);
+  }
+  __device__ __forceinline__ double geog(const double2 u, const double2 v) const {
+    return geo::geog_dist(o.x + u.x, o.y + u.y, o.x + v.x, o.y + v.y, pt.x, pt.y, pt.x, pt.y, true);
+  }
+  __device__ __forceinline__ bool push(const DistQueue& dq, uint32_t p, const double2 u, const double2 v) const {
+    return dq_push(dq, p, o.x + u.x, o.y + u.y, o.x + v.x, o.y + v.y, pt.x, pt.y, pt.x, pt.y);
+  }
+  __device__ __forceinline__ bool crosses(const double2 u, const double2 v) const {   // parity step of the row left of the point
+    if ((u.y > py) == (v.y > py) && u.y != py && v.y != py) return false;
+    const bool so = left_of(u.x, u.y, v.x, v.y, ox, py), sp = left_of(u.x, u.y, v.x, v.y, px, py);
+    if (so == sp) return false;
+    const bool su = orient(ox, py, px, py, u.x, u.y) > 0, sv = orient(ox, py, px, py, v.x, v.y) > 0;
+    return su != sv;
+  }
+};
+
+// A thread per candidate, for pieces of at most one edge chunk. Longer pieces, candidates that only an edge inside the
+// error band would put within d and those whose items find the queue full go to k_pt_dwithin_wave (open_list): one
+// thread on a piece of 256 edges, or on a few calls of geog_dist, outlasts the whole launch. 200k points within 25 m of
+// 154k parcels with distances: 1486 us as one thread per candidate that did all of it, now 294 + 70 (waves) + 72 us (items).
 __global__ void __launch_bounds__(256) k_pt_dwithin(const DPoints pts, const DPolys R, const uint32_t* __restrict__ pa,
                                                     const uint32_t* __restrict__ pb, uint64_t np, double d, int report, uint8_t* __restrict__ hit,
-                                                    double* __restrict__ dist) {
+                                                    double* __restrict__ dist, const DistQueue dq, uint32_t* __restrict__ open_list,
+                                                    OverflowCtl* open_ctl) {
   const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= np) return;
   const uint32_t g = pb[i];
-  const double2 pt = pts.xy[pa[i]], o = R.origin[g];
-  const double px = pt.x - o.x, py = pt.y - o.y;
-  const double reach = d / geo::KY_MIN;   // latitude the closest boundary point can be from the point
-  const geo::Frame F = geo::frame_of(pt.y - reach, pt.y + reach);
-  const double kx = F.kx, ky = F.ky;
-  const double ox = (o.x - o.x) - 1.0;
-  bool par = false, h = false;
+  if (R.cfirst && R.cfirst[g] != NO_CHUNKS) { queue_overflow((uint32_t)i, 0, open_list, open_ctl); return; }
+  const PtFrame f(pts.xy[pa[i]], R.origin[g], R.ext[g], d);
+  bool par = false, h = false, open = false;
   double m_up = INFINITY;
-  const uint32_t r1 = R.gro[g + 1];
-  for (uint32_t r = R.gro[g]; r < r1 && (report || !h); r++) {
+  const uint32_t r0 = R.gro[g], r1 = R.gro[g + 1];
+  for (uint32_t r = r0; r < r1 && (report || !h); r++) {
     const uint64_t s0 = R.rvo[r], e = R.rvo[r + 1];
+    if (s0 == e) continue;
     double2 v0 = R.xy[s0];
     for (uint64_t j = s0 + 1; j < e && (report || !h); j++) {
       const double2 v1 = R.xy[j];
-      const double x0 = v0.x, y0 = v0.y, x1 = v1.x, y1 = v1.y;
-      if (!syn_bit(R.synb, j - 1)) {
-        const double d2 = geo::pt_seg_d2(px * kx, py * ky, x0 * kx, y0 * ky, x1 * kx, y1 * ky);
-        const double ex = (x1 - x0) * kx, ey = (y1 - y0) * ky;
-        const double band = geo::geog_band(d, F, ex * ex + ey * ey, 0.0), dlo = d - band, dhi = d + band;
-        if (d2 <= dlo * dlo || (d2 <= dhi * dhi && geo::geog_dist(o.x + x0, o.y + y0, o.x + x1, o.y + y1, pt.x, pt.y, pt.x, pt.y, true) <= d)) h = true;
+      if (f.near(v0, v1) && !syn_bit(R.synb, j - 1)) {
+        double d2, band;
+        f.dist2(v0, v1, d, d2, band);
+        const double dlo = d - band, dhi = d + band;
+        if (d2 <= dlo * dlo) h = true;
+        else if (d2 <= dhi * dhi) open = true;
         if (report) m_up = fmin(m_up, sqrt(d2) + band);
       }
-      if (!((y0 > py) == (y1 > py) && y0 != py && y1 != py)) {
-        const bool so = left_of(x0, y0, x1, y1, ox, py), sp = left_of(x0, y0, x1, y1, px, py);
-        if (so != sp) {
-          const bool su = orient(ox, py, px, py, x0, y0) > 0, sv = orient(ox, py, px, py, x1, y1) > 0;
-          if (su != sv) par = !par;
-        }
-      }
+      if (f.crosses(v0, v1)) par = !par;
       v0 = v1;
     }
   }
   const bool within = h || par;
+  if (!within && open) { queue_overflow((uint32_t)i, 0, open_list, open_ctl); return; }
   hit[i] = within ? 1 : 0;
   if (!dist) return;
-  if (!within) { dist[i] = NAN; return; }
-  if (par) { dist[i] = 0.0; return; }
-  double best = INFINITY;
-  for (uint32_t r = R.gro[g]; r < r1; r++) {
+  if (!within || par) { dist[i] = within ? 0.0 : NAN; return; }
+  dist[i] = INFINITY;   // the queued items lower it
+  for (uint32_t r = r0; r < r1; r++) {
     const uint64_t s0 = R.rvo[r], e = R.rvo[r + 1];
+    if (s0 == e) continue;
+    double2 v0 = R.xy[s0];
     for (uint64_t j = s0 + 1; j < e; j++) {
-      if (syn_bit(R.synb, j - 1)) continue;
-      const double2 v0 = R.xy[j - 1], v1 = R.xy[j];
-      const double d2 = geo::pt_seg_d2(px * kx, py * ky, v0.x * kx, v0.y * ky, v1.x * kx, v1.y * ky);
-      const double ex = (v1.x - v0.x) * kx, ey = (v1.y - v0.y) * ky;
-      const double band = geo::geog_band(d, F, ex * ex + ey * ey, 0.0);
-      if (sqrt(d2) - band > m_up) continue;
-      best = fmin(best, geo::geog_dist(o.x + v0.x, o.y + v0.y, o.x + v1.x, o.y + v1.y, pt.x, pt.y, pt.x, pt.y, true));
+      const double2 v1 = R.xy[j];
+      if (f.near(v0, v1) && !syn_bit(R.synb, j - 1)) {
+        double d2, band;
+        f.dist2(v0, v1, d, d2, band);
+        // (items queued before the queue was full stay: the wave finds the same distances and takes the minimum)
+        if (!(sqrt(d2) - band > m_up) && !f.push(dq, (uint32_t)i, v0, v1)) { queue_overflow((uint32_t)i, 0, open_list, open_ctl); return; }
+      }
+      v0 = v1;
     }
   }
-  dist[i] = best;
 }
+
+// The candidates left open, a wave each (their number read on the device): the lanes take a run's edges side by side and
+// the chunks that miss both the box and the point's row are skipped 64 decisions at a time (walk_edge_runs).
+__global__ void __launch_bounds__(256) k_pt_dwithin_wave(const DPoints pts, const DPolys R, const uint32_t* __restrict__ pa,
+                                                         const uint32_t* __restrict__ pb, double d, int report, uint8_t* __restrict__ hit,
+                                                         double* __restrict__ dist, const DistQueue dq, const uint32_t* __restrict__ open_list,
+                                                         const OverflowCtl* __restrict__ open_ctl) {
+  const int lane = threadIdx.x & 63;
+  const uint32_t n = open_ctl->count, nw = gridDim.x * (blockDim.x / 64);
+  for (uint32_t k = blockIdx.x * (blockDim.x / 64) + threadIdx.x / 64; k < n; k += nw) {
+    const uint32_t i = open_list[k], g = pb[i];
+    const PtFrame f(pts.xy[pa[i]], R.origin[g], R.ext[g], d);
+    auto misses = [&](const float4 c) { return (double)c.x > f.bx1 || (double)c.z < f.bx0 || (double)c.y > f.by1 || (double)c.w < f.by0; };
+    auto off_row = [&](const float4 c) { return (double)c.y > f.py || (double)c.w < f.py; };
+    bool par = false, h = false;
+    double m_up = INFINITY;
+    walk_edge_runs<64>(R, g, lane, [&](const float4 c) { return misses(c) && off_row(c); }, [&](uint64_t, uint64_t, uint64_t i0, uint64_t i1) {
+      for (uint64_t j = i0 + lane; j < i1; j += 64) {
+        const double2 v0 = R.xy[j], v1 = R.xy[j + 1];
+        if (f.near(v0, v1) && !syn_bit(R.synb, j)) {
+          double d2, band;
+          f.dist2(v0, v1, d, d2, band);
+          const double dlo = d - band, dhi = d + band;
+          if (d2 <= dlo * dlo || (!h && d2 <= dhi * dhi && f.geog(v0, v1) <= d)) h = true;
+          if (report) m_up = fmin(m_up, sqrt(d2) + band);
+        }
+        if (f.crosses(v0, v1)) par = !par;
+      }
+    });
+    h = gany<64>(h);
+    par = (__popcll(gballot<64>(par)) & 1) != 0;
+    const bool within = h || par;
+    double best = within ? (par ? 0.0 : INFINITY) : NAN;
+    if (dist && h && !par) {
+      m_up = group_min<64>(m_up);
+      walk_edge_runs<64>(R, g, lane, misses, [&](uint64_t, uint64_t, uint64_t i0, uint64_t i1) {
+        for (uint64_t j = i0 + lane; j < i1; j += 64) {
+          const double2 v0 = R.xy[j], v1 = R.xy[j + 1];
+          if (!f.near(v0, v1) || syn_bit(R.synb, j)) continue;
+          double d2, band;
+          f.dist2(v0, v1, d, d2, band);
+          if (!(sqrt(d2) - band > m_up) && !f.push(dq, i, v0, v1)) best = fmin(best, f.geog(v0, v1));
+        }
+      });
+      best = group_min<64>(best);
+    }
+    if (lane == 0) {
+      hit[i] = within ? 1 : 0;
+      if (dist) dist[i] = best;
+    }
+  }
+}
+
+__global__ void k_open_clear(OverflowCtl* ctl) { *ctl = OverflowCtl{0, 0, 0, 0}; }
 
 // ---- points in eroded polygons (buffer.cuh:1053-1131) ---------------------------------------------------------------
 constexpr double FILLET_QUANTUM = gm::PI_HI / 16.0;   // GEOS: 8 quadrant segments
@@ -691,12 +865,40 @@ void dw_deliver(Context& c, const uint32_t* orow, const double* odist, uint64_t 
 
 }  // namespace
 
+namespace {
+// The item queue of a launch over np candidates: two items per candidate (the mesh's neighbours within 5 m queue 1.2
+// per candidate), at most 32M (2.3 GB), in segments of about 8192 items, at most 256 of them.
+DistQueue dq_open(Context& c, uint64_t np) {
+  DistQueue q;
+  const uint64_t total = std::min<uint64_t>(std::max<uint64_t>(2 * np, 16384), 1ull << 25);
+  q.nseg = (uint32_t)std::min<uint64_t>(total / 8192, 256);
+  q.seg = (uint32_t)(total / q.nseg);
+  const uint64_t n = (uint64_t)q.nseg * q.seg;
+  q.c = c.s_dq.as<double>(8 * n);
+  q.pair = c.s_dq_pair.as<uint32_t>(n);
+  q.count = c.s_dq_ctl.as<uint32_t>(256);
+  hipLaunchKernelGGL(k_dq_clear, dim3(1), dim3(256), 0, c.stream, q.count);
+  GSJ_LAUNCHED();
+  return q;
+}
+// the queued distances into dist (after every kernel that appends)
+void dq_run(Context& c, const DistQueue& q, bool b_is_point, double* dist) {
+  const uint32_t per = std::max<uint32_t>(1, std::min<uint32_t>(div_up(q.seg, 256), (uint32_t)c.cu_count * 16 / q.nseg));
+  hipLaunchKernelGGL(k_geog_items, dim3(q.nseg * per), dim3(256), 0, c.stream, q, b_is_point ? 1 : 0, dist);
+  GSJ_LAUNCHED();
+}
+}  // namespace
+
 // refine one sub-batch's candidates into A.hit / A.dist (list classes, then the overflow queue)
 void dw_refine(Context& c, const DwArgs& A, uint64_t np, gsj_join_stats& s) {
   hipStream_t stream = c.stream;
   const LaunchShape& sh = c.shape(np);
   const PairClasses pc = partition_pairs(c, A.P, A.R, A.pa, A.pb, np, sh.mcap, true, sh.tcap, sh.dw_size_sort);
-  uint32_t* ovf = c.s_heavy.as<uint32_t>(np + 64);
+  uint32_t* ovf = c.s_heavy.as<uint32_t>(3 * np + 192);
+  uint32_t* open = ovf + np + 64;        // pairs the list kernels left undecided
+  uint32_t* ovf_main = open + np + 64;   // the host-read queue: lists beyond DW_OVF_CAP, undecided pairs with long lists
+  OverflowCtl* open_ctl = pc.ctl + 1;    // (the partition clears these three)
+  OverflowCtl* ctl_main = pc.ctl + 4;
   const uint32_t max_blocks = (uint32_t)c.cu_count * sh.dw_bpc;
   // the classes are independent (each appends its overflowing pairs to the queue with atomics): with sh.fork the
   // mixed and large classes run on the side stream beside the others
@@ -707,37 +909,47 @@ void dw_refine(Context& c, const DwArgs& A, uint64_t np, gsj_join_stats& s) {
     GSJ_HIP(hipStreamWaitEvent(sl, c.ev[10], 0));
   }
   GSJ_HIP(hipEventRecord(c.ev[5], sl));
-  hipLaunchKernelGGL((k_dw_lists<32, 64, false>), dim3(std::min<uint32_t>(div_up(np, 8), max_blocks)), dim3(256), 0, sl, A, pc.list, pc.counts, (int)CL_MIXED,
-                     ovf, pc.ctl);
+  hipLaunchKernelGGL((k_dw_lists<32, 64, false, false>), dim3(std::min<uint32_t>(div_up(np, 8), max_blocks)), dim3(256), 0, sl, A, pc.list, pc.counts, (int)CL_MIXED,
+                     ovf, pc.ctl, open, open_ctl);
   GSJ_LAUNCHED();
   GSJ_HIP(hipEventRecord(c.ev[7], sl));
-  hipLaunchKernelGGL((k_dw_lists<64, 128, false>), dim3(std::min<uint32_t>(div_up(np, 4), max_blocks)), dim3(256), 0, sl, A, pc.list, pc.counts, (int)CL_LARGE,
-                     ovf, pc.ctl);
+  hipLaunchKernelGGL((k_dw_lists<64, 128, false, false>), dim3(std::min<uint32_t>(div_up(np, 4), max_blocks)), dim3(256), 0, sl, A, pc.list, pc.counts, (int)CL_LARGE,
+                     ovf, pc.ctl, open, open_ctl);
   GSJ_LAUNCHED();
   GSJ_HIP(hipEventRecord(c.ev[2], sl));
+  // (only the two classes above have lists that can outgrow theirs; the others hold every vertex of their pieces)
+  hipLaunchKernelGGL(k_dw_overflow<true>, dim3((uint32_t)std::min<uint64_t>(np, (uint64_t)c.cu_count * 4)), dim3(64), 2 * DW_OVF_CAP * sizeof(Ed), sl, A, ovf,
+                     0u, DW_OVF_CAP, nullptr, pc.ctl, ovf_main, ctl_main);
+  GSJ_LAUNCHED();
+  GSJ_HIP(hipEventRecord(c.ev[16], sl));
   GSJ_HIP(hipEventRecord(c.ev[0], stream));
-  hipLaunchKernelGGL((k_dw_lists<8, 16, true>), dim3(std::min<uint32_t>(div_up(np, 32), max_blocks)), dim3(256), 0, stream, A, pc.list, pc.counts, (int)CL_TINY,
-                     ovf, pc.ctl);
+  hipLaunchKernelGGL((k_dw_lists<8, 16, true, false>), dim3(std::min<uint32_t>(div_up(np, 32), max_blocks)), dim3(256), 0, stream, A, pc.list, pc.counts, (int)CL_TINY,
+                     ovf, pc.ctl, open, open_ctl);
   GSJ_LAUNCHED();
   GSJ_HIP(hipEventRecord(c.ev[8], stream));
-  hipLaunchKernelGGL((k_dw_lists<16, 32, true>), dim3(std::min<uint32_t>(div_up(np, 16), max_blocks)), dim3(256), 0, stream, A, pc.list, pc.counts, (int)CL_SMALL,
-                     ovf, pc.ctl);
+  hipLaunchKernelGGL((k_dw_lists<16, 32, true, false>), dim3(std::min<uint32_t>(div_up(np, 16), max_blocks)), dim3(256), 0, stream, A, pc.list, pc.counts, (int)CL_SMALL,
+                     ovf, pc.ctl, open, open_ctl);
   GSJ_LAUNCHED();
   GSJ_HIP(hipEventRecord(c.ev[1], stream));
-  hipLaunchKernelGGL((k_dw_lists<32, 64, true>), dim3(std::min<uint32_t>(div_up(np, 8), max_blocks)), dim3(256), 0, stream, A, pc.list, pc.counts, (int)CL_MEDIUM,
-                     ovf, pc.ctl);
+  hipLaunchKernelGGL((k_dw_lists<32, 64, true, false>), dim3(std::min<uint32_t>(div_up(np, 8), max_blocks)), dim3(256), 0, stream, A, pc.list, pc.counts, (int)CL_MEDIUM,
+                     ovf, pc.ctl, open, open_ctl);
   GSJ_LAUNCHED();
   GSJ_HIP(hipEventRecord(c.ev[9], stream));
   if (sh.fork) {
     GSJ_HIP(hipEventRecord(c.ev[11], sl));
     GSJ_HIP(hipStreamWaitEvent(stream, c.ev[11], 0));
   }
-  struct Host { uint32_t counts[8]; OverflowCtl ctl; };
+  // the undecided pairs of all classes, their number read on the device
+  hipLaunchKernelGGL((k_dw_lists<64, 128, false, true>), dim3(std::min<uint32_t>(div_up(np, 4), (uint32_t)c.cu_count * 2)), dim3(256), 0, stream, A, open,
+                     pc.counts, 0, ovf_main, ctl_main, nullptr, open_ctl);
+  GSJ_LAUNCHED();
+  struct Host { uint32_t counts[16]; OverflowCtl ctl[5]; };
   Host* h = c.h_scal.as<Host>(2);
-  GSJ_HIP(hipMemcpyAsync(h->counts, pc.counts, 32, hipMemcpyDeviceToHost, stream));
-  GSJ_HIP(hipMemcpyAsync(&h->ctl, pc.ctl, sizeof(OverflowCtl), hipMemcpyDeviceToHost, stream));
+  static_assert(sizeof(Host) == 144, "counts and the queues' controls are copied as one block");
+  GSJ_HIP(hipMemcpyAsync(h, pc.counts, sizeof(Host), hipMemcpyDeviceToHost, stream));
   GSJ_HIP(hipStreamSynchronize(stream));
-  float ms_t = 0, ms_s = 0, ms_m = 0, ms_x = 0, ms_l = 0;
+  float ms_t = 0, ms_s = 0, ms_m = 0, ms_x = 0, ms_l = 0, ms_v = 0;
+  GSJ_HIP(hipEventElapsedTime(&ms_v, c.ev[2], c.ev[16]));
   GSJ_HIP(hipEventElapsedTime(&ms_t, c.ev[0], c.ev[8]));
   GSJ_HIP(hipEventElapsedTime(&ms_s, c.ev[8], c.ev[1]));
   GSJ_HIP(hipEventElapsedTime(&ms_m, c.ev[1], c.ev[9]));
@@ -747,24 +959,26 @@ void dw_refine(Context& c, const DwArgs& A, uint64_t np, gsj_join_stats& s) {
   s.n_tiny += h->counts[CL_TINY]; s.n_small += h->counts[CL_SMALL]; s.n_medium += h->counts[CL_MEDIUM]; s.n_mixed += h->counts[CL_MIXED];
   s.n_large += h->counts[CL_LARGE];
   s.launches++;
-  const uint32_t nover = h->ctl.count;
+  const uint32_t nover = h->ctl[4].count, n_side = h->ctl[0].count - h->ctl[0].pad0;   // each pair once
+  s.k_over_ms += ms_v;
+  s.n_over += n_side + nover;
+  s.heavy += n_side + nover;
   if (nover) {
-    const int cap = (int)h->ctl.need;
+    const int cap = (int)h->ctl[4].need;
     const size_t per = 2 * (size_t)cap * sizeof(Ed);
     uint64_t waves = std::max<uint64_t>(1, std::min<uint64_t>(nover, (1ull << 30) / per));
     waves = (waves + 3) / 4 * 4;
     Ed* slab = c.s_heavy_edges.as<Ed>(2 * (uint64_t)cap * waves + 16);
     GSJ_HIP(hipEventRecord(c.ev[3], stream));
-    hipLaunchKernelGGL(k_dw_overflow, dim3((uint32_t)(waves / 4)), dim3(256), 0, stream, A, ovf, nover, cap, slab);
+    hipLaunchKernelGGL(k_dw_overflow<false>, dim3((uint32_t)(waves / 4)), dim3(256), 0, stream, A, ovf_main, nover, cap, slab, pc.ctl, nullptr, nullptr);
     GSJ_LAUNCHED();
     GSJ_HIP(hipEventRecord(c.ev[4], stream));
     GSJ_HIP(hipEventSynchronize(c.ev[4]));
     float ms_o = 0;
     GSJ_HIP(hipEventElapsedTime(&ms_o, c.ev[3], c.ev[4]));
     s.k_over_ms += ms_o;
-    s.n_over += nover;
-    s.heavy += nover;
   }
+  if (A.report) dq_run(c, A.dq, false, A.dist);
 }
 
 void dwithin_run(Context& c, const Layer& PL, const Layer& RL, double d, bool same, bool report, const gsj_join_opts& o, gsj_dist_cb cb, void* user,
@@ -787,7 +1001,8 @@ void dwithin_run(Context& c, const Layer& PL, const Layer& RL, double d, bool sa
   for_each_candidate_batch(c, probes_of(PL), RL.bvh, o.upper != 0, o, s, [&](uint32_t* pa, uint32_t* pb, uint64_t np) {
     WallTimer t2;
     DwArgs A{PL.poly, RL.poly, pa, pb, d, same ? 1 : 0, report ? 1 : 0, c.s_flag.as<uint8_t>(np + 16), report ? c.s_area.as<double>(np + 16) : nullptr,
-             nullptr, DistSet{}};
+             nullptr, DistSet{}, DistQueue{}};
+    if (report) A.dq = dq_open(c, np);
     dw_refine(c, A, np, s);
     GSJ_HIP(hipStreamSynchronize(stream));
     s.refine_ms += t2.ms();
@@ -836,7 +1051,8 @@ void dwithin_batch_run(Context& c, const Layer& PL, const Layer& RL, bool same, 
     for (uint32_t r = 0; r < k; r++) cand[r] += sb.h[r + 1] - sb.h[r];
     WallTimer t2;
     DwArgs A{PL.poly, RL.poly, pa, pb, 0.0, same ? 1 : 0, report ? 1 : 0, c.s_flag.as<uint8_t>(np + 16), report ? c.s_area.as<double>(np + 16) : nullptr,
-             sb.d, ds};
+             sb.d, ds, DistQueue{}};
+    if (report) A.dq = dq_open(c, np);
     dw_refine(c, A, np, s);
     GSJ_HIP(hipStreamSynchronize(stream));
     s.refine_ms += t2.ms();
@@ -891,9 +1107,19 @@ void points_dwithin_run(Context& c, const Layer& PL, const Layer& RL, double d, 
     WallTimer t2;
     uint8_t* hit = c.s_flag.as<uint8_t>(np + 16);
     double* dist = report ? c.s_area.as<double>(np + 16) : nullptr;
-    GSJ_HIP(hipEventRecord(c.ev[0], stream));
-    hipLaunchKernelGGL(k_pt_dwithin, dim3(div_up(np, 256)), dim3(256), 0, stream, PL.pts, RL.poly, pa, pb, np, d, report ? 1 : 0, hit, dist);
+    const DistQueue dq = report ? dq_open(c, np) : DistQueue{};
+    uint32_t* open = c.s_heavy.as<uint32_t>(np + 64);
+    OverflowCtl* open_ctl = reinterpret_cast<OverflowCtl*>(c.s_misc.as<char>(256) + 128);
+    hipLaunchKernelGGL(k_open_clear, dim3(1), dim3(1), 0, stream, open_ctl);
     GSJ_LAUNCHED();
+    GSJ_HIP(hipEventRecord(c.ev[0], stream));
+    hipLaunchKernelGGL(k_pt_dwithin, dim3(div_up(np, 256)), dim3(256), 0, stream, PL.pts, RL.poly, pa, pb, np, d, report ? 1 : 0, hit, dist, dq, open,
+                       open_ctl);
+    GSJ_LAUNCHED();
+    hipLaunchKernelGGL(k_pt_dwithin_wave, dim3(std::min<uint32_t>(div_up(np, 4), (uint32_t)c.cu_count * 8)), dim3(256), 0, stream, PL.pts, RL.poly, pa,
+                       pb, d, report ? 1 : 0, hit, dist, dq, open, open_ctl);
+    GSJ_LAUNCHED();
+    if (report) dq_run(c, dq, true, dist);
     GSJ_HIP(hipEventRecord(c.ev[1], stream));
     GSJ_HIP(hipStreamSynchronize(stream));
     float ms = 0;

@@ -136,52 +136,59 @@ GSJ_PORT double seg_seg_d2(double a0x, double a0y, double a1x, double a1y, doubl
 
 // ---- great-circle arcs on the unit sphere ---------------------------------------------------------------------------
 struct V3 { double x, y, z; };
-GSJ_PORT V3 unit_of(double lon, double lat) {   // radians
-  double sl, cl, sp, cp;
-  gm::sincos(lon, sl, cl);
-  gm::sincos(lat, sp, cp);
-  return V3{cp * cl, cp * sl, sp};
-}
 GSJ_PORT double dot3(V3 a, V3 b) { return a.x * b.x + a.y * b.y + a.z * b.z; }
 GSJ_PORT V3 cross3(V3 a, V3 b) { return V3{a.y * b.z - a.z * b.y, a.z * b.x - a.x * b.z, a.x * b.y - a.y * b.x}; }
 GSJ_PORT V3 unit3(V3 a) {
   const double l = sqrt(dot3(a, a));
   return l > 0 ? V3{a.x / l, a.y / l, a.z / l} : V3{0, 0, 0};
 }
+// angle between unit vectors; the same bits either way round (the cross product only changes sign)
 GSJ_PORT double angle3(V3 a, V3 b) { const V3 c = cross3(a, b); return gm::atan2(sqrt(dot3(c, c)), dot3(a, b)); }
 
-// e - s for the unit vectors of (slon, slat) and (elon, elat) (radians), each coordinate difference written as
-// products of sines of half differences (cos A - cos B = -2 sin((A+B)/2) sin((A-B)/2), sin A - sin B =
-// 2 cos((A+B)/2) sin((A-B)/2)), so that the chord of nearby points carries full relative precision
-GSJ_PORT V3 chord(double slon, double slat, double elon, double elat) {
-  double s_hl, c_hl, s_ml, c_ml, s_hp, c_hp, s_mp, c_mp, sls, cls, sps, cps, spe, cpe;
-  gm::sincos(0.5 * (elon - slon), s_hl, c_hl);   // half the longitude difference
-  gm::sincos(0.5 * (elon + slon), s_ml, c_ml);   // mean longitude
-  gm::sincos(0.5 * (elat - slat), s_hp, c_hp);
-  gm::sincos(0.5 * (elat + slat), s_mp, c_mp);
-  gm::sincos(slon, sls, cls);
-  gm::sincos(slat, sps, cps);
-  gm::sincos(elat, spe, cpe);
-  const double dcos_lon = -2.0 * s_ml * s_hl, dsin_lon = 2.0 * c_ml * s_hl;   // cos(elon) - cos(slon), sin(elon) - sin(slon)
-  const double dcos_lat = -2.0 * s_mp * s_hp, dsin_lat = 2.0 * c_mp * s_hp;   // cos(elat) - cos(slat), sin(elat) - sin(slat)
-  return V3{cpe * dcos_lon + cls * dcos_lat, cpe * dsin_lon + sls * dcos_lat, dsin_lat};
+// a point (radians) with the sines and cosines that every use of it shares, and its unit vector
+struct ArcPt {
+  double lon, lat, sl, cl, sp, cp;
+  V3 u;
+};
+GSJ_PORT ArcPt arc_pt(double lon, double lat) {
+  ArcPt p;
+  p.lon = lon;
+  p.lat = lat;
+  gm::sincos(lon, p.sl, p.cl);
+  gm::sincos(lat, p.sp, p.cp);
+  p.u = V3{p.cp * p.cl, p.cp * p.sl, p.sp};
+  return p;
 }
 
-// closest point (clon, clat, radians) of the great-circle arc s-e to p, and its angle from p. The foot of p on the
-// arc's great circle is p minus its component along the arc normal n = s x (e - s); it lies on the arc when it is on
-// the inner side of both endpoints ((s x k).n >= 0 and (k x e).n >= 0); otherwise the nearer endpoint is closest.
-GSJ_PORT double gc_closest(double slon, double slat, double elon, double elat, double plon, double plat, double& clon, double& clat) {
-  const V3 s = unit_of(slon, slat), e = unit_of(elon, elat), p = unit_of(plon, plat);
-  const double as = angle3(p, s), ae = angle3(p, e);
+// e - s for the unit vectors of s and e, each coordinate difference written as products of sines of half differences
+// (cos A - cos B = -2 sin((A+B)/2) sin((A-B)/2), sin A - sin B = 2 cos((A+B)/2) sin((A-B)/2)), so that the chord of
+// nearby points carries full relative precision
+GSJ_PORT V3 chord(const ArcPt& s, const ArcPt& e) {
+  double s_hl, c_hl, s_ml, c_ml, s_hp, c_hp, s_mp, c_mp;
+  gm::sincos(0.5 * (e.lon - s.lon), s_hl, c_hl);   // half the longitude difference
+  gm::sincos(0.5 * (e.lon + s.lon), s_ml, c_ml);   // mean longitude
+  gm::sincos(0.5 * (e.lat - s.lat), s_hp, c_hp);
+  gm::sincos(0.5 * (e.lat + s.lat), s_mp, c_mp);
+  const double dcos_lon = -2.0 * s_ml * s_hl, dsin_lon = 2.0 * c_ml * s_hl;   // cos(elon) - cos(slon), sin(elon) - sin(slon)
+  const double dcos_lat = -2.0 * s_mp * s_hp, dsin_lat = 2.0 * c_mp * s_hp;   // cos(elat) - cos(slat), sin(elat) - sin(slat)
+  return V3{e.cp * dcos_lon + s.cl * dcos_lat, e.cp * dsin_lon + s.sl * dcos_lat, dsin_lat};
+}
+// unit normal of the arc s-e (0 for a point): s x (e - s)
+GSJ_PORT V3 arc_normal(const ArcPt& s, const ArcPt& e) { return unit3(cross3(s.u, chord(s, e))); }
+
+// closest point (clon, clat, radians) of the great-circle arc s-e with normal n to p, and its angle from p (as, ae:
+// the angles of p from s and e). The foot of p on the arc's great circle is p minus its component along n; it lies on
+// the arc when it is on the inner side of both endpoints ((s x k).n >= 0 and (k x e).n >= 0); otherwise the nearer
+// endpoint is closest.
+GSJ_PORT double gc_closest(const ArcPt& s, const ArcPt& e, V3 n, const ArcPt& p, double as, double ae, double& clon, double& clat) {
   double best = as;
-  clon = slon; clat = slat;
-  if (ae < best) { best = ae; clon = elon; clat = elat; }
-  if (slon == elon && slat == elat) return best;
-  const V3 n = unit3(cross3(s, chord(slon, slat, elon, elat)));
-  const double h = dot3(p, n);
-  const V3 k = unit3(V3{p.x - h * n.x, p.y - h * n.y, p.z - h * n.z});
-  if (dot3(k, k) == 0 || dot3(cross3(s, k), n) < 0 || dot3(cross3(k, e), n) < 0) return best;
-  const double ak = angle3(p, k);
+  clon = s.lon; clat = s.lat;
+  if (ae < best) { best = ae; clon = e.lon; clat = e.lat; }
+  if (s.lon == e.lon && s.lat == e.lat) return best;
+  const double h = dot3(p.u, n);
+  const V3 k = unit3(V3{p.u.x - h * n.x, p.u.y - h * n.y, p.u.z - h * n.z});
+  if (dot3(k, k) == 0 || dot3(cross3(s.u, k), n) < 0 || dot3(cross3(k, e.u), n) < 0) return best;
+  const double ak = angle3(p.u, k);
   if (ak < best) {
     best = ak;
     clat = gm::atan2(k.z, sqrt(k.x * k.x + k.y * k.y));
@@ -192,24 +199,35 @@ GSJ_PORT double gc_closest(double slon, double slat, double elon, double elat, d
 
 // geography distance (metres) between the arcs a0-a1 and b0-b1 that do not cross, or of the arc a from the point b0
 // (b_is_point); degrees in. The closest pair of points has an endpoint of one arc: of the four (endpoint, arc)
-// candidates the one at the smallest angle is measured on the ellipsoid. Not inlined: called only for edge pairs
-// inside the band, it would otherwise dominate the callers' register use.
-__attribute__((noinline)) GSJ_PORT double geog_dist(double a0x, double a0y, double a1x, double a1y, double b0x, double b0y, double b1x, double b1y,
-                                                     bool b_is_point) {
+// candidates the one at the smallest angle is measured on the ellipsoid. What the four candidates share is computed
+// once: the four points' sines and unit vectors, the two arc normals, the four endpoint-to-endpoint angles (16 sincos
+// and 4 + at most 4 angles; candidate by candidate it was 56 and 8 + at most 4).
+GSJ_PORT double geog_dist_of(double a0x, double a0y, double a1x, double a1y, double b0x, double b0y, double b1x, double b1y, bool b_is_point) {
   const double r = DEG;
-  const double A[4] = {a0x * r, a0y * r, a1x * r, a1y * r}, B[4] = {b0x * r, b0y * r, b1x * r, b1y * r};
-  double best = INFINITY, p1x = B[0], p1y = B[1], p2x = B[0], p2y = B[1];
-#pragma unroll
-  for (int k = 0; k < 4; k++) {
-    if (b_is_point && k > 0) break;
-    const double* arc = k < 2 ? A : B;   // endpoint k % 2 of the other side against this arc
-    const double* other = k < 2 ? B : A;
-    const double qx = other[2 * (k & 1)], qy = other[2 * (k & 1) + 1];
-    double cx, cy;
-    const double ang = gc_closest(arc[0], arc[1], arc[2], arc[3], qx, qy, cx, cy);
-    if (ang < best) { best = ang; p1x = cx; p1y = cy; p2x = qx; p2y = qy; }
+  const ArcPt a0 = arc_pt(a0x * r, a0y * r), a1 = arc_pt(a1x * r, a1y * r), b0 = arc_pt(b0x * r, b0y * r);
+  const V3 na = arc_normal(a0, a1);
+  const double a00 = angle3(b0.u, a0.u), a01 = angle3(b0.u, a1.u);   // of b0 from a0 and a1
+  double best = INFINITY, p1x = b0.lon, p1y = b0.lat, p2x = b0.lon, p2y = b0.lat, cx, cy;
+  const double d0 = gc_closest(a0, a1, na, b0, a00, a01, cx, cy);
+  if (d0 < best) { best = d0; p1x = cx; p1y = cy; p2x = b0.lon; p2y = b0.lat; }
+  if (!b_is_point) {
+    const ArcPt b1 = arc_pt(b1x * r, b1y * r);
+    const double a10 = angle3(b1.u, a0.u), a11 = angle3(b1.u, a1.u);
+    const double d1 = gc_closest(a0, a1, na, b1, a10, a11, cx, cy);
+    if (d1 < best) { best = d1; p1x = cx; p1y = cy; p2x = b1.lon; p2y = b1.lat; }
+    const V3 nb = arc_normal(b0, b1);
+    const double d2 = gc_closest(b0, b1, nb, a0, a00, a10, cx, cy);
+    if (d2 < best) { best = d2; p1x = cx; p1y = cy; p2x = a0.lon; p2y = a0.lat; }
+    const double d3 = gc_closest(b0, b1, nb, a1, a01, a11, cx, cy);
+    if (d3 < best) { best = d3; p1x = cx; p1y = cy; p2x = a1.lon; p2y = a1.lat; }
   }
   return vincenty_m(p1x / r, p1y / r, p2x / r, p2y / r);
+}
+// the same out of line, for callers that need it only for edge pairs inside the band: inlined there it would dominate
+// their register use
+__attribute__((noinline)) GSJ_PORT double geog_dist(double a0x, double a0y, double a1x, double a1y, double b0x, double b0y, double b1x, double b1y,
+                                                     bool b_is_point) {
+  return geog_dist_of(a0x, a0y, a1x, a1y, b0x, b0y, b1x, b1y, b_is_point);
 }
 
 // ---- frame distance versus geography distance ------------------------------------------------------------------------

@@ -123,7 +123,8 @@ typedef struct {
   uint64_t hits;           /* result rows delivered (parent pairs) */
   uint64_t heavy;          /* pairs whose local edge lists exceeded on-chip capacity */
   uint64_t batches;
-  /* pair kernels, timed with HIP events on the context's stream, summed durations and pairs handled by each. Polygon
+  /* pair kernels, timed on the device, summed durations and pairs handled by each (launches of few pairs run several
+   * classes side by side: each class that had pairs then reports the span of the launch it shared). Polygon
    * joins: small = 16-lane class (both polygons <= 32 stored vertices and <= 8 rings), medium = 32-lane class (not
    * small, both <= 64 stored vertices and <= 8 rings); these two classes are screened first (contact, containment;
    * k_screen_ms, every small and medium pair) and k_small_ms / k_medium_ms time their edge-contribution kernels over

@@ -53,6 +53,8 @@ void context_init(Context& c, int device) {
   std::string arch;
   if (hipGetDeviceProperties(&p, device) == hipSuccess) {
     c.cu_count = p.multiProcessorCount;
+    int khz = 0;
+    if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, c.device) == hipSuccess && khz > 0) c.clock_khz = khz;
     arch = p.gcnArchName;
     arch = arch.substr(0, arch.find(':'));   // "gfx950:sramecc+:xnack-" -> "gfx950"
   }

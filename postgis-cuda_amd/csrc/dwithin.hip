@@ -192,13 +192,13 @@ __device__ __forceinline__ uint64_t near_mask(const Ed* L, int base, int n, doub
 // the geography distances of the edge pairs that could hold it: a few of them per pair, each thousands of FP64
 // operations. Evaluated where they are found, one or two lanes of a group worked while its others waited; queued, they
 // fill whole waves (k_geog_items), and the pair kernels are left with the frame tests (300k parcels, 5 m self dwithin
-// with distances: the pair kernels 20.0 -> 4.7 ms and 1.1 ms for the items). The minimum does not depend on the
+// with distances: the vertex-list classes 17.9 -> 3.0 ms, the items 0.34, the request 20.3 -> 5.1). The minimum does not depend on the
 // order, so the distances are the same bits. The queue is cut into segments, one counter each, so that the blocks do
-// not all append through one address; items that find their segment full are evaluated in place.
+// not all append through one address; items that find their segment full send their candidate to a GEO kernel.
 struct DistQueue {
   double* c = nullptr;        // [8][nseg * seg] the item's arc a0, a1 and arc b0, b1 (x, y each, degrees)
   uint32_t* pair = nullptr;   // [nseg * seg] its candidate
-  uint32_t* count = nullptr;  // [nseg] items appended (may exceed seg: the rest were evaluated in place)
+  uint32_t* count = nullptr;  // [nseg] items appended (may exceed seg: the rest found no room)
   uint32_t nseg = 0, seg = 0;
 };
 __device__ __forceinline__ bool dq_push(const DistQueue& q, uint32_t p, double a0x, double a0y, double a1x, double a1y, double b0x, double b0y,

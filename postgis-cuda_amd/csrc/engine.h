@@ -110,11 +110,12 @@ struct Context {
   DevBuf s_counts, s_qoffs, s_offs, s_pairs_a, s_pairs_b, s_flag, s_area, s_ev, s_evb, s_tmp, s_tmp2, s_cls, s_out_a, s_out_b, s_out_area,
       s_out_code, s_out_flag, s_keys, s_keys2, s_vals, s_vals2, s_seg, s_heavy, s_heavy_edges, s_scal, s_qbb, s_uf, s_root, s_misc, s_win, s_qidx,
       s_win_off, s_edgeq, s_qlist, s_wtile, s_wtoff, s_wseg, s_slots, s_slots_ctl,
-      s_dq, s_dq_pair, s_dq_ctl;
+      s_dq, s_dq_pair, s_dq_ctl, s_words;
   // erosion pass 2 (it runs inside the join's on-device hook, beside the join's own scratch)
   DevBuf s_er_keep, s_er_off, s_er_pairs, s_er_flag, s_er_list, s_er_slab, s_er_out, s_er_need, s_er_pf;
-  PinBuf h_pairs, h_area, h_code, h_where, h_scal, h_counts, h_seg, h_slots_ctl;
+  PinBuf h_pairs, h_area, h_code, h_where, h_scal, h_counts, h_seg, h_words;
   int cu_count = 256;
+  double clock_khz = 100000;      // rate of the device's wall_clock64
   hipEvent_t ev[17] = {};   // kernel timing events (created with the context); ev[10], ev[11]: fork / join of `side`;
                             // ev[12 .. 15]: the traversal passes and the BVH build; ev[16]: the list classes' overflow
   bool borrowed = false;   // stream and events belong to another context (not destroyed with this one)
@@ -128,14 +129,31 @@ struct Context {
                       &s_out_b, &s_out_area, &s_out_code, &s_out_flag, &s_keys, &s_keys2, &s_vals, &s_vals2, &s_seg, &s_heavy, &s_heavy_edges,
                       &s_scal, &s_qbb, &s_uf, &s_root, &s_misc, &s_win, &s_qidx, &s_win_off, &s_edgeq, &s_qlist, &s_wtile, &s_wtoff, &s_wseg,
                       &s_slots, &s_slots_ctl, &s_er_keep, &s_er_off, &s_er_pairs, &s_er_flag, &s_er_list, &s_er_slab, &s_er_out, &s_er_need,
-                      &s_er_pf, &s_dq, &s_dq_pair, &s_dq_ctl})
+                      &s_er_pf, &s_dq, &s_dq_pair, &s_dq_ctl, &s_words})
       f(*b);
   }
   template <class F> void for_each_pinbuf(F f) {
-    for (PinBuf* b : {&h_pairs, &h_area, &h_code, &h_where, &h_scal, &h_counts, &h_seg, &h_slots_ctl}) f(*b);
+    for (PinBuf* b : {&h_pairs, &h_area, &h_code, &h_where, &h_scal, &h_counts, &h_seg, &h_words}) f(*b);
   }
   ~Context();
 };
+
+// The few words that the host reads between a request's launches (totals, class sizes, queue lengths). Kernels write
+// them straight into pinned host memory, valid once the stream is synchronised; a context whose host memory is not
+// pinned (the no-allocation entry point's) takes them in device memory and copies them over.
+constexpr int HOST_WORDS = 128;   // words of a context: [0, 8) scans, [8, 16) the candidate search, [32, 128) the refinement
+struct HostWords {
+  uint64_t* host;
+  uint64_t* dev;   // where the kernels write (host itself when it is pinned)
+  size_t n;
+  void fetch(Context& c) const {   // enqueue the copy, where one is needed
+    if (dev != host) GSJ_HIP(hipMemcpyAsync(host, dev, n * 8, hipMemcpyDeviceToHost, c.stream));
+  }
+};
+inline HostWords host_words(Context& c, size_t first, size_t n) {
+  uint64_t* h = c.h_words.as<uint64_t>(HOST_WORDS) + first;
+  return HostWords{h, c.dev_arena ? c.s_words.as<uint64_t>(HOST_WORDS) + first : h, n};
+}
 
 // ------------------------------------------------------------------------------------------- primitives (prims.hip)
 // exclusive prefix sum of n u32 values into u64 offsets; returns the total (synchronises)
@@ -242,6 +260,17 @@ struct RefineOut {
 // Kernel durations and per-class pair counts are added to *st (if given).
 uint64_t refine_pairs(Context& c, const DPolys& P, const DPolys& R, const uint32_t* pa, const uint32_t* pb, uint64_t np, const RefineParams& rp,
                       const RefineOut& out, gsj_join_stats* st = nullptr);
+
+// The same for at most STAGED_MAX pairs without a host wait (see refine.hip): refine_stages enqueues the classes, the
+// overflow pass and a report; after the caller's own wait, refine_stages_finish adds to the statistics and refines the
+// pairs left over (lists too long for LDS), returning whether there were any: what the caller computed from the outputs
+// has to be redone then (n_over: pairs that took an overflow pass). refine_staged: whether a launch of np pairs takes this way.
+constexpr uint64_t STAGED_MAX = 32768;
+bool refine_staged(const Context& c, uint64_t np);
+void refine_stages(Context& c, const DPolys& P, const DPolys& R, const uint32_t* pa, const uint32_t* pb, uint64_t np, const RefineParams& rp,
+                   const RefineOut& out);
+bool refine_stages_finish(Context& c, const DPolys& P, const DPolys& R, const uint32_t* pa, const uint32_t* pb, uint64_t np, const RefineParams& rp,
+                          const RefineOut& out, gsj_join_stats& s, uint64_t& n_over);
 
 // ------------------------------------------------------------------------------------------- join driver
 struct JoinHooks {

@@ -8,7 +8,7 @@
 // directly (kept iff its flag is 1). Only pairs touching a subdivided parent are sorted and folded, first by piece
 // pair and then (stable) by parent pair, so every parent's terms are added in the same order as in the CPU
 // restatement: a subdivided layer's aggregated areas are bit-identical too.
-#include "engine.h"
+#include "scan.h"
 #include <algorithm>
 #include <chrono>
 
@@ -169,39 +169,63 @@ static uint64_t compact_rows(Context& c, const Layer& PL, const Layer& RL, const
   return nsingle + nkeep;
 }
 
-// Sub-batches of at most this many candidates whose rows need no piece -> parent folding compact and copy their rows
-// with one host wait (compact_copy_small)
+// Sub-batches of at most this many candidates whose rows need no piece -> parent folding are compacted and delivered
+// with one host wait (compact_small)
 constexpr uint64_t SMALL_COPY_PAIRS = 1u << 20;
 
-// compact_rows and the row copy of such a sub-batch: the copy takes np rows (the candidate count, known on the host, is
-// an upper bound of the row count) together with the device's row count, so the count is not read back first: one
-// host wait instead of two. Returns the row count; the rows are in the context's pinned buffers.
-static uint64_t compact_copy_small(Context& c, const Layer& PL, const Layer& RL, const uint32_t* pa, const uint32_t* pb, uint64_t np,
-                                   const RefineParams& rp, const RefineOut& ro, bool no_agg, uint32_t* orow, double* oarea, uint32_t* ocode,
-                                   uint32_t*& hrow, double*& harea, uint32_t*& hcode) {
+// Compaction and delivery of such a sub-batch without reading the row count first: the scan takes the flags from the
+// refinement's bytes and writes the count, and the emission the rows, straight into pinned host memory, so the host
+// waits once and nothing is copied behind the kernels (three copies of the candidate count's size before). A context
+// without pinned memory writes device buffers and copies np rows, an upper bound. compact_small enqueues, rows_small
+// gives the rows after the caller's wait.
+struct LoadHit {   // kept candidates: flag 1, or any flag (no aggregation)
+  const uint8_t* f;
+  int any;
+  __device__ __forceinline__ bool keep(uint64_t i) const { return any ? f[i] != 0 : f[i] == 1; }
+  __device__ __forceinline__ uint64_t operator()(uint64_t i) const { return keep(i) ? 1u : 0u; }
+};
+struct SmallRows { uint32_t* row; double* area; uint32_t* code; HostWords total; };
+
+__global__ void k_emit_hits(const DPolys P, const DPolys R, const uint32_t* __restrict__ pa, const uint32_t* __restrict__ pb, const LoadHit hit,
+                            const uint64_t* __restrict__ offs, uint64_t n, const double* __restrict__ area, const double4* __restrict__ ev,
+                            const uint32_t* __restrict__ evb, uint32_t* __restrict__ orow, double* __restrict__ oarea, uint32_t* __restrict__ ocode) {
+  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n || !hit.keep(i)) return;
+  const uint64_t o = offs[i];
+  const uint32_t a = pa[i], b = pb[i];
+  reinterpret_cast<uint2*>(orow)[o] = make_uint2(a, b);
+  if (oarea) oarea[o] = area[i];
+  if (ocode) {
+    const double4 e = ev[i];
+    ocode[o] = de9im_code(e.x, e.y, e.z, e.w, evb[i], P.blen[parent_of(P, a)], R.blen[parent_of(R, b)]);
+  }
+}
+
+static SmallRows compact_small(Context& c, const Layer& PL, const Layer& RL, const uint32_t* pa, const uint32_t* pb, uint64_t np, const RefineParams& rp,
+                               const RefineOut& ro, bool no_agg) {
   hipStream_t st = c.stream;
-  const DPolys& P = PL.poly;
-  const DPolys& R = RL.poly;
-  uint32_t* fs = c.s_tmp.as<uint32_t>(2 * np + 16);
-  uint32_t* fm = fs + np;
+  const LoadHit hit{ro.isect, no_agg ? 1 : 0};
   uint64_t* offs = c.s_offs.as<uint64_t>(np + 16);
-  uint64_t* d_total = c.s_misc.as<uint64_t>(4);   // the scan primitives' scalar
-  hipLaunchKernelGGL(k_row_flags, dim3(div_up(np, 256)), dim3(256), 0, st, P, R, pa, pb, ro.isect, np, no_agg ? 1 : 0, fs, fm);
+  SmallRows h;
+  h.total = host_words(c, 0, 1);
+  h.row = c.h_pairs.as<uint32_t>(2 * np);
+  h.area = rp.want_area ? c.h_area.as<double>(np) : nullptr;
+  h.code = rp.want_relate ? c.h_code.as<uint32_t>(np) : nullptr;
+  scan_loaded<uint64_t>(c, hit, offs, np, ScanTotal{h.total.dev, nullptr});
+  const bool direct = !c.dev_arena;
+  uint32_t* orow = direct ? h.row : c.s_out_a.as<uint32_t>(2 * np + 16);
+  double* oarea = !h.area ? nullptr : direct ? h.area : c.s_out_area.as<double>(np + 16);
+  uint32_t* ocode = !h.code ? nullptr : direct ? h.code : c.s_out_code.as<uint32_t>(np + 16);
+  hipLaunchKernelGGL(k_emit_hits, dim3(div_up(np, 256)), dim3(256), 0, st, PL.poly, RL.poly, pa, pb, hit, offs, np, ro.area, ro.ev, ro.evb, orow, oarea,
+                     ocode);
   GSJ_LAUNCHED();
-  scan_u32_to_u64_async(c, fs, offs, np, d_total);
-  hipLaunchKernelGGL(k_emit_single, dim3(div_up(np, 256)), dim3(256), 0, st, P, R, pa, pb, fs, offs, np, no_agg ? 1 : 0, ro.area, ro.ev, ro.evb,
-                     orow, rp.want_area ? oarea : nullptr, rp.want_relate ? ocode : nullptr);
-  GSJ_LAUNCHED();
-  uint64_t* h_total = c.h_scal.as<uint64_t>(4);
-  hrow = c.h_pairs.as<uint32_t>(2 * np);
-  harea = rp.want_area ? c.h_area.as<double>(np) : nullptr;
-  hcode = rp.want_relate ? c.h_code.as<uint32_t>(np) : nullptr;
-  GSJ_HIP(hipMemcpyAsync(h_total, d_total, 8, hipMemcpyDeviceToHost, st));
-  GSJ_HIP(hipMemcpyAsync(hrow, orow, np * 8, hipMemcpyDeviceToHost, st));
-  if (harea) GSJ_HIP(hipMemcpyAsync(harea, oarea, np * 8, hipMemcpyDeviceToHost, st));
-  if (hcode) GSJ_HIP(hipMemcpyAsync(hcode, ocode, np * 4, hipMemcpyDeviceToHost, st));
-  GSJ_HIP(hipStreamSynchronize(st));
-  return h_total[0];
+  if (!direct) {
+    h.total.fetch(c);
+    GSJ_HIP(hipMemcpyAsync(h.row, orow, np * 8, hipMemcpyDeviceToHost, st));
+    if (h.area) GSJ_HIP(hipMemcpyAsync(h.area, oarea, np * 8, hipMemcpyDeviceToHost, st));
+    if (h.code) GSJ_HIP(hipMemcpyAsync(h.code, ocode, np * 4, hipMemcpyDeviceToHost, st));
+  }
+  return h;
 }
 
 void join_run(Context& c, const Layer& PL, const Layer& RL, const gsj_join_opts& o, gsj_rows_cb cb, void* user, gsj_join_stats* st,
@@ -231,22 +255,30 @@ void join_run(Context& c, const Layer& PL, const Layer& RL, const gsj_join_opts&
     ro.evb = rp.want_relate ? c.s_evb.as<uint32_t>(np + 16) : nullptr;
     // no host waits between refinement, compaction and the row copy beyond the ones that read sizes back: the
     // stream orders the work (refine_ms and compact_ms are host times up to those reads)
-    s.heavy += refine_pairs(c, PL.poly, RL.poly, pa, pb, np, rp, ro, &s);
+    const bool small = !hooks && np <= SMALL_COPY_PAIRS && (o.no_agg || (!PL.poly.pfirst && !RL.poly.pfirst));
+    const bool staged = small && refine_staged(c, np);   // then nothing is read back before the rows are there
+    if (staged) refine_stages(c, PL.poly, RL.poly, pa, pb, np, rp, ro);
+    else s.heavy += refine_pairs(c, PL.poly, RL.poly, pa, pb, np, rp, ro, &s);
     s.refine_ms += t2.ms();
     WallTimer t3;
+    if (small) {
+      SmallRows h = compact_small(c, PL, RL, pa, pb, np, rp, ro, o.no_agg != 0);
+      GSJ_HIP(hipStreamSynchronize(stream));
+      uint64_t n_over = 0;
+      if (staged && refine_stages_finish(c, PL.poly, RL.poly, pa, pb, np, rp, ro, s, n_over)) {   // the pairs refined since change the rows
+        h = compact_small(c, PL, RL, pa, pb, np, rp, ro, o.no_agg != 0);
+        GSJ_HIP(hipStreamSynchronize(stream));
+      }
+      s.heavy += n_over;
+      const uint64_t nrows = h.total.host[0];
+      s.compact_ms += t3.ms();
+      s.hits += nrows;
+      if (nrows && cb && cb(user, h.row, h.area, h.code, (size_t)nrows)) throw Error(GSJ_E_CANCEL, "join cancelled by the row callback");
+      return;
+    }
     uint32_t* orow = c.s_out_a.as<uint32_t>(2 * np + 16);
     double* oarea = c.s_out_area.as<double>(np + 16);
     uint32_t* ocode = c.s_out_code.as<uint32_t>(np + 16);
-    if (!hooks && np <= SMALL_COPY_PAIRS && (o.no_agg || (!PL.poly.pfirst && !RL.poly.pfirst))) {
-      uint32_t* hrow = nullptr;
-      double* harea = nullptr;
-      uint32_t* hcode = nullptr;
-      const uint64_t nrows = compact_copy_small(c, PL, RL, pa, pb, np, rp, ro, o.no_agg != 0, orow, oarea, ocode, hrow, harea, hcode);
-      s.compact_ms += t3.ms();
-      s.hits += nrows;
-      if (nrows && cb && cb(user, hrow, harea, hcode, (size_t)nrows)) throw Error(GSJ_E_CANCEL, "join cancelled by the row callback");
-      return;
-    }
     const uint64_t nrows = compact_rows(c, PL, RL, pa, pb, np, rp, ro, o.no_agg != 0, orow, oarea, ocode);
     s.compact_ms += t3.ms();
     s.hits += nrows;

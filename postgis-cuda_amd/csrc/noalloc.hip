@@ -82,6 +82,7 @@ extern "C" int gsj_join_noalloc(gsj_ctx* ctx, const gsj_layer* P, const gsj_laye
     c.side = owner.side;
     for (size_t i = 0; i < sizeof c.ev / sizeof c.ev[0]; i++) c.ev[i] = owner.ev[i];
     c.cu_count = owner.cu_count;
+    c.clock_khz = owner.clock_khz;
     c.tune_from = &owner.tune;
     c.borrowed = true;
     c.dev_arena = &dev;

@@ -1,157 +1,19 @@
 // Device primitives written for CDNA (wave64): exclusive scan and a stable LSD radix sort of (u64 key, u32 value).
 //
-// Scan: reduce-then-scan over 2048-element tiles (256 threads x 8 items, one u64 running sum per thread); inputs of
-// up to 16384 elements are scanned by one block in one launch (a request's small scans cost one launch, not three).
+// Scan: scan.h. A total that the host waits for is written into pinned host memory by the scan itself, so no copy stands
+// between the scan and the wait (a copy of 8 bytes takes 3 us of the stream).
 // Radix sort: 8-bit digits, 4096-element tiles (256 threads x 16 items). Per pass one histogram kernel, one scan of
 // the digit-major histogram, one scatter kernel. Ranks inside a tile come from a wave-level "match" (8 ballots give
 // the mask of lanes holding the same digit) plus per-wave digit counts in LDS, so each element's destination is
 // computed without per-element LDS atomics and the order of equal keys is preserved. Digits that are identical in
 // every key are skipped (found from the OR / AND of all keys).
-#include "engine.h"
+#include "scan.h"
 
 namespace gsj {
 
 namespace {
 
-constexpr int SCAN_T = 256, SCAN_ITEMS = 8, SCAN_TILE = SCAN_T * SCAN_ITEMS;
 constexpr int RS_T = 256, RS_ITEMS = 16, RS_TILE = RS_T * RS_ITEMS, RS_WAVES = RS_T / 64;
-
-__device__ __forceinline__ uint64_t wave_incl_scan(uint64_t v) {
-  const int lane = threadIdx.x & 63;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    uint64_t t = __shfl_up(v, o, 64);
-    if (lane >= o) v += t;
-  }
-  return v;
-}
-
-// block-wide exclusive scan of one value per thread (blockDim == SCAN_T); returns exclusive prefix, *total = sum
-__device__ __forceinline__ uint64_t block_excl_scan(uint64_t v, uint64_t* total) {
-  __shared__ uint64_t wsum[SCAN_T / 64];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  uint64_t inc = wave_incl_scan(v);
-  if (lane == 63) wsum[w] = inc;
-  __syncthreads();
-  uint64_t base = 0, tot = 0;
-#pragma unroll
-  for (int k = 0; k < SCAN_T / 64; k++) {
-    if (k < w) base += wsum[k];
-    tot += wsum[k];
-  }
-  __syncthreads();
-  *total = tot;
-  return base + inc - v;
-}
-
-template <class TI>
-__global__ void __launch_bounds__(SCAN_T) k_tile_sums(const TI* in, uint64_t n, uint64_t* sums) {
-  const uint64_t base = (uint64_t)blockIdx.x * SCAN_TILE;
-  uint64_t s = 0;
-#pragma unroll
-  for (int k = 0; k < SCAN_ITEMS; k++) {
-    uint64_t i = base + (uint64_t)k * SCAN_T + threadIdx.x;
-    if (i < n) s += (uint64_t)in[i];
-  }
-  uint64_t tot;
-  (void)block_excl_scan(s, &tot);
-  if (threadIdx.x == 0) sums[blockIdx.x] = tot;
-}
-
-// single block: exclusive scan of nb tile sums in place; grand total to *total
-__global__ void __launch_bounds__(SCAN_T) k_scan_sums(uint64_t* sums, uint64_t nb, uint64_t* total) {
-  uint64_t carry = 0;
-  for (uint64_t base = 0; base < nb; base += SCAN_T) {
-    uint64_t i = base + threadIdx.x;
-    uint64_t v = i < nb ? sums[i] : 0;
-    uint64_t tot;
-    uint64_t ex = block_excl_scan(v, &tot);
-    if (i < nb) sums[i] = carry + ex;
-    carry += tot;
-  }
-  if (threadIdx.x == 0 && total) *total = carry;
-}
-
-template <class TI, class TO>
-__global__ void __launch_bounds__(SCAN_T) k_tile_scan(const TI* in, TO* out, uint64_t n, const uint64_t* offs) {
-  const uint64_t base = (uint64_t)blockIdx.x * SCAN_TILE + (uint64_t)threadIdx.x * SCAN_ITEMS;   // contiguous per thread
-  uint64_t v[SCAN_ITEMS];
-  uint64_t s = 0;
-#pragma unroll
-  for (int k = 0; k < SCAN_ITEMS; k++) {
-    uint64_t i = base + k;
-    v[k] = i < n ? (uint64_t)in[i] : 0;
-    s += v[k];
-  }
-  uint64_t tot;
-  uint64_t ex = block_excl_scan(s, &tot) + offs[blockIdx.x];
-#pragma unroll
-  for (int k = 0; k < SCAN_ITEMS; k++) {
-    uint64_t i = base + k;
-    if (i < n) out[i] = (TO)ex;
-    ex += v[k];
-  }
-}
-
-// one block: exclusive scan of n <= SS_MAX elements (thread t holds elements [SS_ITEMS t, SS_ITEMS (t + 1))); every
-// element is read before the barrier and written after it, so in and out may be the same array
-constexpr int SS_T = 1024, SS_ITEMS = 16, SS_MAX = SS_T * SS_ITEMS;
-template <class TI, class TO>
-__global__ void __launch_bounds__(SS_T) k_scan_small(const TI* in, TO* out, uint64_t n, uint64_t* total) {
-  __shared__ uint64_t wsum[SS_T / 64];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const uint64_t base = (uint64_t)threadIdx.x * SS_ITEMS;
-  uint64_t v[SS_ITEMS];
-  uint64_t s = 0;
-#pragma unroll
-  for (int k = 0; k < SS_ITEMS; k++) {
-    v[k] = base + k < n ? (uint64_t)in[base + k] : 0;
-    s += v[k];
-  }
-  const uint64_t inc = wave_incl_scan(s);
-  if (lane == 63) wsum[w] = inc;
-  __syncthreads();
-  uint64_t ex = inc - s, tot = 0;
-#pragma unroll
-  for (int k = 0; k < SS_T / 64; k++) {
-    if (k < w) ex += wsum[k];
-    tot += wsum[k];
-  }
-#pragma unroll
-  for (int k = 0; k < SS_ITEMS; k++) {
-    if (base + k < n) out[base + k] = (TO)ex;
-    ex += v[k];
-  }
-  if (threadIdx.x == 0 && total) *total = tot;
-}
-
-// tile sums for the contiguous-per-thread layout used by k_tile_scan (same tile boundaries, any order inside)
-template <class TI>
-void scan_impl(Context& c, const TI* in, void* out, bool out64, uint64_t n, uint64_t* d_total) {
-  if (n == 0) {
-    if (d_total) GSJ_HIP(hipMemsetAsync(d_total, 0, 8, c.stream));
-    return;
-  }
-  if (n <= (uint64_t)SS_MAX) {
-    if (out64)
-      hipLaunchKernelGGL((k_scan_small<TI, uint64_t>), dim3(1), dim3(SS_T), 0, c.stream, in, (uint64_t*)out, n, d_total);
-    else
-      hipLaunchKernelGGL((k_scan_small<TI, uint32_t>), dim3(1), dim3(SS_T), 0, c.stream, in, (uint32_t*)out, n, d_total);
-    GSJ_LAUNCHED();
-    return;
-  }
-  const uint64_t nb = (n + SCAN_TILE - 1) / SCAN_TILE;
-  uint64_t* sums = c.s_scal.as<uint64_t>(nb + 8);
-  hipLaunchKernelGGL(k_tile_sums<TI>, dim3((uint32_t)nb), dim3(SCAN_T), 0, c.stream, in, n, sums);
-  GSJ_LAUNCHED();
-  hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(SCAN_T), 0, c.stream, sums, nb, d_total);
-  GSJ_LAUNCHED();
-  if (out64)
-    hipLaunchKernelGGL((k_tile_scan<TI, uint64_t>), dim3((uint32_t)nb), dim3(SCAN_T), 0, c.stream, in, (uint64_t*)out, n, sums);
-  else
-    hipLaunchKernelGGL((k_tile_scan<TI, uint32_t>), dim3((uint32_t)nb), dim3(SCAN_T), 0, c.stream, in, (uint32_t*)out, n, sums);
-  GSJ_LAUNCHED();
-}
 
 // ------------------------------------------------------------------------------------------- radix sort
 __device__ __forceinline__ uint64_t lanemask_lt() {
@@ -235,16 +97,15 @@ __global__ void k_init_bits(unsigned long long* acc) { acc[0] = 0ull; acc[1] = ~
 }  // namespace
 
 uint64_t scan_u32_to_u64(Context& c, const uint32_t* in, uint64_t* out, uint64_t n) {
-  uint64_t* d_total = c.s_misc.as<uint64_t>(4);
-  scan_impl<uint32_t>(c, in, out, true, n, d_total);
-  uint64_t* h = c.h_scal.as<uint64_t>(4);
-  GSJ_HIP(hipMemcpyAsync(h, d_total, 8, hipMemcpyDeviceToHost, c.stream));
+  const HostWords w = host_words(c, 0, 1);
+  scan_loaded<uint64_t>(c, LoadArray<uint32_t>{in}, out, n, ScanTotal{w.dev, nullptr});
+  w.fetch(c);
   GSJ_HIP(hipStreamSynchronize(c.stream));
-  return h[0];
+  return w.host[0];
 }
 
 void scan_u32_to_u64_async(Context& c, const uint32_t* in, uint64_t* out, uint64_t n, uint64_t* d_total) {
-  scan_impl<uint32_t>(c, in, out, true, n, d_total);
+  scan_loaded<uint64_t>(c, LoadArray<uint32_t>{in}, out, n, ScanTotal{d_total, nullptr});
 }
 
 void key_bits(Context& c, const uint64_t* keys, uint64_t n, uint64_t& or_all, uint64_t& and_all) {
@@ -278,7 +139,7 @@ void radix_sort_pairs(Context& c, uint64_t*& keys, uint64_t*& keys_alt, uint32_t
     if (((varying >> shift) & 255u) == 0) continue;
     hipLaunchKernelGGL(k_rs_hist, dim3(ntiles), dim3(RS_T), 0, c.stream, keys, n, shift, ntiles, ghist);
     GSJ_LAUNCHED();
-    scan_impl<uint32_t>(c, ghist, ghist, false, (uint64_t)256 * ntiles, nullptr);
+    scan_loaded<uint32_t>(c, LoadArray<uint32_t>{ghist}, ghist, (uint64_t)256 * ntiles, ScanTotal{});
     hipLaunchKernelGGL(k_rs_scatter, dim3(ntiles), dim3(RS_T), 0, c.stream, keys, vals, n, shift, ntiles, ghist, keys_alt, vals_alt);
     GSJ_LAUNCHED();
     std::swap(keys, keys_alt);

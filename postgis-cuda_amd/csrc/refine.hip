@@ -21,6 +21,7 @@
 //    restatement, so a pair gives the same bits alone or batched with any other request.
 //  * FP64 on the vector ALUs only; nothing here is a dense contraction, so MFMA is not used.
 #include "pairs.h"
+#include <type_traits>
 
 namespace gsj {
 
@@ -408,10 +409,18 @@ __device__ __forceinline__ int probe_small(const SmallPoly<CAP>& sp, int r, bool
 // its waves hold only pairs with edge work (the screen's verdict travels in isect[p]).
 constexpr uint8_t ST_HIT = 1, ST_RTOUCH = 2, ST_INA = 4, ST_INB = 8;
 
+// what the host reads after the staged launches
+struct StageReport {
+  uint32_t counts[16];
+  OverflowCtl ctl[2];   // the overflow queue's, the host's queue's
+  uint64_t start[4];    // wall_clock64 at the screens, the edges, the overflow pass and the report
+};
+HostWords stage_words(Context& c) { return host_words(c, 32, sizeof(StageReport) / 8); }
+
 struct EdgeQueue {   // pairs with edge work: flag[k] per position k of the class list (set by the screen), then the
   uint32_t* flag;    // flagged pairs in class-list order: class c's at list[first[c] .. first[c] + count[c])
   uint64_t* off;
-  uint32_t* list;
+  uint32_t* list;    // (staged launches append instead: any order)
   uint32_t* count;   // [3]: tiny, small, medium
   uint32_t* first;   // [3]
 };
@@ -494,24 +503,23 @@ __device__ __forceinline__ void load_pair(const DPolys& P, const DPolys& R, uint
   wave_lds_sync();
 }
 
-template <int G, int CAP, int WHICH, int OCC>
-__global__ void __launch_bounds__(256, OCC) k_screen_small(const DPolys P, const DPolys R, const uint32_t* __restrict__ pa, const uint32_t* __restrict__ pb,
-                                                      const uint32_t* __restrict__ list, const uint32_t* __restrict__ counts, RefineParams rp,
-                                                      RefineOut out, EdgeQueue q) {
-  extern __shared__ __align__(16) unsigned char smem[];
+// The screens of class WHICH's pairs first, first + stride, ... of its list, by a G-lane group with SA / SB in LDS.
+// Pairs with edge work are flagged by list position, or (APPEND) appended to the class's part of q.list at once.
+template <int G, int CAP, int WHICH, bool APPEND>
+__device__ __forceinline__ void screen_loop(const DPolys& P, const DPolys& R, const uint32_t* __restrict__ pa, const uint32_t* __restrict__ pb,
+                                            const uint32_t* __restrict__ list, const uint32_t* __restrict__ counts, const RefineParams& rp,
+                                            const RefineOut& out, const EdgeQueue& q, SmallPoly<CAP>& SA, SmallPoly<CAP>& SB, int gl, uint32_t first,
+                                            uint32_t stride) {
   using SP = SmallPoly<CAP>;
-  const int gpb = blockDim.x / G;
-  const int gib = threadIdx.x / G, gl = threadIdx.x % G;
   const bool rel = rp.want_relate != 0;
-  SP& SA = *reinterpret_cast<SP*>(smem + (size_t)gib * 2 * sizeof(SP));
-  SP& SB = *(&SA + 1);
   const uint32_t nlist = counts[WHICH];
   const uint32_t base = class_first(counts, WHICH);
   const uint32_t* cl = list + base;
-  PairStream ps(cl, pa, pb, nlist, blockIdx.x * gpb + gib, gridDim.x * gpb);
+  PairStream ps(cl, pa, pb, nlist, first, stride);
   for (; ps.k < nlist; ps.advance()) {
     ps.prefetch();
-    const uint32_t k = ps.k, p = ps.p, a = ps.a, b = ps.b;
+    const uint32_t p = ps.p, a = ps.a, b = ps.b;
+    [[maybe_unused]] const uint32_t k = ps.k;
     const uint32_t ra = P.pk_off[a], rb = R.pk_off[b];   // record offsets (32-bit: fewer registers than pointers)
     const PairSetup f = setup_pair_rec(P.pk + ra, R.pk + rb, rp);
     const bool self = is_self(P, R, a, b);
@@ -569,21 +577,35 @@ __global__ void __launch_bounds__(256, OCC) k_screen_small(const DPolys P, const
     } else if (gl == 0) {
       out.isect[p] = (hit ? ST_HIT : 0) | (rtouch ? ST_RTOUCH : 0) | (inA_c ? ST_INA : 0) | (inB_c ? ST_INB : 0);
     }
-    if (gl == 0) q.flag[base + k] = computed ? 1u : 0u;
+    if constexpr (APPEND) {
+      if (gl == 0 && computed) q.list[base + atomicAdd(&q.count[WHICH], 1u)] = p;
+    } else {
+      if (gl == 0) q.flag[base + k] = computed ? 1u : 0u;
+    }
     wave_lds_sync();
   }
 }
 
-template <int G, int CAP, int WHICH>
-__global__ void __launch_bounds__(256, 3) k_edges_small(const DPolys P, const DPolys R, const uint32_t* __restrict__ pa, const uint32_t* __restrict__ pb,
-                                                        const uint32_t* __restrict__ counts, RefineParams rp, RefineOut out, EdgeQueue q,
-                                                        uint32_t* __restrict__ ovf_list, OverflowCtl* ctl) {
+template <int G, int CAP, int WHICH, int OCC>
+__global__ void __launch_bounds__(256, OCC) k_screen_small(const DPolys P, const DPolys R, const uint32_t* __restrict__ pa, const uint32_t* __restrict__ pb,
+                                                      const uint32_t* __restrict__ list, const uint32_t* __restrict__ counts, RefineParams rp,
+                                                      RefineOut out, EdgeQueue q) {
   extern __shared__ __align__(16) unsigned char smem[];
   using SP = SmallPoly<CAP>;
   const int gpb = blockDim.x / G;
   const int gib = threadIdx.x / G, gl = threadIdx.x % G;
+  SP& SA = *reinterpret_cast<SP*>(smem + (size_t)gib * 2 * sizeof(SP));
+  screen_loop<G, CAP, WHICH, false>(P, R, pa, pb, list, counts, rp, out, q, SA, *(&SA + 1), gl, blockIdx.x * gpb + gib, gridDim.x * gpb);
+}
+
+// The edge work of class WHICH's queued pairs first, first + stride, ..., by a G-lane group with small_bytes<CAP>(rel)
+// bytes of LDS at gbase
+template <int G, int CAP, int WHICH>
+__device__ __forceinline__ void edges_loop(const DPolys& P, const DPolys& R, const uint32_t* __restrict__ pa, const uint32_t* __restrict__ pb,
+                                           const RefineParams& rp, const RefineOut& out, const EdgeQueue& q, uint32_t* __restrict__ ovf_list,
+                                           OverflowCtl* ctl, unsigned char* gbase, int gl, uint32_t first, uint32_t stride) {
+  using SP = SmallPoly<CAP>;
   const bool rel = rp.want_relate != 0;
-  unsigned char* gbase = smem + (size_t)gib * small_bytes<CAP>(rel);
   SP& SA = *reinterpret_cast<SP*>(gbase);
   SP& SB = *(reinterpret_cast<SP*>(gbase) + 1);
   double* acc = reinterpret_cast<double*>(gbase + ((2 * sizeof(SP) + 15) & ~size_t(15)));
@@ -591,7 +613,7 @@ __global__ void __launch_bounds__(256, 3) k_edges_small(const DPolys P, const DP
   double* lon = lin + 2 * CAP;
   const uint32_t nlist = q.count[WHICH];
   const uint32_t* cl = q.list + q.first[WHICH];
-  PairStream ps(cl, pa, pb, nlist, blockIdx.x * gpb + gib, gridDim.x * gpb);
+  PairStream ps(cl, pa, pb, nlist, first, stride);
   for (; ps.k < nlist; ps.advance()) {
     ps.prefetch();
     const uint32_t p = ps.p, a = ps.a, b = ps.b;
@@ -630,6 +652,17 @@ __global__ void __launch_bounds__(256, 3) k_edges_small(const DPolys P, const DP
     }
     wave_lds_sync();
   }
+}
+
+template <int G, int CAP, int WHICH>
+__global__ void __launch_bounds__(256, 3) k_edges_small(const DPolys P, const DPolys R, const uint32_t* __restrict__ pa, const uint32_t* __restrict__ pb,
+                                                        const uint32_t* __restrict__ counts, RefineParams rp, RefineOut out, EdgeQueue q,
+                                                        uint32_t* __restrict__ ovf_list, OverflowCtl* ctl) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int gpb = blockDim.x / G;
+  const int gib = threadIdx.x / G, gl = threadIdx.x % G;
+  edges_loop<G, CAP, WHICH>(P, R, pa, pb, rp, out, q, ovf_list, ctl, smem + (size_t)gib * small_bytes<CAP>(rp.want_relate != 0), gl,
+                            blockIdx.x * gpb + gib, gridDim.x * gpb);
 }
 
 // the flagged pairs of the vertex-list classes (tiny, small, medium) in class-list order (stable compaction of the
@@ -742,18 +775,13 @@ __device__ bool refine_lists(const DPolys& P, const DPolys& R, uint32_t a, uint3
 
 // large class: a wave per pair, compacted lists in LDS (cap edges per side); overflowing pairs are queued. Its pairs
 // are the partition's last class followed by the mixed pairs promoted because their lists outgrew the mixed class.
-__global__ void __launch_bounds__(256, 3) k_refine_large(const DPolys P, const DPolys R, const uint32_t* __restrict__ pa, const uint32_t* __restrict__ pb,
-                                                      const uint32_t* __restrict__ list, const uint32_t* __restrict__ counts, const uint32_t* __restrict__ promo,
-                                                      const OverflowCtl* __restrict__ promo_ctl, RefineParams rp, RefineOut out, int cap,
-                                                      uint32_t* __restrict__ ovf_list, OverflowCtl* ctl) {
-  extern __shared__ __align__(16) unsigned char smem[];
-  const int wpb = blockDim.x / 64;
-  const int wib = threadIdx.x / 64, gl = threadIdx.x % 64;
-  const bool rel = rp.want_relate != 0;
-  const Scratch S = carve(smem + (size_t)wib * list_bytes(cap, rel), cap, rel);
+__device__ __forceinline__ void large_loop(const DPolys& P, const DPolys& R, const uint32_t* __restrict__ pa, const uint32_t* __restrict__ pb,
+                                           const uint32_t* __restrict__ list, const uint32_t* __restrict__ counts, const uint32_t* __restrict__ promo,
+                                           const OverflowCtl* __restrict__ promo_ctl, const RefineParams& rp, const RefineOut& out, int cap,
+                                           uint32_t* __restrict__ ovf_list, OverflowCtl* ctl, const Scratch& S, int gl, uint32_t first, uint32_t stride) {
   const uint32_t nclass = counts[CL_LARGE], nlist = nclass + promo_ctl->count;
   const uint32_t* large = list + class_first(counts, CL_LARGE);   // the large class comes last
-  for (uint32_t k = blockIdx.x * wpb + wib; k < nlist; k += gridDim.x * wpb) {
+  for (uint32_t k = first; k < nlist; k += stride) {
     const uint32_t p = k < nclass ? large[k] : promo[k - nclass];
     const uint32_t a = pa[p], b = pb[p];
     const PairSetup f = setup_pair(P, R, a, b, rp);
@@ -768,26 +796,33 @@ __global__ void __launch_bounds__(256, 3) k_refine_large(const DPolys P, const D
     wave_lds_sync();
   }
 }
+__global__ void __launch_bounds__(256, 3) k_refine_large(const DPolys P, const DPolys R, const uint32_t* __restrict__ pa, const uint32_t* __restrict__ pb,
+                                                      const uint32_t* __restrict__ list, const uint32_t* __restrict__ counts, const uint32_t* __restrict__ promo,
+                                                      const OverflowCtl* __restrict__ promo_ctl, RefineParams rp, RefineOut out, int cap,
+                                                      uint32_t* __restrict__ ovf_list, OverflowCtl* ctl) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int wpb = blockDim.x / 64;
+  const int wib = threadIdx.x / 64, gl = threadIdx.x % 64;
+  const bool rel = rp.want_relate != 0;
+  large_loop(P, R, pa, pb, list, counts, promo, promo_ctl, rp, out, cap, ovf_list, ctl, carve(smem + (size_t)wib * list_bytes(cap, rel), cap, rel), gl,
+             blockIdx.x * wpb + wib, gridDim.x * wpb);
+}
 
 // mixed class (one polygon small, the other large): a 16-lane group per pair, compacted lists of CAP_MIXED edges per
 // side in LDS (the large polygon's edges meeting the overlap box, found through its edge-chunk boxes); pairs whose
 // lists overflow are queued
-constexpr int CAP_MIXED = 32, MIXED_T = 128;
+constexpr int CAP_MIXED = 32, MIXED_T = 128, MIXED_G = 16;
+constexpr uint32_t MIXED_WAVE_ROUNDS = 1;
 constexpr uint32_t OVF_LDS_CAP = 448;   // overflow lists up to this many edges per side go to LDS (448 x 128 B = 56 KiB)
 constexpr uint32_t OVF_SIDE_CAP = 256;  // the list classes' own overflow launch (ovf_lds 2): LDS lists of up to 256 edges
-__global__ void __launch_bounds__(MIXED_T) k_refine_mixed(const DPolys P, const DPolys R, const uint32_t* __restrict__ pa, const uint32_t* __restrict__ pb,
-                                                          const uint32_t* __restrict__ list, const uint32_t* __restrict__ counts, RefineParams rp,
-                                                          RefineOut out, uint32_t* __restrict__ promo, OverflowCtl* promo_ctl,
-                                                          uint32_t* __restrict__ ovf_list, OverflowCtl* ctl) {
-  extern __shared__ __align__(16) unsigned char smem[];
-  constexpr int G = 16;
-  const int gpb = blockDim.x / G;
-  const int gib = threadIdx.x / G, gl = threadIdx.x % G;
-  const bool rel = rp.want_relate != 0;
-  const Scratch S = carve(smem + (size_t)gib * list_bytes(CAP_MIXED, rel), CAP_MIXED, rel);
+template <int G>
+__device__ __forceinline__ void mixed_loop(const DPolys& P, const DPolys& R, const uint32_t* __restrict__ pa, const uint32_t* __restrict__ pb,
+                                           const uint32_t* __restrict__ list, const uint32_t* __restrict__ counts, const RefineParams& rp,
+                                           const RefineOut& out, uint32_t* __restrict__ promo, OverflowCtl* promo_ctl, uint32_t* __restrict__ ovf_list,
+                                           OverflowCtl* ctl, const Scratch& S, int gl, uint32_t first, uint32_t stride) {
   const uint32_t nlist = counts[CL_MIXED];
   const uint32_t* cl = list + class_first(counts, CL_MIXED);
-  for (uint32_t k = blockIdx.x * gpb + gib; k < nlist; k += gridDim.x * gpb) {
+  for (uint32_t k = first; k < nlist; k += stride) {
     const uint32_t p = cl[k];
     const uint32_t a = pa[p], b = pb[p];
     const PairSetup f = setup_pair(P, R, a, b, rp);
@@ -802,6 +837,17 @@ __global__ void __launch_bounds__(MIXED_T) k_refine_mixed(const DPolys P, const 
     wave_lds_sync();
   }
 }
+__global__ void __launch_bounds__(MIXED_T) k_refine_mixed(const DPolys P, const DPolys R, const uint32_t* __restrict__ pa, const uint32_t* __restrict__ pb,
+                                                          const uint32_t* __restrict__ list, const uint32_t* __restrict__ counts, RefineParams rp,
+                                                          RefineOut out, uint32_t* __restrict__ promo, OverflowCtl* promo_ctl,
+                                                          uint32_t* __restrict__ ovf_list, OverflowCtl* ctl) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int gpb = blockDim.x / MIXED_G;
+  const int gib = threadIdx.x / MIXED_G, gl = threadIdx.x % MIXED_G;
+  const bool rel = rp.want_relate != 0;
+  mixed_loop<MIXED_G>(P, R, pa, pb, list, counts, rp, out, promo, promo_ctl, ovf_list, ctl, carve(smem + (size_t)gib * list_bytes(CAP_MIXED, rel), CAP_MIXED, rel),
+             gl, blockIdx.x * gpb + gib, gridDim.x * gpb);
+}
 
 // overflow: a block of T threads per pair (T = 64: one wave), lists and partial sums in LDS when the launch's largest
 // lists fit (IN_LDS; the edge loops then read LDS instead of global memory), else in a per-block slab of global
@@ -813,13 +859,14 @@ __global__ void __launch_bounds__(MIXED_T) k_refine_mixed(const DPolys P, const 
 // the pair and on values the block has read back from shared memory after a barrier).
 // With `dev_n` the queue length is read on the device (a launch enqueued behind the kernels that fill the queue, with
 // no host read in between), and with `defer` a pair whose lists exceed `cap` is handed on to that queue (its count
-// of such pairs kept in dev_n->pad0) instead of being refined here.
+// of such pairs kept in dev_n->pad0) instead of being refined here. start (or null) takes the launch's start time.
 template <int T, bool IN_LDS>
 __global__ void __launch_bounds__(T) k_refine_overflow(const DPolys P, const DPolys R, const uint32_t* __restrict__ pa, const uint32_t* __restrict__ pb,
                                                            const uint32_t* __restrict__ list, uint32_t nlist, RefineParams rp, RefineOut out, int cap,
                                                            unsigned char* __restrict__ slab, OverflowCtl* dev_n, uint32_t* __restrict__ defer_list,
-                                                           OverflowCtl* defer) {
+                                                           OverflowCtl* defer, uint64_t* start) {
   extern __shared__ __align__(16) unsigned char smem[];
+  if (start && blockIdx.x == 0 && threadIdx.x == 0) *start = wall_clock64();
   __shared__ int s_na, s_nb, s_hit, s_hit_any, s_found, s_contain, s_inA, s_inB;   // s_hit: contact; s_found: contact or containment
   __shared__ int s_defer;
   __shared__ uint32_t s_bits;
@@ -947,11 +994,247 @@ void launch_screens(uint32_t gt, uint32_t gs, uint32_t gm, hipStream_t st, const
 }
 }  // namespace
 
+namespace {
+
+// the host-read overflow queue: nover pairs whose longest lists need `need` edges per side
+void overflow_launch(Context& c, const DPolys& P, const DPolys& R, const uint32_t* pa, const uint32_t* pb, const uint32_t* list, uint32_t nover,
+                     uint32_t need, const RefineParams& rp, const RefineOut& out, bool in_lds, gsj_join_stats* stats) {
+  hipStream_t st = c.stream;
+  const bool rel = rp.want_relate != 0;
+  if (in_lds && need <= OVF_LDS_CAP) {   // lists in LDS: no slab
+    const size_t lds = list_bytes((int)need, rel);
+    GSJ_HIP(hipEventRecord(c.ev[3], st));
+    // pairs too few to fill the GPU (a windowed request's few largest): eight waves each, so that the edge
+    // contributions of both lists (up to 2 x 448 edges) take one or two rounds
+    const bool few = nover <= (uint64_t)c.cu_count;
+    const uint32_t blocks = (uint32_t)std::min<uint64_t>(nover, (uint64_t)c.cu_count * (few ? 1 : 8));
+    if (few)
+      hipLaunchKernelGGL((k_refine_overflow<512, true>), dim3(blocks), dim3(512), lds, st, P, R, pa, pb, list, nover, rp, out, (int)need, nullptr, nullptr, nullptr, nullptr, nullptr);
+    else
+      hipLaunchKernelGGL((k_refine_overflow<64, true>), dim3(blocks), dim3(64), lds, st, P, R, pa, pb, list, nover, rp, out, (int)need, nullptr, nullptr, nullptr, nullptr, nullptr);
+    GSJ_LAUNCHED();
+    GSJ_HIP(hipEventRecord(c.ev[4], st));
+    if (stats) {
+      GSJ_HIP(hipEventSynchronize(c.ev[4]));
+      float ms_o = 0;
+      GSJ_HIP(hipEventElapsedTime(&ms_o, c.ev[3], c.ev[4]));
+      stats->k_over_ms += ms_o;
+    }
+  } else {
+    const size_t per = list_bytes((int)need, rel);
+    // slabs of at most 1 GiB (half of what is left when the scratch is a fixed arena: compaction still needs room)
+    const uint64_t budget = c.dev_arena ? std::min<uint64_t>(1ull << 30, c.dev_arena->left() / 2) : (1ull << 30);
+    GSJ_REQUIRE(!c.dev_arena || per <= budget, GSJ_E_LIMIT, "overflow pair lists exceed the no-allocation scratch left for them");
+    const uint64_t blocks = std::max<uint64_t>(1, std::min<uint64_t>(nover, budget / std::max<size_t>(per, 1)));   // one slab per block
+    unsigned char* slab = c.s_heavy_edges.as<unsigned char>(per * blocks + 64);
+    GSJ_HIP(hipEventRecord(c.ev[3], st));
+    if (nover <= 2ull * c.cu_count)   // a few pairs: four waves each (2.4M relate: one wave each, 2.5 vs 4.5 ms)
+      hipLaunchKernelGGL((k_refine_overflow<256, false>), dim3((uint32_t)blocks), dim3(256), 0, st, P, R, pa, pb, list, nover, rp, out, (int)need, slab, nullptr, nullptr, nullptr, nullptr);
+    else
+      hipLaunchKernelGGL((k_refine_overflow<64, false>), dim3((uint32_t)blocks), dim3(64), 0, st, P, R, pa, pb, list, nover, rp, out, (int)need, slab, nullptr, nullptr, nullptr, nullptr);
+    GSJ_LAUNCHED();
+    GSJ_HIP(hipEventRecord(c.ev[4], st));
+    if (stats) {
+      GSJ_HIP(hipEventSynchronize(c.ev[4]));
+      float ms_o = 0;
+      GSJ_HIP(hipEventElapsedTime(&ms_o, c.ev[3], c.ev[4]));
+      stats->k_over_ms += ms_o;
+    }
+  }
+}
+
+}  // namespace
+
+namespace {
+
+// ---- launches of few candidates: two stages for all classes
+// A request of a few thousand candidates spends its time between kernels, not in them: a launch takes about 3 us of the
+// stream, a timing event 4, a fork to a second stream and back 20. So every class runs in the same two launches (the mixed
+// class and the screens, then the large class and the edge work of the pairs the screens appended), the overflow queue is
+// emptied by a third that reads its length on the device, and the host waits once, at the end, for the rows, the class
+// sizes, the queues' state and the launches' start times together. Blocks are single waves; each walks the classes
+// longest pairs first, and a class's pairs start at the block where the previous class's end, so that a few pairs of
+// each class spread over the grid. 143 parcels x 4 regions with areas: 21 launches, 14 events, 6 copies and 3 waits ->
+// 9 launches and 2 waits, 195 -> 94 us; 10k parcels x 16 regions 271 -> 160 us. Up to STAGED_MAX pairs: a launch of 200k
+// pairs is slower this way (1.17 -> 1.72 ms as one subdivided self relate), its kernels being long enough to profit
+// from registers and LDS of their own, and from the second stream.
+struct StageArgs {
+  DPolys P, R;
+  const uint32_t* pa;
+  const uint32_t* pb;
+  const uint32_t* list;
+  const uint32_t* counts;
+  uint32_t* promo;
+  OverflowCtl* promo_ctl;
+  uint32_t* ovf;
+  OverflowCtl* ctl;
+  RefineParams rp;
+  RefineOut out;
+  EdgeQueue q;
+  int cap_large;
+  uint64_t* start;   // start times of the stages (wall_clock64)
+};
+
+// first item of this block's group gib (of gpb) among a class's n items, when the classes before it took `used` blocks
+__device__ __forceinline__ uint32_t stage_first(uint32_t& used, uint32_t n, uint32_t gpb, uint32_t gib) {
+  const uint32_t nb = gridDim.x, shift = used % nb, b = blockIdx.x >= shift ? blockIdx.x - shift : blockIdx.x + nb - shift;
+  used += (n + gpb - 1) / gpb;
+  return b * gpb + gib;
+}
+
+__global__ void __launch_bounds__(64, 3) k_stage_screens(const StageArgs A) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  if (blockIdx.x == 0 && threadIdx.x == 0) A.start[0] = wall_clock64();
+  const bool rel = A.rp.want_relate != 0;
+  const uint32_t* n = A.counts;
+  uint32_t used = 0;
+  auto mixed = [&](auto g_) {
+    constexpr int G = decltype(g_)::value;
+    const int g = threadIdx.x / G, gl = threadIdx.x % G, gpb = 64 / G;
+    const uint32_t f = stage_first(used, n[CL_MIXED], gpb, g);
+    mixed_loop<G>(A.P, A.R, A.pa, A.pb, A.list, n, A.rp, A.out, A.promo, A.promo_ctl, A.ovf, A.ctl,
+                  carve(smem + (size_t)g * list_bytes(CAP_MIXED, rel), CAP_MIXED, rel), gl, f, gridDim.x * gpb);
+  };
+  // one round of whole waves finishes sooner than one of quarter waves (165 pairs: the stage 30 -> 23 us), several do
+  // not (10.6k pairs in four rounds: the request 166 -> 198 us)
+  if (n[CL_MIXED] <= MIXED_WAVE_ROUNDS * gridDim.x) mixed(std::integral_constant<int, 64>{});
+  else mixed(std::integral_constant<int, MIXED_G>{});
+  auto screens = [&](auto g_, auto cap_, auto cl_) {
+    constexpr int G = decltype(g_)::value, CAP = decltype(cap_)::value, CL = decltype(cl_)::value;
+    using SP = SmallPoly<CAP>;
+    const int g = threadIdx.x / G, gl = threadIdx.x % G, gpb = 64 / G;
+    SP& SA = *reinterpret_cast<SP*>(smem + (size_t)g * 2 * sizeof(SP));
+    const uint32_t f = stage_first(used, n[CL], gpb, g);
+    screen_loop<G, CAP, CL, true>(A.P, A.R, A.pa, A.pb, A.list, n, A.rp, A.out, A.q, SA, *(&SA + 1), gl, f, gridDim.x * gpb);
+  };
+  wave_lds_sync();   // the classes' LDS overlaps; a block is one wave
+  screens(std::integral_constant<int, 32>{}, std::integral_constant<int, MCAP>{}, std::integral_constant<int, CL_MEDIUM>{});
+  wave_lds_sync();
+  screens(std::integral_constant<int, 16>{}, std::integral_constant<int, VCAP>{}, std::integral_constant<int, CL_SMALL>{});
+  wave_lds_sync();
+  screens(std::integral_constant<int, 8>{}, std::integral_constant<int, TCAP>{}, std::integral_constant<int, CL_TINY>{});
+}
+
+__global__ void __launch_bounds__(64, 3) k_stage_edges(const StageArgs A) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  if (blockIdx.x == 0 && threadIdx.x == 0) A.start[1] = wall_clock64();
+  const bool rel = A.rp.want_relate != 0;
+  const uint32_t* n = A.counts;
+  uint32_t used = 0;
+  {
+    const uint32_t f = stage_first(used, n[CL_LARGE] + A.promo_ctl->count, 1, 0);
+    large_loop(A.P, A.R, A.pa, A.pb, A.list, n, A.promo, A.promo_ctl, A.rp, A.out, A.cap_large, A.ovf, A.ctl, carve(smem, A.cap_large, rel), threadIdx.x, f,
+               gridDim.x);
+  }
+  auto edges = [&](auto g_, auto cap_, auto cl_) {
+    constexpr int G = decltype(g_)::value, CAP = decltype(cap_)::value, CL = decltype(cl_)::value;
+    const int g = threadIdx.x / G, gl = threadIdx.x % G, gpb = 64 / G;
+    const uint32_t f = stage_first(used, A.q.count[CL], gpb, g);
+    edges_loop<G, CAP, CL>(A.P, A.R, A.pa, A.pb, A.rp, A.out, A.q, A.ovf, A.ctl, smem + (size_t)g * small_bytes<CAP>(rel), gl, f, gridDim.x * gpb);
+  };
+  wave_lds_sync();
+  edges(std::integral_constant<int, 32>{}, std::integral_constant<int, MCAP>{}, std::integral_constant<int, CL_MEDIUM>{});
+  wave_lds_sync();
+  edges(std::integral_constant<int, 16>{}, std::integral_constant<int, VCAP>{}, std::integral_constant<int, CL_SMALL>{});
+  wave_lds_sync();
+  edges(std::integral_constant<int, 8>{}, std::integral_constant<int, TCAP>{}, std::integral_constant<int, CL_TINY>{});
+}
+
+// class sizes, edge queue sizes, queue controls and stage start times into the host's words
+__global__ void k_stage_report(const uint32_t* __restrict__ counts, const OverflowCtl* __restrict__ ctl, uint64_t* start, StageReport* __restrict__ out) {
+  const int t = threadIdx.x;
+  if (t == 0) { start[3] = wall_clock64(); out->start[3] = start[3]; }
+  if (t < 16) out->counts[t] = counts[t];
+  if (t < 2) out->ctl[t] = ctl[t];
+  if (t < 3) out->start[t] = start[t];
+}
+
+// LDS of the two stages' single-wave blocks
+constexpr size_t stage_screen_bytes(bool rel) {
+  return std::max(std::max((64 / MIXED_G) * list_bytes(CAP_MIXED, rel), size_t(8) * 2 * sizeof(SmallPoly<TCAP>)),
+                  std::max(size_t(4) * 2 * sizeof(SmallPoly<VCAP>), size_t(2) * 2 * sizeof(SmallPoly<MCAP>)));
+}
+inline size_t stage_edge_bytes(bool rel, int cap_large) {
+  return std::max(std::max(list_bytes(std::max(cap_large, 1), rel), 8 * small_bytes<TCAP>(rel)),
+                  std::max(4 * small_bytes<VCAP>(rel), 2 * small_bytes<MCAP>(rel)));
+}
+
+}  // namespace
+
+bool refine_staged(const Context& c, uint64_t np) { return np <= STAGED_MAX && c.shape(np).ovf_lds != 0; }
+
+void refine_stages(Context& c, const DPolys& P, const DPolys& R, const uint32_t* pa, const uint32_t* pb, uint64_t np, const RefineParams& rp,
+                   const RefineOut& out) {
+  hipStream_t st = c.stream;
+  const bool rel = rp.want_relate != 0;
+  const LaunchShape& sh = c.shape(np);
+  const PairClasses pc = partition_pairs(c, P, R, pa, pb, np, sh.mcap, sh.mixed != 0, sh.tcap, sh.size_sort);
+  StageArgs A{};
+  A.P = P; A.R = R; A.pa = pa; A.pb = pb; A.list = pc.list; A.counts = pc.counts; A.rp = rp; A.out = out;
+  A.ovf = c.s_heavy.as<uint32_t>(3 * np + 192);
+  A.ctl = pc.ctl;
+  A.promo = A.ovf + np + 64;
+  A.promo_ctl = pc.ctl + 4;
+  uint32_t* ovf_main = A.promo + np + 64;   // lists beyond OVF_LDS_CAP, for the host
+  A.q.list = c.s_edgeq.as<uint32_t>(2 * np + 32);
+  A.q.count = pc.counts + 8;
+  A.q.first = pc.counts + 11;   // where each class's part of q.list starts (the partition leaves it there)
+  A.cap_large = (int)sh.large_cap;
+  A.start = pc.start;
+  const uint32_t cu = (uint32_t)c.cu_count;
+  // a wave per two pairs at most (the medium class) in the first stage, per pair in the second (the large class); 12 of
+  // these waves fit a CU by their registers, fewer by the mixed class's lists
+  hipLaunchKernelGGL(k_stage_screens, dim3((uint32_t)std::min<uint64_t>(np, cu * 12)), dim3(64), stage_screen_bytes(rel), st, A);
+  GSJ_LAUNCHED();
+  hipLaunchKernelGGL(k_stage_edges, dim3((uint32_t)std::min<uint64_t>(np, cu * 12)), dim3(64), stage_edge_bytes(rel, A.cap_large), st, A);
+  GSJ_LAUNCHED();
+  // few pairs, eight waves each (see the host-sized launch below); longer lists go on to the host's queue
+  hipLaunchKernelGGL((k_refine_overflow<512, true>), dim3((uint32_t)std::min<uint64_t>(np, cu)), dim3(512), list_bytes(OVF_LDS_CAP, rel), st, P, R, pa, pb,
+                     A.ovf, 0u, rp, out, (int)OVF_LDS_CAP, nullptr, A.ctl, ovf_main, A.ctl + 1, A.start + 2);
+  GSJ_LAUNCHED();
+  const HostWords w = stage_words(c);
+  hipLaunchKernelGGL(k_stage_report, dim3(1), dim3(64), 0, st, pc.counts, pc.ctl, A.start, reinterpret_cast<StageReport*>(w.dev));
+  GSJ_LAUNCHED();
+  w.fetch(c);
+}
+
+bool refine_stages_finish(Context& c, const DPolys& P, const DPolys& R, const uint32_t* pa, const uint32_t* pb, uint64_t np, const RefineParams& rp,
+                          const RefineOut& out, gsj_join_stats& s, uint64_t& n_over) {
+  const StageReport r = *reinterpret_cast<const StageReport*>(stage_words(c).host);
+  const uint32_t handed = r.ctl[1].count;   // pairs whose lists exceed OVF_LDS_CAP
+  n_over = r.ctl[0].count;                  // (they are counted in it too)
+  auto ms = [&](int k) { return (double)(r.start[k + 1] - r.start[k]) / c.clock_khz; };
+  const double m0 = ms(0), m1 = ms(1), m2 = ms(2);
+  s.n_tiny += r.counts[CL_TINY]; s.n_small += r.counts[CL_SMALL]; s.n_medium += r.counts[CL_MEDIUM]; s.n_mixed += r.counts[CL_MIXED];
+  s.n_large += r.counts[CL_LARGE];
+  s.n_tiny_edge += r.counts[8 + CL_TINY]; s.n_small_edge += r.counts[8 + CL_SMALL]; s.n_medium_edge += r.counts[8 + CL_MEDIUM];
+  // the classes of a stage run side by side: each that had pairs reports the stage's time
+  if (r.counts[CL_MIXED]) s.k_mixed_ms += m0;
+  if (r.counts[CL_TINY] + r.counts[CL_SMALL] + r.counts[CL_MEDIUM]) s.k_screen_ms += m0;
+  if (r.counts[CL_LARGE]) s.k_large_ms += m1;
+  if (r.counts[8 + CL_TINY]) s.k_tiny_ms += m1;
+  if (r.counts[8 + CL_SMALL]) s.k_small_ms += m1;
+  if (r.counts[8 + CL_MEDIUM]) s.k_medium_ms += m1;
+  if (n_over) s.k_over_ms += m2;
+  s.n_over += n_over;
+  s.launches++;
+  if (handed) overflow_launch(c, P, R, pa, pb, c.s_heavy.as<uint32_t>(3 * np + 192) + 2 * (np + 64), handed, r.ctl[1].need, rp, out, false, &s);
+  return handed != 0;
+}
+
 uint64_t refine_pairs(Context& c, const DPolys& P, const DPolys& R, const uint32_t* pa, const uint32_t* pb, uint64_t np, const RefineParams& rp,
                       const RefineOut& out, gsj_join_stats* stats) {
   if (np == 0) return 0;
   GSJ_REQUIRE(np < (1ull << 32), GSJ_E_LIMIT, "refine: more than 2^32 pairs in one launch");
   hipStream_t st = c.stream;
+  if (refine_staged(c, np)) {
+    refine_stages(c, P, R, pa, pb, np, rp, out);
+    GSJ_HIP(hipStreamSynchronize(st));
+    gsj_join_stats none{};
+    uint64_t n_over = 0;
+    (void)refine_stages_finish(c, P, R, pa, pb, np, rp, out, stats ? *stats : none, n_over);
+    return n_over;
+  }
   const bool rel = rp.want_relate != 0;
   const LaunchShape& sh = c.shape(np);
   const PairClasses pc = partition_pairs(c, P, R, pa, pb, np, sh.mcap, sh.mixed != 0, sh.tcap, sh.size_sort);
@@ -1009,7 +1292,7 @@ uint64_t refine_pairs(Context& c, const DPolys& P, const DPolys& R, const uint32
   if (side_ovf) {   // one wave per pair over a grid sized for the largest queue the launch can have, idle blocks leave at once
     const uint32_t g = std::min<uint32_t>((uint32_t)std::min<uint64_t>(np, 1u << 30), cu * 8);
     hipLaunchKernelGGL((k_refine_overflow<64, true>), dim3(g), dim3(64), list_bytes(OVF_SIDE_CAP, rel), sl, P, R, pa, pb, ovf, 0u, rp, out,
-                       (int)OVF_SIDE_CAP, nullptr, ctl, ovf_main, ctl_main);
+                       (int)OVF_SIDE_CAP, nullptr, ctl, ovf_main, ctl_main, nullptr);
     GSJ_LAUNCHED();
     GSJ_HIP(hipEventRecord(c.ev[16], sl));
   }
@@ -1077,46 +1360,7 @@ uint64_t refine_pairs(Context& c, const DPolys& P, const DPolys& R, const uint32
     stats->n_tiny_edge += h->counts[8 + CL_TINY]; stats->n_small_edge += h->counts[8 + CL_SMALL]; stats->n_medium_edge += h->counts[8 + CL_MEDIUM];
     stats->launches++;
   }
-  if (nover && sh.ovf_lds && need <= OVF_LDS_CAP) {   // lists in LDS: no slab
-    const size_t lds = list_bytes((int)need, rel);
-    GSJ_HIP(hipEventRecord(c.ev[3], st));
-    // pairs too few to fill the GPU (a windowed request's few largest): eight waves each, so that the edge
-    // contributions of both lists (up to 2 x 448 edges) take one or two rounds
-    const bool few = nover <= (uint64_t)c.cu_count;
-    const uint32_t blocks = (uint32_t)std::min<uint64_t>(nover, (uint64_t)c.cu_count * (few ? 1 : 8));
-    if (few)
-      hipLaunchKernelGGL((k_refine_overflow<512, true>), dim3(blocks), dim3(512), lds, st, P, R, pa, pb, ovf_main, nover, rp, out, (int)need, nullptr, nullptr, nullptr, nullptr);
-    else
-      hipLaunchKernelGGL((k_refine_overflow<64, true>), dim3(blocks), dim3(64), lds, st, P, R, pa, pb, ovf_main, nover, rp, out, (int)need, nullptr, nullptr, nullptr, nullptr);
-    GSJ_LAUNCHED();
-    GSJ_HIP(hipEventRecord(c.ev[4], st));
-    if (stats) {
-      GSJ_HIP(hipEventSynchronize(c.ev[4]));
-      float ms_o = 0;
-      GSJ_HIP(hipEventElapsedTime(&ms_o, c.ev[3], c.ev[4]));
-      stats->k_over_ms += ms_o;
-    }
-  } else if (nover) {
-    const size_t per = list_bytes((int)need, rel);
-    // slabs of at most 1 GiB (half of what is left when the scratch is a fixed arena: compaction still needs room)
-    const uint64_t budget = c.dev_arena ? std::min<uint64_t>(1ull << 30, c.dev_arena->left() / 2) : (1ull << 30);
-    GSJ_REQUIRE(!c.dev_arena || per <= budget, GSJ_E_LIMIT, "overflow pair lists exceed the no-allocation scratch left for them");
-    const uint64_t blocks = std::max<uint64_t>(1, std::min<uint64_t>(nover, budget / std::max<size_t>(per, 1)));   // one slab per block
-    unsigned char* slab = c.s_heavy_edges.as<unsigned char>(per * blocks + 64);
-    GSJ_HIP(hipEventRecord(c.ev[3], st));
-    if (nover <= 2ull * c.cu_count)   // a few pairs: four waves each (2.4M relate: one wave each, 2.5 vs 4.5 ms)
-      hipLaunchKernelGGL((k_refine_overflow<256, false>), dim3((uint32_t)blocks), dim3(256), 0, st, P, R, pa, pb, ovf_main, nover, rp, out, (int)need, slab, nullptr, nullptr, nullptr);
-    else
-      hipLaunchKernelGGL((k_refine_overflow<64, false>), dim3((uint32_t)blocks), dim3(64), 0, st, P, R, pa, pb, ovf_main, nover, rp, out, (int)need, slab, nullptr, nullptr, nullptr);
-    GSJ_LAUNCHED();
-    GSJ_HIP(hipEventRecord(c.ev[4], st));
-    if (stats) {
-      GSJ_HIP(hipEventSynchronize(c.ev[4]));
-      float ms_o = 0;
-      GSJ_HIP(hipEventElapsedTime(&ms_o, c.ev[3], c.ev[4]));
-      stats->k_over_ms += ms_o;
-    }
-  }
+  if (nover) overflow_launch(c, P, R, pa, pb, ovf_main, nover, need, rp, out, sh.ovf_lds != 0, stats);
   return n_over;
 }
 
@@ -1127,11 +1371,7 @@ constexpr int CLASS_BIT = 5;   // partition key: class above, size bucket below
 // tcap is 0), small (both within VCAP), medium (both within mcap; none when mcap is 0), all three with rings within
 // RCAP; mixed (when enabled: none of those, one polygon within VCAP stored vertices); large — and the pair's stored vertex
 // count in buckets (saturated at 31) below, so that the groups of a wave get pairs of similar work
-__global__ void k_class_keys(const DPolys P, const DPolys R, const uint32_t* __restrict__ pa, const uint32_t* __restrict__ pb, uint64_t np,
-                             uint32_t mcap, int mixed, uint32_t tcap, uint32_t size_sort, uint64_t* __restrict__ key, uint32_t* __restrict__ val) {
-  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= np) return;
-  const uint32_t ia = P.ginfo[pa[i]], ib = R.ginfo[pb[i]];
+__device__ __forceinline__ uint32_t class_key(uint32_t ia, uint32_t ib, uint32_t mcap, int mixed, uint32_t tcap, uint32_t size_sort) {
   const uint32_t va = ia & 0xFFFFu, vb = ib & 0xFFFFu;
   const bool rings = (ia >> 16) <= RCAP && (ib >> 16) <= RCAP;
   const uint32_t cls = (rings && va <= tcap && vb <= tcap) ? CL_TINY
@@ -1142,8 +1382,93 @@ __global__ void k_class_keys(const DPolys P, const DPolys R, const uint32_t* __r
   // class spans hundreds of vertices, so its buckets are 8 vertices wide (1 for tiny, 2 for small and mixed, 4 for
   // medium); size_sort > 1 widens them by powers of two (fewer, longer runs of candidate order)
   const uint32_t shift = (cls == CL_LARGE ? 3u : (cls == CL_MEDIUM ? 2u : (cls == CL_TINY ? 0u : 1u))) + size_sort - 1;
-  key[i] = (uint64_t)((cls << CLASS_BIT) | (size_sort ? min(31u, (va + vb) >> shift) : 0u));
+  return (cls << CLASS_BIT) | (size_sort ? min(31u, (va + vb) >> shift) : 0u);
+}
+__global__ void k_class_keys(const DPolys P, const DPolys R, const uint32_t* __restrict__ pa, const uint32_t* __restrict__ pb, uint64_t np,
+                             uint32_t mcap, int mixed, uint32_t tcap, uint32_t size_sort, uint64_t* __restrict__ key, uint32_t* __restrict__ val) {
+  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= np) return;
+  key[i] = class_key(P.ginfo[pa[i]], R.ginfo[pb[i]], mcap, mixed, tcap, size_sort);
   val[i] = (uint32_t)i;
+}
+
+// k_class_keys, the sort and the class sizes in one block, for at most PART_MAX pairs: wave w takes the w-th run of the
+// candidates and counts its keys (256 of them) in LDS; once the counts are scanned over (key, wave), every candidate
+// knows its place: the order of the sort but for candidates that the same wave counted in the same instruction. Two
+// counters per wave and key, by the lane's parity, halve the same-address chains (a few keys hold most pairs).
+// 10.6k pairs: one launch of 14 us (24 us as a stable sort with ranks from ballots) instead of six launches.
+constexpr int PART_T = 1024, PART_MAX = 16384, PART_ITEMS = PART_MAX / PART_T;
+__global__ void __launch_bounds__(PART_T) k_partition_small(const DPolys P, const DPolys R, const uint32_t* __restrict__ pa, const uint32_t* __restrict__ pb,
+                                                            uint32_t np, uint32_t mcap, int mixed, uint32_t tcap, uint32_t size_sort,
+                                                            uint32_t* __restrict__ list, uint32_t* __restrict__ counts, OverflowCtl* ctl) {
+  constexpr int NC = PART_T / 64 * 2, PARTS = PART_T / 256, CPP = NC / PARTS;   // counter columns; a thread scans CPP of a key's
+  __shared__ uint32_t hist[NC][256];
+  __shared__ uint32_t psum[PARTS][256];
+  __shared__ uint32_t kfirst[256];
+  __shared__ uint32_t wtot[4];
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6, col = 2 * w + (lane & 1);
+  const uint32_t per = (np + PART_T - 1) / PART_T;             // rounds of 64 candidates per wave
+  const uint32_t base = (uint32_t)w * per * 64 + (uint32_t)lane;
+  uint32_t key[PART_ITEMS], rank[PART_ITEMS];
+  {
+    uint32_t a[PART_ITEMS], b[PART_ITEMS];
+#pragma unroll
+    for (int j = 0; j < PART_ITEMS; j++) {
+      const uint32_t i = base + j * 64;
+      const bool v = j < (int)per && i < np;
+      a[j] = v ? pa[i] : 0u;
+      b[j] = v ? pb[i] : 0u;
+    }
+#pragma unroll
+    for (int j = 0; j < PART_ITEMS; j++) {   // (every layer with a candidate has a geometry 0)
+      a[j] = j < (int)per ? P.ginfo[a[j]] : 0u;
+      b[j] = j < (int)per ? R.ginfo[b[j]] : 0u;
+    }
+#pragma unroll
+    for (int j = 0; j < PART_ITEMS; j++) key[j] = class_key(a[j], b[j], mcap, mixed, tcap, size_sort);
+  }
+  for (int k = t; k < NC * 256; k += PART_T) (&hist[0][0])[k] = 0;
+  if (t < 5) ctl[t] = OverflowCtl{0, 0, 0, 0};
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < PART_ITEMS; j++)
+    if (j < (int)per && base + j * 64 < np) rank[j] = atomicAdd(&hist[col][key[j]], 1u);
+  __syncthreads();
+  const int k = t & 255, part = t >> 8;
+  uint32_t own = 0;
+#pragma unroll
+  for (int c = 0; c < CPP; c++) own += hist[part * CPP + c][k];
+  psum[part][k] = own;
+  __syncthreads();
+  if (t < 256) {   // exclusive scan over the keys
+    uint32_t sum = 0;
+#pragma unroll
+    for (int q = 0; q < PARTS; q++) sum += psum[q][t];
+    uint32_t inc = sum;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const uint32_t v = __shfl_up(inc, o, 64);
+      if (lane >= o) inc += v;
+    }
+    if (lane == 63) wtot[w] = inc;
+    kfirst[t] = inc - sum;   // within the wave's 64 keys
+  }
+  __syncthreads();
+  {
+    uint32_t at = kfirst[k];
+    for (int q = 0; q < (k >> 6); q++) at += wtot[q];
+    for (int q = 0; q < part; q++) at += psum[q][k];
+#pragma unroll
+    for (int c = 0; c < CPP; c++) { const uint32_t v = hist[part * CPP + c][k]; hist[part * CPP + c][k] = at; at += v; }
+  }
+  __syncthreads();
+  if (t < 16) {   // class sizes [0, 5), the edge queues' counts [8, 11) and, for the staged launches, their starts [11, 14)
+    auto first = [&](int cl) { return cl >= CL_COUNT ? np : hist[0][cl << CLASS_BIT]; };
+    counts[t] = t < CL_COUNT ? first(t + 1) - first(t) : (t >= 11 && t < 14) ? first(t - 11) : 0u;
+  }
+#pragma unroll
+  for (int j = 0; j < PART_ITEMS; j++)
+    if (j < (int)per && base + j * 64 < np) list[hist[col][key[j]] + rank[j]] = base + j * 64;
 }
 
 // class sizes from the sorted keys: first index of every class after the first by binary search
@@ -1161,6 +1486,7 @@ __global__ void k_class_counts(const uint64_t* __restrict__ key, uint64_t np, ui
     first[c] = lo;
   }
   for (int c = 0; c < CL_COUNT; c++) counts[c] = (uint32_t)(first[c + 1] - first[c]);
+  for (int c = CL_TINY; c <= CL_MEDIUM; c++) counts[11 + c] = (uint32_t)first[c];   // the staged launches' queue starts
 }
 
 // the overflow queue's control at ctl, the host-read queue's (ovf_lds 2) right after it, the promotion queue's 64 bytes on
@@ -1175,11 +1501,19 @@ __global__ void k_ctl_reset(OverflowCtl* ctl, uint32_t* counts) {
 PairClasses partition_pairs(Context& c, const DPolys& P, const DPolys& R, const uint32_t* pa, const uint32_t* pb, uint64_t np, uint32_t mcap,
                             bool mixed, uint32_t tcap, uint32_t size_sort) {
   hipStream_t st = c.stream;
-  char* misc = c.s_misc.as<char>(256);   // [0, 32) belongs to the scan / sort primitives
+  char* misc = c.s_misc.as<char>(512);   // [0, 32) belongs to the sort primitives
   PairClasses pc;
   pc.counts = reinterpret_cast<uint32_t*>(misc + 64);
   pc.ctl = reinterpret_cast<OverflowCtl*>(misc + 128);
+  pc.start = reinterpret_cast<uint64_t*>(misc + 256);
   pc.list = nullptr;
+  if (np && np <= (uint64_t)PART_MAX) {
+    pc.list = c.s_vals.as<uint32_t>(np + 16);
+    hipLaunchKernelGGL(k_partition_small, dim3(1), dim3(PART_T), 0, st, P, R, pa, pb, (uint32_t)np, mcap, mixed ? 1 : 0, tcap, size_sort, pc.list,
+                       pc.counts, pc.ctl);
+    GSJ_LAUNCHED();
+    return pc;
+  }
   hipLaunchKernelGGL(k_ctl_reset, dim3(1), dim3(1), 0, st, pc.ctl, pc.counts);
   GSJ_LAUNCHED();
   if (np == 0) return pc;

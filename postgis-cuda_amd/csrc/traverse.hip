@@ -7,7 +7,7 @@
 // One walk per probe in the common case: it counts the probe's candidates and keeps the first SLOT_K of them in the
 // probe's slots; after the scan, a gather writes them at their offsets (SoA pair buffers), and only the probes with
 // more candidates than slots walk again, writing at their offsets.
-#include "engine.h"
+#include "scan.h"
 
 namespace gsj {
 
@@ -277,17 +277,22 @@ void walk_batches(Context& c, const Probes& pr, const DBvh& t, bool upper, const
     WallTimer tt;
     uint32_t* counts = c.s_counts.as<uint32_t>(nq + 16);
     uint32_t* slots = c.s_slots.as<uint32_t>((uint64_t)nq * SLOT_K + 16);
+    const bool fresh = c.s_slots_ctl.cap == 0 || c.dev_arena;   // the counter starts at 0, and every scan leaves it at 0
     uint32_t* nover = c.s_slots_ctl.as<uint32_t>(16);
-    uint32_t* hover = c.h_slots_ctl.as<uint32_t>(4);
-    hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, stream, nover, (uint64_t)1);
-    GSJ_LAUNCHED();
+    if (fresh) {
+      hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, stream, nover, (uint64_t)1);
+      GSJ_LAUNCHED();
+    }
     GSJ_HIP(hipEventRecord(c.ev[12], stream));
     traverse_count(c, qbb, qidx, q0, nq, t, upper, counts, slots, nover, box_by_pos);
     GSJ_HIP(hipEventRecord(c.ev[13], stream));
-    GSJ_HIP(hipMemcpyAsync(hover, nover, 4, hipMemcpyDeviceToHost, stream));
     uint64_t* offs = c.s_qoffs.as<uint64_t>((uint64_t)nq + 16);   // probe offsets (s_offs belongs to compaction)
-    const uint64_t total = scan_u32_to_u64(c, counts, offs, nq);   // synchronises: *hover is there too
-    const bool any_over = *hover != 0;
+    const HostWords w = host_words(c, 8, 2);   // the candidates, the probes with more of them than slots
+    scan_loaded<uint64_t>(c, LoadArray<uint32_t>{counts}, offs, nq, ScanTotal{w.dev, nover});
+    w.fetch(c);
+    GSJ_HIP(hipStreamSynchronize(stream));
+    const uint64_t total = w.host[0];
+    const bool any_over = w.host[1] != 0;
     {
       float ms = 0;
       GSJ_HIP(hipEventElapsedTime(&ms, c.ev[12], c.ev[13]));

@@ -94,6 +94,7 @@ struct Layer {
   DPoints pts;
   DBvh bvh;
   bool has_bvh = false;
+  uint32_t max_pieces = 1;          // most pieces of one parent
   std::vector<uint32_t> h_parent;   // host copy: keeps a parent's pieces in one probe batch
   std::vector<float4> h_tiles;      // host copy of the probe tile boxes (scratch estimates of windowed requests)
   double build_ms = 0;              // device time of the last BVH build (HIP events around its kernels)

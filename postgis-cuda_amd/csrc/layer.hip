@@ -165,6 +165,10 @@ void layer_upload_polys(Layer& L, const uint64_t* gro, const uint64_t* rvo, cons
   if (parent && n) {
     for (uint64_t g = 1; g < n; g++) GSJ_REQUIRE(parent[g] >= parent[g - 1], GSJ_E_ARG, "parent[] must be non-decreasing");
     nparent = parent[n - 1] + 1;
+    for (uint64_t g = 0, first = 0; g < n; g++) {
+      if (parent[g] != parent[first]) first = g;
+      L.max_pieces = std::max(L.max_pieces, (uint32_t)(g - first + 1));
+    }
     L.h_parent.assign(parent, parent + n);
   }
   L.nparent = nparent;

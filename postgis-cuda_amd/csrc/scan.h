@@ -43,17 +43,21 @@ __device__ __forceinline__ uint64_t block_excl_scan(uint64_t v, uint64_t* total)
 // loader of a plain count or flag array
 template <class T>
 struct LoadArray {
+  static constexpr bool PACKED = false;
   const T* p;
   __device__ __forceinline__ uint64_t operator()(uint64_t i) const { return (uint64_t)p[i]; }
 };
 
 // Where the total goes: words[0] (device memory, or pinned host memory that the kernel writes directly), and with `over`
-// a counter that the caller's earlier kernel incremented: its value goes to words[1] and it starts at 0 again.
+// a counter that the caller's earlier kernel incremented: its value goes to words[1] and it starts at 0 again; dev (or
+// null) takes the total for a later kernel.
 struct ScanTotal {
   uint64_t* words = nullptr;
   uint32_t* over = nullptr;
+  uint64_t* dev = nullptr;
   __device__ __forceinline__ void put(uint64_t total) const {
     if (words) words[0] = total;
+    if (dev) *dev = total;
     if (over) { words[1] = *over; *over = 0; }
   }
 };
@@ -110,9 +114,12 @@ __global__ void __launch_bounds__(SCAN_T) k_tile_scan(const Ld in, TO* out, uint
 // one block: exclusive scan of n <= SS_MAX elements; thread t scans elements [per t, per (t + 1)). They are read and
 // written in order, 64 lanes side by side, and pass through LDS between (each thread reading its own run from memory
 // touched a line per element: 10.6k probe counts 8.3 -> 5.9 us). An odd `per` spreads the threads' runs over the banks. A total of
-// 2^32 or more (prefixes that do not fit the LDS words) is written from the registers. Every element is read before
+// 2^32 or more (prefixes that do not fit the LDS words) is written from the registers. A PACKED loader counts two kinds in
+// the halves of a word, at most one each: they pass through LDS as 16-bit halves, and so do their prefixes. Every element is read before
 // the first is written, so in and out may be the same array.
 constexpr int SS_T = 1024, SS_ITEMS = 17, SS_MAX = 16384;
+template <bool PACKED> __device__ __forceinline__ uint32_t ss_pack(uint64_t v) { return PACKED ? (uint32_t)v | (uint32_t)(v >> 16) : (uint32_t)v; }
+template <bool PACKED> __device__ __forceinline__ uint64_t ss_unpack(uint32_t v) { return PACKED ? (uint64_t)(v & 0xFFFFu) | (uint64_t)(v >> 16) << 32 : v; }
 template <class Ld, class TO>
 __global__ void __launch_bounds__(SS_T) k_scan_small(const Ld in, TO* out, uint64_t n64, ScanTotal total) {
   __shared__ uint64_t wsum[SS_T / 64];
@@ -121,7 +128,7 @@ __global__ void __launch_bounds__(SS_T) k_scan_small(const Ld in, TO* out, uint6
   const uint32_t n = (uint32_t)n64, per = (n + SS_T - 1) / SS_T | 1u;
   uint32_t v[SS_ITEMS];
 #pragma unroll
-  for (int k = 0; k < SS_MAX / SS_T; k++) v[k] = t + (uint32_t)k * SS_T < n ? (uint32_t)in(t + (uint32_t)k * SS_T) : 0u;   // all loads in flight
+  for (int k = 0; k < SS_MAX / SS_T; k++) v[k] = t + (uint32_t)k * SS_T < n ? ss_pack<Ld::PACKED>(in(t + (uint32_t)k * SS_T)) : 0u;   // all loads in flight
 #pragma unroll
   for (int k = 0; k < SS_MAX / SS_T; k++)
     if (t + (uint32_t)k * SS_T < n) buf[t + k * SS_T] = v[k];
@@ -131,7 +138,7 @@ __global__ void __launch_bounds__(SS_T) k_scan_small(const Ld in, TO* out, uint6
 #pragma unroll
   for (int k = 0; k < SS_ITEMS; k++) {
     v[k] = k < (int)per && base + k < n ? buf[base + k] : 0u;
-    s += v[k];
+    s += ss_unpack<Ld::PACKED>(v[k]);
   }
   const uint64_t inc = wave_incl_scan(s);
   if (lane == 63) wsum[w] = inc;
@@ -142,21 +149,21 @@ __global__ void __launch_bounds__(SS_T) k_scan_small(const Ld in, TO* out, uint6
     if (k < w) ex += wsum[k];
     tot += wsum[k];
   }
-  if (tot >> 32) {
+  if (!Ld::PACKED && (tot >> 32)) {
 #pragma unroll
     for (int k = 0; k < SS_ITEMS; k++) {
       if (k < (int)per && base + k < n) out[base + k] = (TO)ex;
       ex += v[k];
     }
   } else {
-    uint32_t e = (uint32_t)ex;
+    uint32_t e = ss_pack<Ld::PACKED>(ex);   // (halves of at most SS_MAX = 2^14)
 #pragma unroll
     for (int k = 0; k < SS_ITEMS; k++) {
       if (k < (int)per && base + k < n) buf[base + k] = e;
       e += v[k];
     }
     __syncthreads();
-    for (uint32_t i = t; i < n; i += SS_T) out[i] = (TO)buf[i];
+    for (uint32_t i = t; i < n; i += SS_T) out[i] = (TO)ss_unpack<Ld::PACKED>(buf[i]);
   }
   if (t == 0) total.put(tot);
 }

@@ -43,22 +43,81 @@ struct ListSrc {   // compacted list (large / overflow classes)
   __device__ __forceinline__ bool get(int k, Ed& e) const { e = L[k]; return true; }
 };
 
+// whether edge e crosses the segment c->x
+__device__ __forceinline__ bool edge_crosses_cx(const Ed& e, double cx, double cy, double x, double y) {
+  const bool sc = left_of(e.x0, e.y0, e.x1, e.y1, cx, cy), sx = left_of(e.x0, e.y0, e.x1, e.y1, x, y);
+  if (sc == sx) return false;
+  const bool su = orient(cx, cy, x, y, e.x0, e.y0) > 0, sv = orient(cx, cy, x, y, e.x1, e.y1) > 0;
+  return su != sv;
+}
+// the list entries [base, base + 64) whose boxes meet the box [x0, x1] x [y0, y1], a bit each: the loops over "the other
+// polygon's edges near this one" take the box tests of a whole run first and then the expensive test for the marked
+// entries alone, in order: the lanes of a wave make those iterations together, about as many as the most crowded lane
+// has neighbours, instead of one per entry whenever any lane has one
+template <class Src>
+__device__ __forceinline__ uint64_t box_bits(const Src& L, int base, int n, double x0, double x1, double y0, double y1) {
+  const int m = min(64, n - base);
+  uint64_t bits = 0;
+  for (int j = 0; j < m; j++) {
+    Ed e;
+    if (!L.get(base + j, e)) continue;
+    if (!(fmax(e.x0, e.x1) < x0 || fmin(e.x0, e.x1) > x1 || fmax(e.y0, e.y1) < y0 || fmin(e.y0, e.y1) > y1)) bits |= 1ull << j;
+  }
+  return bits;
+}
+
 // inside(x) = inside(c) xor parity of segment c->x across the local edges (engine/engine.cuh:400-412)
 template <class Src>
 __device__ bool inside_from_c(const Src& L, double cx, double cy, bool in_c, double x, double y) {
   bool in = in_c;
   const double sx0 = fmin(cx, x), sx1 = fmax(cx, x), sy0 = fmin(cy, y), sy1 = fmax(cy, y);
   const int n = L.size();
-  for (int k = 0; k < n; k++) {
+  for (int base = 0; base < n; base += 64) {
+    uint64_t bits = box_bits(L, base, n, sx0, sx1, sy0, sy1);
+    while (bits != 0) {
+      const int k = base + __builtin_ctzll(bits);
+      bits &= bits - 1;
+      Ed e;
+      L.get(k, e);
+      if (edge_crosses_cx(e, cx, cy, x, y)) in = !in;
+    }
+  }
+  return in;
+}
+// the same for one point on a G-lane group (group-uniform arguments), the lanes sharing the edges: the same parity
+template <int G, class Src>
+__device__ __forceinline__ bool inside_from_c_g(const Src& L, double cx, double cy, bool in_c, double x, double y, int gl) {
+  const double sx0 = fmin(cx, x), sx1 = fmax(cx, x), sy0 = fmin(cy, y), sy1 = fmax(cy, y);
+  const int n = L.size();
+  bool par = false;
+  for (int k = gl; k < n; k += G) {
     Ed e;
     if (!L.get(k, e)) continue;
     if (fmax(e.x0, e.x1) < sx0 || fmin(e.x0, e.x1) > sx1 || fmax(e.y0, e.y1) < sy0 || fmin(e.y0, e.y1) > sy1) continue;
-    const bool sc = left_of(e.x0, e.y0, e.x1, e.y1, cx, cy), sx = left_of(e.x0, e.y0, e.x1, e.y1, x, y);
-    if (sc == sx) continue;
-    const bool su = orient(cx, cy, x, y, e.x0, e.y0) > 0, sv = orient(cx, cy, x, y, e.x1, e.y1) > 0;
-    if (su != sv) in = !in;
+    if (edge_crosses_cx(e, cx, cy, x, y)) par = !par;
   }
-  return in;
+  return in_c != ((__popcll(gballot<G>(par)) & 1) != 0);
+}
+
+// boundary contact of edge ea with the entries [j0, j1) of list L: `any` contact, or a `real` one (both edges real), which
+// ends the search (marked entries first, as above: overflow pass of 4.3M pairs 2.03 -> 1.71 ms, large class of 397k parcels'
+// clusters 550 -> 450 us)
+template <class Src>
+__device__ __forceinline__ void edge_contacts(const Ed& ea, const Src& L, int j0, int j1, bool& any, bool& real) {
+  const double x0 = fmin(ea.x0, ea.x1), x1 = fmax(ea.x0, ea.x1), y0 = fmin(ea.y0, ea.y1), y1 = fmax(ea.y0, ea.y1);
+  for (int base = j0; base < j1 && !real; base += 64) {
+    uint64_t bits = box_bits(L, base, j1, x0, x1, y0, y1);
+    while (bits != 0 && !real) {
+      const int j = base + __builtin_ctzll(bits);
+      bits &= bits - 1;
+      Ed eb;
+      L.get(j, eb);
+      if (seg_isect(ea.x0, ea.y0, ea.x1, ea.y1, eb.x0, eb.y0, eb.x1, eb.y1)) {
+        any = true;
+        if (!(ea.syn | eb.syn)) real = true;
+      }
+    }
+  }
 }
 
 // ------------------------------------------------------------------------------------------- edge chunks

@@ -250,6 +250,7 @@ uint64_t* wseg(Context& c, int region);
 struct RefineParams {   // engine/engine.cuh:517-518
   double tol_rel = 1e-12, eps_par = 1e-7, tol_abs = 1e-11;
   int want_area = 1, want_relate = 0, snap_half_ulp = 0;
+  const uint8_t* done = nullptr;   // [np] candidates whose outputs the caller has written itself (byte set), or none
 };
 struct RefineOut {
   uint8_t* isect;   // [np] 0 / 1 real contact or containment / 2 area-only piece overlap
@@ -281,6 +282,8 @@ struct JoinHooks {
   // candidate filter before refinement (JoinOpts::prefilter, engine/engine.cuh:812, 935): compacts the sub-batch's
   // pairs in place on the device and returns how many are kept
   std::function<uint64_t(uint32_t* pa, uint32_t* pb, uint64_t np)> prefilter;
+  // decides candidates before the refinement: enqueues the writing of their outputs and returns RefineParams::done
+  std::function<const uint8_t*(const uint32_t* pa, const uint32_t* pb, uint64_t np, const RefineOut& out)> decide;
   // the probes about to be walked (for_each_candidate_batch's on_members)
   MembersFn on_members;
 };

@@ -394,6 +394,7 @@ void join_run(Context& c, const Layer& PL, const Layer& RL, const gsj_join_opts&
     ro.area = rp.want_area ? c.s_area.as<double>(np + 16) : nullptr;
     ro.ev = rp.want_relate ? c.s_ev.as<double4>(np + 16) : nullptr;
     ro.evb = rp.want_relate ? c.s_evb.as<uint32_t>(np + 16) : nullptr;
+    rp.done = hooks && hooks->decide ? hooks->decide(pa, pb, np, ro) : nullptr;
     // no host waits between refinement, compaction and the row copy beyond the ones that read sizes back: the
     // stream orders the work (refine_ms and compact_ms are host times up to those reads)
     const bool folds = !o.no_agg && (PL.poly.pfirst || RL.poly.pfirst);

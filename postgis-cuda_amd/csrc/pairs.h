@@ -304,8 +304,7 @@ enum PairClass : int { CL_TINY = 0, CL_SMALL = 1, CL_MEDIUM = 2, CL_MIXED = 3, C
 // within mcap / RCAP; none when mcap is 0), counts[3] mixed pairs (with `mixed`: one polygon within VCAP vertices),
 // then the counts[4] others; within a class by mean vertex count, then candidate order; ctl cleared for the overflow
 // queue. counts[8 ..) is left zeroed for the callers' queues.
-// Uses the context's s_keys, s_keys2, s_vals, s_vals2, s_tmp2 and s_misc scratch (the list lives in one of the
-// s_vals buffers until their next use).
+// Uses the context's s_keys, s_vals, s_tmp2 and s_misc scratch (the list lives in s_vals until its next use).
 struct PairClasses {
   uint32_t* list;
   uint32_t* counts;
@@ -313,9 +312,10 @@ struct PairClasses {
   uint64_t* start;   // words for launches' start times
 };
 // size_sort: within a class, pairs of similar size side by side, in buckets 2^(size_sort-1) times the class's base
-// width (0: candidate order, a probe's pairs together)
+// width (0: candidate order, a probe's pairs together); done (or null): the candidates whose byte is set are in no class
+// (they come last in the list)
 PairClasses partition_pairs(Context& c, const DPolys& P, const DPolys& R, const uint32_t* pa, const uint32_t* pb, uint64_t np, uint32_t mcap,
-                            bool mixed, uint32_t tcap, uint32_t size_sort = 1);
+                            bool mixed, uint32_t tcap, uint32_t size_sort = 1, const uint8_t* done = nullptr);
 // first list position of class cl
 __host__ __device__ __forceinline__ uint32_t class_first(const uint32_t* counts, int cl) {
   uint32_t f = 0;

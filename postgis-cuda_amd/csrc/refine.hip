@@ -21,6 +21,7 @@
 //    restatement, so a pair gives the same bits alone or batched with any other request.
 //  * FP64 on the vector ALUs only; nothing here is a dense contraction, so MFMA is not used.
 #include "pairs.h"
+#include "scan.h"
 #include <type_traits>
 
 namespace gsj {
@@ -1135,7 +1136,7 @@ void refine_stages(Context& c, const DPolys& P, const DPolys& R, const uint32_t*
   hipStream_t st = c.stream;
   const bool rel = rp.want_relate != 0;
   const LaunchShape& sh = c.shape(np);
-  const PairClasses pc = partition_pairs(c, P, R, pa, pb, np, sh.mcap, sh.mixed != 0, sh.tcap, sh.size_sort);
+  const PairClasses pc = partition_pairs(c, P, R, pa, pb, np, sh.mcap, sh.mixed != 0, sh.tcap, sh.size_sort, rp.done);
   StageArgs A{};
   A.P = P; A.R = R; A.pa = pa; A.pb = pb; A.list = pc.list; A.counts = pc.counts; A.rp = rp; A.out = out;
   A.ovf = c.s_heavy.as<uint32_t>(3 * np + 192);
@@ -1204,7 +1205,7 @@ uint64_t refine_pairs(Context& c, const DPolys& P, const DPolys& R, const uint32
   }
   const bool rel = rp.want_relate != 0;
   const LaunchShape& sh = c.shape(np);
-  const PairClasses pc = partition_pairs(c, P, R, pa, pb, np, sh.mcap, sh.mixed != 0, sh.tcap, sh.size_sort);
+  const PairClasses pc = partition_pairs(c, P, R, pa, pb, np, sh.mcap, sh.mixed != 0, sh.tcap, sh.size_sort, rp.done);
   uint32_t* list = pc.list;
   uint32_t* counts = pc.counts;
   OverflowCtl* ctl = pc.ctl;
@@ -1338,6 +1339,7 @@ constexpr int CLASS_BIT = 5;   // partition key: class above, size bucket below
 // tcap is 0), small (both within VCAP), medium (both within mcap; none when mcap is 0), all three with rings within
 // RCAP; mixed (when enabled: none of those, one polygon within VCAP stored vertices); large — and the pair's stored vertex
 // count in buckets (saturated at 31) below, so that the groups of a wave get pairs of similar work
+constexpr uint32_t KEY_DONE = (uint32_t)CL_COUNT << CLASS_BIT;   // decided already: in no class
 __device__ __forceinline__ uint32_t class_key(uint32_t ia, uint32_t ib, uint32_t mcap, int mixed, uint32_t tcap, uint32_t size_sort) {
   const uint32_t va = ia & 0xFFFFu, vb = ib & 0xFFFFu;
   const bool rings = (ia >> 16) <= RCAP && (ib >> 16) <= RCAP;
@@ -1351,23 +1353,16 @@ __device__ __forceinline__ uint32_t class_key(uint32_t ia, uint32_t ib, uint32_t
   const uint32_t shift = (cls == CL_LARGE ? 3u : (cls == CL_MEDIUM ? 2u : (cls == CL_TINY ? 0u : 1u))) + size_sort - 1;
   return (cls << CLASS_BIT) | (size_sort ? min(31u, (va + vb) >> shift) : 0u);
 }
-__global__ void k_class_keys(const DPolys P, const DPolys R, const uint32_t* __restrict__ pa, const uint32_t* __restrict__ pb, uint64_t np,
-                             uint32_t mcap, int mixed, uint32_t tcap, uint32_t size_sort, uint64_t* __restrict__ key, uint32_t* __restrict__ val) {
-  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= np) return;
-  key[i] = class_key(P.ginfo[pa[i]], R.ginfo[pb[i]], mcap, mixed, tcap, size_sort);
-  val[i] = (uint32_t)i;
-}
-
-// k_class_keys, the sort and the class sizes in one block, for at most PART_MAX pairs: wave w takes the w-th run of the
+// The keys, their sort and the class sizes in one block, for at most PART_MAX pairs: wave w takes the w-th run of the
 // candidates and counts its keys (256 of them) in LDS; once the counts are scanned over (key, wave), every candidate
 // knows its place: the order of the sort but for candidates that the same wave counted in the same instruction. Two
 // counters per wave and key, by the lane's parity, halve the same-address chains (a few keys hold most pairs).
 // 10.6k pairs: one launch of 14 us (24 us as a stable sort with ranks from ballots) instead of six launches.
 constexpr int PART_T = 1024, PART_MAX = 16384, PART_ITEMS = PART_MAX / PART_T;
 __global__ void __launch_bounds__(PART_T) k_partition_small(const DPolys P, const DPolys R, const uint32_t* __restrict__ pa, const uint32_t* __restrict__ pb,
-                                                            uint32_t np, uint32_t mcap, int mixed, uint32_t tcap, uint32_t size_sort,
-                                                            uint32_t* __restrict__ list, uint32_t* __restrict__ counts, OverflowCtl* ctl) {
+                                                            const uint8_t* __restrict__ done, uint32_t np, uint32_t mcap, int mixed, uint32_t tcap,
+                                                            uint32_t size_sort, uint32_t* __restrict__ list, uint32_t* __restrict__ counts,
+                                                            OverflowCtl* ctl) {
   constexpr int NC = PART_T / 64 * 2, PARTS = PART_T / 256, CPP = NC / PARTS;   // counter columns; a thread scans CPP of a key's
   __shared__ uint32_t hist[NC][256];
   __shared__ uint32_t psum[PARTS][256];
@@ -1392,7 +1387,10 @@ __global__ void __launch_bounds__(PART_T) k_partition_small(const DPolys P, cons
       b[j] = j < (int)per ? R.ginfo[b[j]] : 0u;
     }
 #pragma unroll
-    for (int j = 0; j < PART_ITEMS; j++) key[j] = class_key(a[j], b[j], mcap, mixed, tcap, size_sort);
+    for (int j = 0; j < PART_ITEMS; j++) {
+      key[j] = class_key(a[j], b[j], mcap, mixed, tcap, size_sort);
+      if (done && j < (int)per && base + j * 64 < np && done[base + j * 64]) key[j] = KEY_DONE;
+    }
   }
   for (int k = t; k < NC * 256; k += PART_T) (&hist[0][0])[k] = 0;
   if (t < 5) ctl[t] = OverflowCtl{0, 0, 0, 0};
@@ -1430,7 +1428,7 @@ __global__ void __launch_bounds__(PART_T) k_partition_small(const DPolys P, cons
   }
   __syncthreads();
   if (t < 16) {   // class sizes [0, 5), the edge queues' counts [8, 11) and, for the staged launches, their starts [11, 14)
-    auto first = [&](int cl) { return cl >= CL_COUNT ? np : hist[0][cl << CLASS_BIT]; };
+    auto first = [&](int cl) { return hist[0][cl << CLASS_BIT]; };
     counts[t] = t < CL_COUNT ? first(t + 1) - first(t) : (t >= 11 && t < 14) ? first(t - 11) : 0u;
   }
 #pragma unroll
@@ -1438,35 +1436,84 @@ __global__ void __launch_bounds__(PART_T) k_partition_small(const DPolys P, cons
     if (j < (int)per && base + j * 64 < np) list[hist[col][key[j]] + rank[j]] = base + j * 64;
 }
 
-// class sizes from the sorted keys: first index of every class after the first by binary search
-__global__ void k_class_counts(const uint64_t* __restrict__ key, uint64_t np, uint32_t* __restrict__ counts) {
-  uint64_t first[CL_COUNT + 1];
-  first[0] = 0;
-  first[CL_COUNT] = np;
-  for (int c = 1; c < CL_COUNT; c++) {
-    uint64_t lo = 0, hi = np;
-    while (lo < hi) {
-      const uint64_t mid = (lo + hi) / 2;
-      if ((key[mid] >> CLASS_BIT) < (uint64_t)c) lo = mid + 1;
-      else hi = mid;
-    }
-    first[c] = lo;
+// The same for more pairs, as one 8-bit pass over tiles of TILE_PAIRS: the keys (a byte per candidate) and every tile's
+// counts, their scan in (key, tile) order, and the scatter, which also leaves the class sizes (a class starts where its
+// first key's first tile does) and clears what the callers' queues need at 0. 215k pairs: 45 us; the 64-bit radix pass
+// with its own kernels for keys, class sizes (a binary search: 15 us) and clearing took 105.
+constexpr int TILE_T = 256, TILE_ITEMS = 16, TILE_PAIRS = TILE_T * TILE_ITEMS, TILE_COLS = TILE_T / 64 * 2;
+__global__ void __launch_bounds__(TILE_T) k_part_count(const DPolys P, const DPolys R, const uint32_t* __restrict__ pa, const uint32_t* __restrict__ pb,
+                                                       const uint8_t* __restrict__ done, uint64_t np, uint32_t mcap, int mixed, uint32_t tcap,
+                                                       uint32_t size_sort, uint8_t* __restrict__ keys, uint32_t ntiles, uint32_t* __restrict__ ghist,
+                                                       OverflowCtl* ctl) {
+  __shared__ uint32_t hist[TILE_COLS][256];
+  const int t = threadIdx.x, col = (t >> 6) * 2 + (t & 1);
+  const uint64_t base = (uint64_t)blockIdx.x * TILE_PAIRS;
+  if (blockIdx.x == 0 && t < 5) ctl[t] = OverflowCtl{0, 0, 0, 0};
+#pragma unroll
+  for (int c = 0; c < TILE_COLS; c++) hist[c][t] = 0;
+  uint32_t a[TILE_ITEMS], b[TILE_ITEMS];
+#pragma unroll
+  for (int j = 0; j < TILE_ITEMS; j++) {
+    const uint64_t i = base + (uint64_t)j * TILE_T + t;
+    a[j] = i < np ? pa[i] : 0u;
+    b[j] = i < np ? pb[i] : 0u;
   }
-  for (int c = 0; c < CL_COUNT; c++) counts[c] = (uint32_t)(first[c + 1] - first[c]);
-  for (int c = CL_TINY; c <= CL_MEDIUM; c++) counts[11 + c] = (uint32_t)first[c];   // the staged launches' queue starts
+#pragma unroll
+  for (int j = 0; j < TILE_ITEMS; j++) { a[j] = P.ginfo[a[j]]; b[j] = R.ginfo[b[j]]; }   // (a layer with candidates has a geometry 0)
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < TILE_ITEMS; j++) {
+    const uint64_t i = base + (uint64_t)j * TILE_T + t;
+    if (i < np) {
+      const uint32_t k = done && done[i] ? KEY_DONE : class_key(a[j], b[j], mcap, mixed, tcap, size_sort);
+      keys[i] = (uint8_t)k;
+      atomicAdd(&hist[col][k], 1u);
+    }
+  }
+  __syncthreads();
+  uint32_t sum = 0;
+#pragma unroll
+  for (int c = 0; c < TILE_COLS; c++) sum += hist[c][t];
+  ghist[(uint64_t)t * ntiles + blockIdx.x] = sum;
+}
+// wave w of a tile takes its w-th run of 64 TILE_ITEMS candidates, so that its list order follows the candidates'
+__global__ void __launch_bounds__(TILE_T) k_part_scatter(const uint8_t* __restrict__ keys, uint64_t np, uint32_t ntiles, const uint32_t* __restrict__ goff,
+                                                         uint32_t* __restrict__ list, uint32_t* __restrict__ counts) {
+  __shared__ uint32_t hist[TILE_COLS][256];
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6, col = 2 * w + (t & 1);
+  const uint64_t base = (uint64_t)blockIdx.x * TILE_PAIRS + (uint64_t)w * 64 * TILE_ITEMS + lane;
+  uint32_t key[TILE_ITEMS], rank[TILE_ITEMS];
+#pragma unroll
+  for (int j = 0; j < TILE_ITEMS; j++) key[j] = base + j * 64 < np ? keys[base + j * 64] : 256u;
+#pragma unroll
+  for (int c = 0; c < TILE_COLS; c++) hist[c][t] = 0;
+  if (blockIdx.x == 0 && t < 16) {   // class sizes [0, 5), the edge queues' counts [8, 11), the staged launches' starts [11, 14)
+    auto first = [&](int cl) { return goff[(uint64_t)(cl << CLASS_BIT) * ntiles]; };
+    counts[t] = t < CL_COUNT ? first(t + 1) - first(t) : (t >= 11 && t < 14) ? first(t - 11) : 0u;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < TILE_ITEMS; j++)
+    if (key[j] < 256) rank[j] = atomicAdd(&hist[col][key[j]], 1u);
+  __syncthreads();
+  uint32_t at = goff[(uint64_t)t * ntiles + blockIdx.x];
+#pragma unroll
+  for (int c = 0; c < TILE_COLS; c++) { const uint32_t v = hist[c][t]; hist[c][t] = at; at += v; }
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < TILE_ITEMS; j++)
+    if (key[j] < 256) list[hist[col][key[j]] + rank[j]] = (uint32_t)(base + j * 64);
 }
 
 // the overflow queue's control at ctl, the host-read queue's (ovf_lds 2) right after it, the promotion queue's 64 bytes on
 __global__ void k_ctl_reset(OverflowCtl* ctl, uint32_t* counts) {
-  ctl[0] = OverflowCtl{0, 0, 0, 0};
-  ctl[1] = OverflowCtl{0, 0, 0, 0};
-  ctl[4] = OverflowCtl{0, 0, 0, 0};
-  for (int k = 0; k < 16; k++) counts[k] = 0;   // class sizes [0, 5) and the edge queues' counts and firsts [8, 14)
+  if (threadIdx.x < 5) ctl[threadIdx.x] = OverflowCtl{0, 0, 0, 0};
+  counts[threadIdx.x] = 0;   // class sizes [0, 5) and the edge queues' counts and firsts [8, 14)
 }
 }  // namespace
 
 PairClasses partition_pairs(Context& c, const DPolys& P, const DPolys& R, const uint32_t* pa, const uint32_t* pb, uint64_t np, uint32_t mcap,
-                            bool mixed, uint32_t tcap, uint32_t size_sort) {
+                            bool mixed, uint32_t tcap, uint32_t size_sort, const uint8_t* done) {
   hipStream_t st = c.stream;
   char* misc = c.s_misc.as<char>(512);   // [0, 32) belongs to the sort primitives
   PairClasses pc;
@@ -1474,28 +1521,27 @@ PairClasses partition_pairs(Context& c, const DPolys& P, const DPolys& R, const 
   pc.ctl = reinterpret_cast<OverflowCtl*>(misc + 128);
   pc.start = reinterpret_cast<uint64_t*>(misc + 256);
   pc.list = nullptr;
-  if (np && np <= (uint64_t)PART_MAX) {
-    pc.list = c.s_vals.as<uint32_t>(np + 16);
-    hipLaunchKernelGGL(k_partition_small, dim3(1), dim3(PART_T), 0, st, P, R, pa, pb, (uint32_t)np, mcap, mixed ? 1 : 0, tcap, size_sort, pc.list,
+  if (np == 0) {
+    hipLaunchKernelGGL(k_ctl_reset, dim3(1), dim3(16), 0, st, pc.ctl, pc.counts);
+    GSJ_LAUNCHED();
+    return pc;
+  }
+  pc.list = c.s_vals.as<uint32_t>(np + 16);
+  if (np <= (uint64_t)PART_MAX) {
+    hipLaunchKernelGGL(k_partition_small, dim3(1), dim3(PART_T), 0, st, P, R, pa, pb, done, (uint32_t)np, mcap, mixed ? 1 : 0, tcap, size_sort, pc.list,
                        pc.counts, pc.ctl);
     GSJ_LAUNCHED();
     return pc;
   }
-  hipLaunchKernelGGL(k_ctl_reset, dim3(1), dim3(1), 0, st, pc.ctl, pc.counts);
+  const uint32_t ntiles = div_up(np, TILE_PAIRS);
+  uint8_t* keys = c.s_keys.as<uint8_t>(np + 16);
+  uint32_t* ghist = c.s_tmp2.as<uint32_t>((uint64_t)256 * ntiles + 8);
+  hipLaunchKernelGGL(k_part_count, dim3(ntiles), dim3(TILE_T), 0, st, P, R, pa, pb, done, np, mcap, mixed ? 1 : 0, tcap, size_sort, keys, ntiles, ghist,
+                     pc.ctl);
   GSJ_LAUNCHED();
-  if (np == 0) return pc;
-  uint64_t* keys = c.s_keys.as<uint64_t>(np + 16);
-  uint64_t* keys2 = c.s_keys2.as<uint64_t>(np + 16);
-  uint32_t* vals = c.s_vals.as<uint32_t>(np + 16);
-  uint32_t* vals2 = c.s_vals2.as<uint32_t>(np + 16);
-  hipLaunchKernelGGL(k_class_keys, dim3(div_up(np, 256)), dim3(256), 0, st, P, R, pa, pb, np, mcap, mixed ? 1 : 0, tcap, size_sort, keys, vals);
+  scan_loaded<uint32_t>(c, LoadArray<uint32_t>{ghist}, ghist, (uint64_t)256 * ntiles, ScanTotal{});
+  hipLaunchKernelGGL(k_part_scatter, dim3(ntiles), dim3(TILE_T), 0, st, keys, np, ntiles, ghist, pc.list, pc.counts);
   GSJ_LAUNCHED();
-  // stable (candidate order within a key); one 8-bit digit, sorted without probing whether it varies: no host
-  // synchronisation
-  radix_sort_pairs(c, keys, keys2, vals, vals2, np, 0, 8, false);
-  hipLaunchKernelGGL(k_class_counts, dim3(1), dim3(1), 0, st, keys, np, pc.counts);
-  GSJ_LAUNCHED();
-  pc.list = vals;
   return pc;
 }
 

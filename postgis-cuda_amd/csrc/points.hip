@@ -1,6 +1,6 @@
 // Points in polygons (reference: k_pip_pairs / join_points_stream, engine/engine.cuh:1079-1178) and
 // ST_ClusterIntersecting by lock-free union-find over the intersects rows (engine/engine.cuh:1183-1234).
-#include "engine.h"
+#include "scan.h"
 #include <algorithm>
 #include <chrono>
 
@@ -10,67 +10,174 @@ namespace {
 
 __device__ __forceinline__ int syn_bit(const uint32_t* synb, uint64_t i) { return synb ? (int)((synb[i >> 5] >> (i & 31)) & 1u) : 0; }
 
-// thread per (point, piece): 2 = on a real edge, 1 = interior (crossing parity of a horizontal segment from a point
-// left of the piece's bbox), 0 = outside. Coordinates relative to the piece's origin (exact, as everywhere).
+// where a point lies in a piece, edge by edge: on a real edge, or by the crossing parity of a horizontal segment from a
+// point left of the piece's bbox. Coordinates relative to the piece's origin (exact, as everywhere).
+struct PipTest {
+  double px, py, ox;
+  bool par = false, on = false;
+  __device__ __forceinline__ PipTest(const double2 pt, const double2 o) : px(pt.x - o.x), py(pt.y - o.y), ox((o.x - o.x) - 1.0) {}
+  template <class Syn>
+  __device__ __forceinline__ void edge(const double2 v0, const double2 v1, const Syn& syn) {
+    const double x0 = v0.x, y0 = v0.y, x1 = v1.x, y1 = v1.y;
+    if ((y0 > py) == (y1 > py) && y0 != py && y1 != py) return;
+    if (orient(x0, y0, x1, y1, px, py) == 0 && !syn() && onseg(x0, y0, x1, y1, px, py)) { on = true; return; }
+    const bool so = left_of(x0, y0, x1, y1, ox, py), sp = left_of(x0, y0, x1, y1, px, py);
+    if (so == sp) return;
+    const bool su = orient(ox, py, px, py, x0, y0) > 0, sv = orient(ox, py, px, py, x1, y1) > 0;
+    if (su != sv) par = !par;
+  }
+  __device__ __forceinline__ uint8_t result() const { return on ? 2 : (par ? 1 : 0); }
+};
+
+// thread per (point, piece): 2 = on a real edge, 1 = interior, 0 = outside. Pieces with a packed record are read from it
+// (one contiguous run instead of geometry -> ring -> vertices), four vertices in flight at a time; the others by their
+// edge chunks. Bound by the latency of those loads: neighbouring points (the walk is in Morton order) share their
+// pieces in cache. 3M points, 4.2M candidates in parcels of 13 vertices: 321 -> 251 us.
 __global__ void __launch_bounds__(256) k_pip(const DPoints pts, const DPolys R, const uint32_t* __restrict__ pa, const uint32_t* __restrict__ pb,
                                              uint64_t np, uint8_t* __restrict__ hit) {
   const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= np) return;
-  const uint32_t g = pb[i];
-  const double2 pt = pts.xy[pa[i]], o = R.origin[g];
-  const double px = pt.x - o.x, py = pt.y - o.y;
-  const double ox = (o.x - o.x) - 1.0;
-  bool par = false, on = false;
+  const uint32_t g = pb[i], po = R.pk_off[g];
+  const double2 pt = pts.xy[pa[i]];
+  if (po != NO_PACK) {
+    const uint4* rec = R.pk + po;
+    PipTest t(pt, reinterpret_cast<const double2*>(rec)[0]);
+    const uint8_t* h = reinterpret_cast<const uint8_t*>(rec + 2);
+    const int nv = h[0];
+    const double2* V = reinterpret_cast<const double2*>(rec + 3);
+    const uint8_t* F = reinterpret_cast<const uint8_t*>(rec + 3 + nv);
+    int ring = 0, end = nv ? h[3] : 0;   // the ring that holds vertex k ends at `end`
+    double2 v0 = nv ? V[0] : make_double2(0.0, 0.0);
+    for (int k = 0; k + 1 < nv && !t.on; k += 4) {
+      double2 v[4];
+#pragma unroll
+      for (int j = 0; j < 4; j++) v[j] = V[min(k + 1 + j, nv - 1)];
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        const int e = k + j;   // the edge e, e + 1
+        if (e + 1 >= nv || t.on) break;
+        while (e >= end) end = h[3 + ++ring];
+        if (e + 1 < end) t.edge(v0, v[j], [&] { return (F[e] & VF_SYN) != 0; });
+        v0 = v[j];
+      }
+    }
+    hit[i] = t.result();
+    return;
+  }
+  PipTest t(pt, R.origin[g]);
   const uint32_t r1 = R.gro[g + 1];
   const uint64_t vg = R.rvo[R.gro[g]];
   const uint32_t cf = R.cfirst ? R.cfirst[g] : NO_CHUNKS;
-  for (uint32_t r = R.gro[g]; r < r1 && !on; r++) {
+  for (uint32_t r = R.gro[g]; r < r1 && !t.on; r++) {
     const uint64_t s0 = R.rvo[r], e = R.rvo[r + 1];
     // edges (j-1, j) taken an edge chunk at a time; a chunk whose vertices all lie strictly above or strictly below
     // the row y = py holds only edges the parity test skips
-    for (uint64_t a = s0; a + 1 < e && !on;) {
+    for (uint64_t a = s0; a + 1 < e && !t.on;) {
       uint64_t b = e - 1;
       if (cf != NO_CHUNKS) {
         const uint64_t k = (a - vg) / CHUNK;
         b = min(b, vg + (k + 1) * CHUNK);
         const float4 c = R.cbb[cf + k];
-        if ((double)c.y > py || (double)c.w < py) { a = b; continue; }
+        if ((double)c.y > t.py || (double)c.w < t.py) { a = b; continue; }
       }
       double2 v0 = R.xy[a];
-      for (uint64_t j = a + 1; j <= b; j++) {
+      for (uint64_t j = a + 1; j <= b && !t.on; j++) {
         const double2 v1 = R.xy[j];
-        const double x0 = v0.x, y0 = v0.y, x1 = v1.x, y1 = v1.y;
-        if (!((y0 > py) == (y1 > py) && y0 != py && y1 != py)) {
-          if (orient(x0, y0, x1, y1, px, py) == 0 && !syn_bit(R.synb, j - 1) && onseg(x0, y0, x1, y1, px, py)) { on = true; break; }
-          const bool so = left_of(x0, y0, x1, y1, ox, py), sp = left_of(x0, y0, x1, y1, px, py);
-          if (so != sp) {
-            const bool su = orient(ox, py, px, py, x0, y0) > 0, sv = orient(ox, py, px, py, x1, y1) > 0;
-            if (su != sv) par = !par;
-          }
-        }
+        t.edge(v0, v1, [&] { return syn_bit(R.synb, j - 1) != 0; });
         v0 = v1;
       }
       a = b;
     }
   }
-  hit[i] = on ? 2 : (par ? 1 : 0);
+  hit[i] = t.result();
 }
 
-__global__ void k_hit_flags(const uint8_t* __restrict__ hit, uint64_t n, uint32_t* __restrict__ f) {
-  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) f[i] = hit[i] != 0;
-}
+struct LoadAny {
+  static constexpr bool PACKED = false;
+  const uint8_t* f;
+  __device__ __forceinline__ uint64_t operator()(uint64_t i) const { return f[i] != 0; }
+};
 
 // direct rows (no subdivided parents) or (point, parent) keys for the fold
 __global__ void k_pip_emit(const DPolys R, const uint32_t* __restrict__ pa, const uint32_t* __restrict__ pb, const uint8_t* __restrict__ hit,
-                           const uint32_t* __restrict__ f, const uint64_t* __restrict__ offs, uint64_t n, uint32_t* __restrict__ orow,
+                           const uint64_t* __restrict__ offs, uint64_t n, uint32_t* __restrict__ orow,
                            uint8_t* __restrict__ owhere, uint64_t* __restrict__ keys, uint32_t* __restrict__ vals) {
   const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n || !f[i]) return;
+  if (i >= n || !hit[i]) return;
   const uint64_t o = offs[i];
   const uint32_t b = R.parent ? R.parent[pb[i]] : pb[i];
   if (keys) { keys[o] = ((uint64_t)pa[i] << 32) | b; vals[o] = hit[i]; return; }
-  orow[2 * o] = pa[i]; orow[2 * o + 1] = b; owhere[o] = hit[i];
+  reinterpret_cast<uint2*>(orow)[o] = make_uint2(pa[i], b);
+  owhere[o] = hit[i];
+}
+
+// Rows of a subdivided layer come by point, then parent, the pieces of a parent folded (boundary wins over interior). A
+// point's candidates are a run, so its rows are counted, the counts scanned in point order, and every run writes its
+// own: two passes over the candidates and a scan instead of a 64-bit sort of the rows (1.76M candidates of 3M points:
+// 813 -> 231 us, half of it the scattered rows). RUN_MAX: a run is searched once per parent, so a batch with a longer one
+// (counted in *over) keeps the sort. COUNT_POINTS: the scan takes 12 us per million points of the layer, whatever the
+// batch holds of them, and the sort 180 us and 0.36 us per thousand candidates, so that layers of more points than this
+// are scanned only for batches of a 32nd of them (500 candidates: 178 -> 49 us of 300k points, 248 -> 82 of 3M).
+constexpr int RUN_MAX = 16;
+constexpr uint32_t COUNT_POINTS = 8u << 20;
+// calls row(parent, where) for the distinct parents of the run's hits, ascending
+template <class Row>
+__device__ __forceinline__ void run_rows(const DPolys& R, const uint32_t* pb, const uint8_t* hit, uint64_t i, uint64_t e, const Row& row) {
+  int64_t last = -1;
+  for (;;) {
+    int64_t next = -1;
+    uint8_t w = 0;
+    for (uint64_t j = i; j < e; j++) {
+      if (!hit[j]) continue;
+      const int64_t q = R.parent[pb[j]];
+      if (q <= last || (next >= 0 && q > next)) continue;
+      w = q == next ? max(w, hit[j]) : hit[j];
+      next = q;
+    }
+    if (next < 0) return;
+    row((uint32_t)next, w);
+    last = next;
+  }
+}
+// end of the run of candidates that starts at i (at most RUN_MAX; the rest is then left out), or i when one is under way
+__device__ __forceinline__ uint64_t run_end(const uint32_t* pa, uint64_t i, uint64_t np, bool& longer) {
+  const uint32_t q = pa[i];
+  if (i > 0 && pa[i - 1] == q) return i;
+  uint64_t e = i + 1;
+  while (e < np && e < i + RUN_MAX && pa[e] == q) e++;
+  longer = e < np && e == i + RUN_MAX && pa[e] == q;
+  return e;
+}
+__global__ void k_pip_count(const DPolys R, const uint32_t* __restrict__ pa, const uint32_t* __restrict__ pb, const uint8_t* __restrict__ hit, uint64_t np,
+                            uint32_t* __restrict__ cnt, uint32_t* __restrict__ over) {
+  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= np) return;
+  bool longer = false;
+  const uint64_t e = run_end(pa, i, np, longer);
+  if (e == i) return;
+  if (longer) atomicAdd(over, 1u);
+  uint32_t n = 0;
+  run_rows(R, pb, hit, i, e, [&](uint32_t, uint8_t) { n++; });
+  cnt[pa[i]] = n;
+}
+__global__ void k_pip_rows(const DPolys R, const uint32_t* __restrict__ pa, const uint32_t* __restrict__ pb, const uint8_t* __restrict__ hit, uint64_t np,
+                           const uint64_t* __restrict__ off, uint32_t* __restrict__ orow, uint8_t* __restrict__ owhere) {
+  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= np) return;
+  bool longer = false;
+  const uint64_t e = run_end(pa, i, np, longer);
+  if (e == i) return;
+  const uint32_t q = pa[i];
+  uint64_t o = off[q];
+  run_rows(R, pb, hit, i, e, [&](uint32_t parent, uint8_t w) {
+    reinterpret_cast<uint2*>(orow)[o] = make_uint2(q, parent);
+    owhere[o] = w;
+    o++;
+  });
+}
+__global__ void k_fill_zero(uint32_t* p, uint64_t n) {
+  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) p[i] = 0u;
 }
 
 __global__ void k_heads64(const uint64_t* __restrict__ keys, uint64_t m, uint32_t* __restrict__ head) {
@@ -175,42 +282,65 @@ void points_join_run(Context& c, const Layer& PL, const Layer& RL, const gsj_joi
       hipLaunchKernelGGL(k_pip, dim3(div_up(np, 256)), dim3(256), 0, stream, PL.pts, RL.poly, pa, pb, np, hit);
       GSJ_LAUNCHED();
       GSJ_HIP(hipEventRecord(c.ev[1], stream));
-      GSJ_HIP(hipStreamSynchronize(stream));
-      float ms = 0;
+      s.refine_ms += t2.ms();
+      WallTimer t3;
+      uint64_t* hoffs = c.s_offs.as<uint64_t>(np + 16);
+      uint32_t* orow = c.s_out_a.as<uint32_t>(2 * np + 16);
+      uint8_t* owhere = c.s_out_flag.as<uint8_t>(np + 16);
+      const HostWords w = host_words(c, 0, 2);
+      uint64_t nrows = 0;
+      bool sort = RL.poly.parent && PL.n > COUNT_POINTS && np < PL.n / 32;
+      if (!RL.poly.parent) {
+        scan_loaded<uint64_t>(c, LoadAny{hit}, hoffs, np, ScanTotal{w.dev});
+        hipLaunchKernelGGL(k_pip_emit, dim3(div_up(np, 256)), dim3(256), 0, stream, RL.poly, pa, pb, hit, hoffs, np, orow, owhere, nullptr, nullptr);
+        GSJ_LAUNCHED();
+        w.fetch(c);
+        GSJ_HIP(hipStreamSynchronize(stream));
+        nrows = w.host[0];
+      } else if (!sort) {
+        uint32_t* cnt = c.s_seg.as<uint32_t>(PL.n + 17);
+        uint32_t* over = cnt + PL.n;
+        uint64_t* off = c.s_tmp2.as<uint64_t>(PL.n + 16);
+        hipLaunchKernelGGL(k_fill_zero, dim3(div_up(PL.n + 1, 256)), dim3(256), 0, stream, cnt, PL.n + 1);
+        GSJ_LAUNCHED();
+        hipLaunchKernelGGL(k_pip_count, dim3(div_up(np, 256)), dim3(256), 0, stream, RL.poly, pa, pb, hit, np, cnt, over);
+        GSJ_LAUNCHED();
+        scan_loaded<uint64_t>(c, LoadArray<uint32_t>{cnt}, off, PL.n, ScanTotal{w.dev, over});
+        hipLaunchKernelGGL(k_pip_rows, dim3(div_up(np, 256)), dim3(256), 0, stream, RL.poly, pa, pb, hit, np, off, orow, owhere);
+        GSJ_LAUNCHED();
+        w.fetch(c);
+        GSJ_HIP(hipStreamSynchronize(stream));
+        nrows = w.host[0];
+        sort = w.host[1] != 0;
+      }
+      if (sort) {
+        scan_loaded<uint64_t>(c, LoadAny{hit}, hoffs, np, ScanTotal{w.dev});
+        w.fetch(c);
+        GSJ_HIP(hipStreamSynchronize(stream));
+        const uint64_t nh = w.host[0];
+        nrows = 0;
+        if (nh) {
+          uint64_t* keys = c.s_keys.as<uint64_t>(nh);
+          uint64_t* keys2 = c.s_keys2.as<uint64_t>(nh);
+          uint32_t* vals = c.s_vals.as<uint32_t>(nh);
+          uint32_t* vals2 = c.s_vals2.as<uint32_t>(nh);
+          hipLaunchKernelGGL(k_pip_emit, dim3(div_up(np, 256)), dim3(256), 0, stream, RL.poly, pa, pb, hit, hoffs, np, orow, owhere, keys, vals);
+          GSJ_LAUNCHED();
+          radix_sort_pairs(c, keys, keys2, vals, vals2, nh, 0, 64);
+          uint32_t* head = c.s_seg.as<uint32_t>(nh + 16);
+          uint64_t* hoff2 = c.s_tmp2.as<uint64_t>(nh + 16);
+          hipLaunchKernelGGL(k_heads64, dim3(div_up(nh, 256)), dim3(256), 0, stream, keys, nh, head);
+          GSJ_LAUNCHED();
+          nrows = scan_u32_to_u64(c, head, hoff2, nh);
+          hipLaunchKernelGGL(k_pip_fold, dim3(div_up(nh, 256)), dim3(256), 0, stream, keys, vals, head, hoff2, nh, orow, owhere);
+          GSJ_LAUNCHED();
+        }
+      }
+      float ms = 0;   // (every way here has waited for the stream since)
       GSJ_HIP(hipEventElapsedTime(&ms, c.ev[0], c.ev[1]));
       s.k_small_ms += ms;
       s.n_small += np;
       s.launches++;
-      s.refine_ms += t2.ms();
-      WallTimer t3;
-      uint32_t* f = c.s_tmp.as<uint32_t>(np + 16);
-      uint64_t* hoffs = c.s_offs.as<uint64_t>(np + 16);
-      hipLaunchKernelGGL(k_hit_flags, dim3(div_up(np, 256)), dim3(256), 0, stream, hit, np, f);
-      GSJ_LAUNCHED();
-      const uint64_t nh = scan_u32_to_u64(c, f, hoffs, np);
-      uint32_t* orow = c.s_out_a.as<uint32_t>(2 * np + 16);
-      uint8_t* owhere = c.s_out_flag.as<uint8_t>(np + 16);
-      uint64_t nrows = nh;
-      if (!RL.poly.parent) {
-        hipLaunchKernelGGL(k_pip_emit, dim3(div_up(np, 256)), dim3(256), 0, stream, RL.poly, pa, pb, hit, f, hoffs, np, orow, owhere, nullptr, nullptr);
-        GSJ_LAUNCHED();
-      } else if (nh) {
-        uint64_t* keys = c.s_keys.as<uint64_t>(nh);
-        uint64_t* keys2 = c.s_keys2.as<uint64_t>(nh);
-        uint32_t* vals = c.s_vals.as<uint32_t>(nh);
-        uint32_t* vals2 = c.s_vals2.as<uint32_t>(nh);
-        hipLaunchKernelGGL(k_pip_emit, dim3(div_up(np, 256)), dim3(256), 0, stream, RL.poly, pa, pb, hit, f, hoffs, np, orow, owhere, keys, vals);
-        GSJ_LAUNCHED();
-        radix_sort_pairs(c, keys, keys2, vals, vals2, nh, 0, 64);
-        uint32_t* head = c.s_seg.as<uint32_t>(nh + 16);
-        uint64_t* hoff2 = c.s_tmp2.as<uint64_t>(nh + 16);
-        hipLaunchKernelGGL(k_heads64, dim3(div_up(nh, 256)), dim3(256), 0, stream, keys, nh, head);
-        GSJ_LAUNCHED();
-        nrows = scan_u32_to_u64(c, head, hoff2, nh);
-        hipLaunchKernelGGL(k_pip_fold, dim3(div_up(nh, 256)), dim3(256), 0, stream, keys, vals, head, hoff2, nh, orow, owhere);
-        GSJ_LAUNCHED();
-      }
-      GSJ_HIP(hipStreamSynchronize(stream));
       s.compact_ms += t3.ms();
       s.hits += nrows;
       if (!nrows) return;

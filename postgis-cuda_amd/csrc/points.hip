@@ -115,11 +115,8 @@ __global__ void k_pip_emit(const DPolys R, const uint32_t* __restrict__ pa, cons
 // point's candidates are a run, so its rows are counted, the counts scanned in point order, and every run writes its
 // own: two passes over the candidates and a scan instead of a 64-bit sort of the rows (1.76M candidates of 3M points:
 // 813 -> 231 us, half of it the scattered rows). RUN_MAX: a run is searched once per parent, so a batch with a longer one
-// (counted in *over) keeps the sort. COUNT_POINTS: the scan takes 12 us per million points of the layer, whatever the
-// batch holds of them, and the sort 180 us and 0.36 us per thousand candidates, so that layers of more points than this
-// are scanned only for batches of a 32nd of them (500 candidates: 178 -> 49 us of 300k points, 248 -> 82 of 3M).
+// (counted in *over) keeps the sort.
 constexpr int RUN_MAX = 16;
-constexpr uint32_t COUNT_POINTS = 8u << 20;
 // calls row(parent, where) for the distinct parents of the run's hits, ascending
 template <class Row>
 __device__ __forceinline__ void run_rows(const DPolys& R, const uint32_t* pb, const uint8_t* hit, uint64_t i, uint64_t e, const Row& row) {
@@ -289,7 +286,7 @@ void points_join_run(Context& c, const Layer& PL, const Layer& RL, const gsj_joi
       uint8_t* owhere = c.s_out_flag.as<uint8_t>(np + 16);
       const HostWords w = host_words(c, 0, 2);
       uint64_t nrows = 0;
-      bool sort = RL.poly.parent && PL.n > COUNT_POINTS && np < PL.n / 32;
+      bool sort = RL.poly.parent && !points_counted(PL.n, np);
       if (!RL.poly.parent) {
         scan_loaded<uint64_t>(c, LoadAny{hit}, hoffs, np, ScanTotal{w.dev});
         hipLaunchKernelGGL(k_pip_emit, dim3(div_up(np, 256)), dim3(256), 0, stream, RL.poly, pa, pb, hit, hoffs, np, orow, owhere, nullptr, nullptr);

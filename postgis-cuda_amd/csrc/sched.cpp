@@ -41,7 +41,8 @@ struct Req {
 // Scratch estimate of a request: candidate pairs bounded by the sub-batch limit, ~120 B of pair state each
 // (pairs, flags, areas, evidence, partition lists, compaction keys) and, where distances are reported, 136 B more (two
 // queued items of 68 B, at most 2^25 of them), plus per-probe traversal counters. The probes are
-// the probe layer's, or for a window over a layer with tile boxes, the probes of the tiles meeting the window.
+// the probe layer's, or for a window over a layer with tile boxes, the probes of the tiles meeting the window. Points in
+// polygons count their rows per point of the layer (12 B each).
 uint64_t estimate_scratch(const gsj_request& r) {
   uint64_t nq = r.P ? r.P->L.n : 0;
   const std::vector<float4>& tiles = r.P ? r.P->L.h_tiles : std::vector<float4>();
@@ -54,7 +55,8 @@ uint64_t estimate_scratch(const gsj_request& r) {
   const uint64_t max_pairs = r.opts.max_pairs ? r.opts.max_pairs : (128ull << 20);
   const uint64_t pairs = std::min<uint64_t>(max_pairs, 8 * nq + 1024);
   const uint64_t items = r.report_distance ? std::min<uint64_t>(2 * pairs, 1ull << 25) : 0;
-  return pairs * 120 + items * 68 + nq * 24;
+  const uint64_t counted = r.kind == GSJ_REQ_POINTS_IN_POLYGONS && r.P && r.R && r.R->L.poly.parent ? gsj::points_counted(r.P->L.n, pairs) : 0;
+  return pairs * 120 + items * 68 + nq * 24 + counted * 12;
 }
 
 }  // namespace

@@ -856,11 +856,10 @@ void dw_deliver(Context& c, const uint32_t* orow, const double* odist, uint64_t 
   WallTimer t4;
   uint32_t* hrow = c.h_pairs.as<uint32_t>(2 * nrows);
   double* hd = odist ? c.h_area.as<double>(nrows) : nullptr;
-  GSJ_HIP(hipMemcpyAsync(hrow, orow, nrows * 8, hipMemcpyDeviceToHost, c.stream));
-  if (hd) GSJ_HIP(hipMemcpyAsync(hd, odist, nrows * 8, hipMemcpyDeviceToHost, c.stream));
-  GSJ_HIP(hipStreamSynchronize(c.stream));
+  const RowPart parts[2] = {{orow, hrow, 8}, {odist, hd, 8}};
+  const bool stop = deliver_rows(c, parts, hd ? 2 : 1, nrows, [&](uint64_t r, uint64_t n) { return cb ? cb(user, hrow + 2 * r, hd ? hd + r : nullptr, (size_t)n) : 0; });
   s.copy_ms += t4.ms();
-  if (cb && cb(user, hrow, hd, (size_t)nrows)) throw Error(GSJ_E_CANCEL, "distance join cancelled by the row callback");
+  if (stop) throw Error(GSJ_E_CANCEL, "distance join cancelled by the row callback");
 }
 
 }  // namespace

@@ -362,10 +362,10 @@ uint64_t compact_rows(Context& c, const Layer& PL, const Layer& RL, const uint32
 
 // Sub-batches of at most this many candidates write their rows straight into pinned host memory (at the link's rate: 258k
 // rows of 12 bytes in 59 us) instead of copying them once their number is known: one host wait instead of two, and none
-// for the refinement where it reads nothing back. The buffers take as many rows as candidates; larger sub-batches copy
-// what they kept. A context without pinned memory copies np rows, an upper bound, in the same wait where nothing is
-// folded.
-constexpr uint64_t DIRECT_ROWS = 8u << 20;
+// for the refinement where it reads nothing back. Larger ones deliver from device memory, where the copy of all but the
+// first rows hides behind the callback's work (deliver_rows). A context without pinned memory copies np rows, an upper
+// bound, in the same wait where nothing is folded.
+constexpr uint64_t DIRECT_ROWS = 256u << 10;
 
 }  // namespace
 
@@ -448,12 +448,15 @@ void join_run(Context& c, const Layer& PL, const Layer& RL, const gsj_join_opts&
     uint32_t* hrow = c.h_pairs.as<uint32_t>(2 * nrows);
     double* harea = rp.want_area ? c.h_area.as<double>(nrows) : nullptr;
     uint32_t* hcode = rp.want_relate ? c.h_code.as<uint32_t>(nrows) : nullptr;
-    GSJ_HIP(hipMemcpyAsync(hrow, orow, nrows * 8, hipMemcpyDeviceToHost, stream));
-    if (harea) GSJ_HIP(hipMemcpyAsync(harea, oarea, nrows * 8, hipMemcpyDeviceToHost, stream));
-    if (hcode) GSJ_HIP(hipMemcpyAsync(hcode, ocode, nrows * 4, hipMemcpyDeviceToHost, stream));
-    GSJ_HIP(hipStreamSynchronize(stream));
+    RowPart parts[3] = {{orow, hrow, 8}};
+    int np_ = 1;
+    if (harea) parts[np_++] = {oarea, harea, 8};
+    if (hcode) parts[np_++] = {ocode, hcode, 4};
+    const bool stop = deliver_rows(c, parts, np_, nrows, [&](uint64_t r, uint64_t n) {
+      return cb ? cb(user, hrow + 2 * r, harea ? harea + r : nullptr, hcode ? hcode + r : nullptr, (size_t)n) : 0;
+    });
     s.copy_ms += t4.ms();
-    if (cb && cb(user, hrow, harea, hcode, (size_t)nrows)) throw Error(GSJ_E_CANCEL, "join cancelled by the row callback");
+    if (stop) throw Error(GSJ_E_CANCEL, "join cancelled by the row callback");
   }, hooks ? hooks->on_members : none);
   if (st) *st = s;
 }

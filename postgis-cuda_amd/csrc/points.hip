@@ -344,11 +344,10 @@ void points_join_run(Context& c, const Layer& PL, const Layer& RL, const gsj_joi
       WallTimer t4;
       uint32_t* hrow = c.h_pairs.as<uint32_t>(2 * nrows);
       uint8_t* hw = c.h_where.as<uint8_t>(nrows);
-      GSJ_HIP(hipMemcpyAsync(hrow, orow, nrows * 8, hipMemcpyDeviceToHost, stream));
-      GSJ_HIP(hipMemcpyAsync(hw, owhere, nrows, hipMemcpyDeviceToHost, stream));
-      GSJ_HIP(hipStreamSynchronize(stream));
+      const RowPart parts[2] = {{orow, hrow, 8}, {owhere, hw, 1}};
+      const bool stop = deliver_rows(c, parts, 2, nrows, [&](uint64_t r, uint64_t n) { return cb ? cb(user, hrow + 2 * r, hw + r, (size_t)n) : 0; });
       s.copy_ms += t4.ms();
-      if (cb && cb(user, hrow, hw, (size_t)nrows)) throw Error(GSJ_E_CANCEL, "points join cancelled by the row callback");
+      if (stop) throw Error(GSJ_E_CANCEL, "points join cancelled by the row callback");
   });
   if (st) *st = s;
 }

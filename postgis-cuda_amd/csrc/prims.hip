@@ -147,4 +147,27 @@ void radix_sort_pairs(Context& c, uint64_t*& keys, uint64_t*& keys_alt, uint32_t
   }
 }
 
+bool deliver_rows(Context& c, const RowPart* parts, int nparts, uint64_t nrows, const std::function<int(uint64_t first, uint64_t n)>& give) {
+  const uint64_t nchunks = (nrows + DELIVER_ROWS - 1) / DELIVER_ROWS;
+  auto rows_of = [&](uint64_t k) { return std::min(DELIVER_ROWS, nrows - k * DELIVER_ROWS); };
+  auto send = [&](uint64_t k) {
+    for (int p = 0; p < nparts; p++) {
+      const size_t off = k * DELIVER_ROWS * parts[p].bytes;
+      GSJ_HIP(hipMemcpyAsync(static_cast<char*>(parts[p].host) + off, static_cast<const char*>(parts[p].dev) + off, rows_of(k) * parts[p].bytes,
+                             hipMemcpyDeviceToHost, c.stream));
+    }
+    GSJ_HIP(hipEventRecord(c.ev[17 + (k & 1)], c.stream));
+  };
+  if (nchunks) send(0);
+  for (uint64_t k = 0; k < nchunks; k++) {
+    if (k + 1 < nchunks) send(k + 1);
+    GSJ_HIP(hipEventSynchronize(c.ev[17 + (k & 1)]));
+    if (give(k * DELIVER_ROWS, rows_of(k))) {
+      GSJ_HIP(hipStreamSynchronize(c.stream));
+      return true;
+    }
+  }
+  return false;
+}
+
 }  // namespace gsj

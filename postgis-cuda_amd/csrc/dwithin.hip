@@ -853,12 +853,10 @@ uint64_t dw_compact(Context& c, const uint32_t* Ppar, const uint32_t* Rpar, cons
 // deliver one sub-batch's rows through the callback
 void dw_deliver(Context& c, const uint32_t* orow, const double* odist, uint64_t nrows, gsj_join_stats& s, gsj_dist_cb cb, void* user) {
   if (nrows == 0) return;
-  WallTimer t4;
   uint32_t* hrow = c.h_pairs.as<uint32_t>(2 * nrows);
   double* hd = odist ? c.h_area.as<double>(nrows) : nullptr;
   const RowPart parts[2] = {{orow, hrow, 8}, {odist, hd, 8}};
-  const bool stop = deliver_rows(c, parts, hd ? 2 : 1, nrows, [&](uint64_t r, uint64_t n) { return cb ? cb(user, hrow + 2 * r, hd ? hd + r : nullptr, (size_t)n) : 0; });
-  s.copy_ms += t4.ms();
+  const bool stop = deliver_rows(c, parts, hd ? 2 : 1, nrows, s.copy_ms, [&](uint64_t r, uint64_t n) { return cb ? cb(user, hrow + 2 * r, hd ? hd + r : nullptr, (size_t)n) : 0; });
   if (stop) throw Error(GSJ_E_CANCEL, "distance join cancelled by the row callback");
 }
 

@@ -174,14 +174,15 @@ void key_bits(Context& c, const uint64_t* keys, uint64_t n, uint64_t& or_all, ui
 // before it (3M points in parcels, 24 MB of rows: 2277 -> 1975 us a call, of a 1M self-join 9.85 -> 9.5 ms). Chunks of 512k
 // rows are within 1-4% of it, of 64k slower (2462 us: each costs two copies, an event and a wait). parts: the arrays of a
 // row (bytes per row); give(first, n) hands rows [first, first + n) on from the host arrays and returns nonzero to stop.
-// Returns whether it was stopped; nothing is in flight then.
+// Returns whether it was stopped; nothing is in flight then. copy_ms grows by the time spent sending and waiting.
 constexpr uint64_t DELIVER_ROWS = 256u << 10;
 struct RowPart {
   const void* dev;
   void* host;
   size_t bytes;
 };
-bool deliver_rows(Context& c, const RowPart* parts, int nparts, uint64_t nrows, const std::function<int(uint64_t first, uint64_t n)>& give);
+bool deliver_rows(Context& c, const RowPart* parts, int nparts, uint64_t nrows, double& copy_ms,
+                  const std::function<int(uint64_t first, uint64_t n)>& give);
 
 // ------------------------------------------------------------------------------------------- layers / bvh
 void layer_upload_polys(Layer& L, const uint64_t* gro, const uint64_t* rvo, const double* xy, uint64_t n, uint64_t nr, uint64_t nv,

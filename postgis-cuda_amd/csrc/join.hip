@@ -444,7 +444,6 @@ void join_run(Context& c, const Layer& PL, const Layer& RL, const gsj_join_opts&
     s.hits += nrows;
     if (hooks && hooks->on_device && nrows) hooks->on_device(orow, rp.want_area ? oarea : nullptr, nrows);
     if ((hooks && hooks->device_only) || nrows == 0) return;
-    WallTimer t4;
     uint32_t* hrow = c.h_pairs.as<uint32_t>(2 * nrows);
     double* harea = rp.want_area ? c.h_area.as<double>(nrows) : nullptr;
     uint32_t* hcode = rp.want_relate ? c.h_code.as<uint32_t>(nrows) : nullptr;
@@ -452,10 +451,9 @@ void join_run(Context& c, const Layer& PL, const Layer& RL, const gsj_join_opts&
     int np_ = 1;
     if (harea) parts[np_++] = {oarea, harea, 8};
     if (hcode) parts[np_++] = {ocode, hcode, 4};
-    const bool stop = deliver_rows(c, parts, np_, nrows, [&](uint64_t r, uint64_t n) {
+    const bool stop = deliver_rows(c, parts, np_, nrows, s.copy_ms, [&](uint64_t r, uint64_t n) {
       return cb ? cb(user, hrow + 2 * r, harea ? harea + r : nullptr, hcode ? hcode + r : nullptr, (size_t)n) : 0;
     });
-    s.copy_ms += t4.ms();
     if (stop) throw Error(GSJ_E_CANCEL, "join cancelled by the row callback");
   }, hooks ? hooks->on_members : none);
   if (st) *st = s;

@@ -341,12 +341,10 @@ void points_join_run(Context& c, const Layer& PL, const Layer& RL, const gsj_joi
       s.compact_ms += t3.ms();
       s.hits += nrows;
       if (!nrows) return;
-      WallTimer t4;
       uint32_t* hrow = c.h_pairs.as<uint32_t>(2 * nrows);
       uint8_t* hw = c.h_where.as<uint8_t>(nrows);
       const RowPart parts[2] = {{orow, hrow, 8}, {owhere, hw, 1}};
-      const bool stop = deliver_rows(c, parts, 2, nrows, [&](uint64_t r, uint64_t n) { return cb ? cb(user, hrow + 2 * r, hw + r, (size_t)n) : 0; });
-      s.copy_ms += t4.ms();
+      const bool stop = deliver_rows(c, parts, 2, nrows, s.copy_ms, [&](uint64_t r, uint64_t n) { return cb ? cb(user, hrow + 2 * r, hw + r, (size_t)n) : 0; });
       if (stop) throw Error(GSJ_E_CANCEL, "points join cancelled by the row callback");
   });
   if (st) *st = s;

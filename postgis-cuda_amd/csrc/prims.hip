@@ -147,7 +147,8 @@ void radix_sort_pairs(Context& c, uint64_t*& keys, uint64_t*& keys_alt, uint32_t
   }
 }
 
-bool deliver_rows(Context& c, const RowPart* parts, int nparts, uint64_t nrows, const std::function<int(uint64_t first, uint64_t n)>& give) {
+bool deliver_rows(Context& c, const RowPart* parts, int nparts, uint64_t nrows, double& copy_ms,
+                  const std::function<int(uint64_t first, uint64_t n)>& give) {
   const uint64_t nchunks = (nrows + DELIVER_ROWS - 1) / DELIVER_ROWS;
   auto rows_of = [&](uint64_t k) { return std::min(DELIVER_ROWS, nrows - k * DELIVER_ROWS); };
   auto send = [&](uint64_t k) {
@@ -158,10 +159,13 @@ bool deliver_rows(Context& c, const RowPart* parts, int nparts, uint64_t nrows, 
     }
     GSJ_HIP(hipEventRecord(c.ev[17 + (k & 1)], c.stream));
   };
+  WallTimer t0;
   if (nchunks) send(0);
   for (uint64_t k = 0; k < nchunks; k++) {
+    WallTimer t;
     if (k + 1 < nchunks) send(k + 1);
     GSJ_HIP(hipEventSynchronize(c.ev[17 + (k & 1)]));
+    copy_ms += k ? t.ms() : t0.ms();
     if (give(k * DELIVER_ROWS, rows_of(k))) {
       GSJ_HIP(hipStreamSynchronize(c.stream));
       return true;

@@ -217,25 +217,42 @@ __global__ void k_ewkb_coords(const uint8_t* __restrict__ buf, const RingRec* __
   const double ox = ld64(p, little), oy = ld64(p + 8, little);
   double sum = 0.0, comp = 0.0;
   double ax = ld64(p + stride, little) - ox, ay = ld64(p + stride + 8, little) - oy;
-  for (uint32_t i = 1; i + 2 < R.np; i++) {
-    const uint8_t* q = p + (uint64_t)(i + 1) * stride;
-    const double bx = ld64(q, little) - ox, by = ld64(q + 8, little) - oy;
-    const double pp = ax * by, qq = ay * bx;
-    const double terms[4] = {pp, -qq, fma(ax, by, -pp), -fma(ay, bx, -qq)};
-    for (int t = 0; t < 4; t++) {
-      const double v = terms[t], s = sum + v;
-      comp += fabs(sum) >= fabs(v) ? (sum - s) + v : (v - s) + sum;
-      sum = s;
+  constexpr int AHEAD = 16;   // points loaded ahead of the serial sum: a batch of loads takes longer than its terms
+  for (uint32_t i0 = 1; i0 + 2 < R.np; i0 += AHEAD) {
+    double2 b[AHEAD];
+#pragma unroll
+    for (int j = 0; j < AHEAD; j++) {
+      const uint8_t* q = p + (uint64_t)min(i0 + 1 + j, R.np - 1) * stride;
+      b[j] = make_double2(ld64(q, little), ld64(q + 8, little));
     }
-    ax = bx;
-    ay = by;
+#pragma unroll
+    for (int j = 0; j < AHEAD; j++) {
+      if (i0 + j + 2 >= R.np) break;
+      const double bx = b[j].x - ox, by = b[j].y - oy;
+      const double pp = ax * by, qq = ay * bx;
+      const double terms[4] = {pp, -qq, fma(ax, by, -pp), -fma(ay, bx, -qq)};
+      for (int t = 0; t < 4; t++) {
+        const double v = terms[t], s = sum + v;
+        comp += fabs(sum) >= fabs(v) ? (sum - s) + v : (v - s) + sum;
+        sum = s;
+      }
+      ax = bx;
+      ay = by;
+    }
   }
   const bool ccw = sum + comp > 0;
   const bool flip = ccw != (R.shell != 0);
   double2* out = xy + R.dst;
-  for (uint32_t i = 0; i < R.np; i++) {
-    const uint8_t* q = p + (uint64_t)i * stride;
-    out[flip ? R.np - 1 - i : i] = make_double2(ld64(q, little), ld64(q + 8, little));
+  for (uint32_t i0 = 0; i0 < R.np; i0 += AHEAD) {
+    double2 b[AHEAD];
+#pragma unroll
+    for (int j = 0; j < AHEAD; j++) {
+      const uint8_t* q = p + (uint64_t)min(i0 + j, R.np - 1) * stride;
+      b[j] = make_double2(ld64(q, little), ld64(q + 8, little));
+    }
+#pragma unroll
+    for (int j = 0; j < AHEAD; j++)
+      if (i0 + j < R.np) out[flip ? R.np - 1 - (i0 + j) : i0 + j] = b[j];
   }
 }
 

@@ -3,7 +3,7 @@
 //
 // Stackless: nodes are in depth-first preorder, so a lane walks forward through the node array, descending into
 // the next node on overlap and jumping to the node's skip link otherwise. No per-lane stack (which would live in
-// scratch memory on CDNA), one 16-byte + one 8-byte load per visited node, monotonically increasing addresses.
+// scratch memory on CDNA), one 16-byte + one 8-byte load per visited node, sent together, monotonically increasing addresses.
 // One walk per probe in the common case: it counts the probe's candidates and keeps the first SLOT_K of them in the
 // probe's slots; after the scan, a gather writes them at their offsets (SoA pair buffers), and only the probes with
 // more candidates than slots walk again, writing at their offsets.
@@ -30,27 +30,27 @@ __global__ void __launch_bounds__(256) k_traverse(const float4* __restrict__ qbb
   uint64_t o = WRITE ? offs[t] : 0;
   uint32_t cnt = 0;
   uint32_t i = 0;
-  // every step moves strictly forward (left child = i + 1, skip > i), so the walk ends within nnodes steps
+  // every step moves strictly forward (left child = i + 1, skip > i), so the walk ends within nnodes steps. The walk is a
+  // chain of loads, one wait per node: the box and both links go out together, and the box test reads all four sides
+  // (with || and the leaf's link read behind it, the compiler fetched the first side alone, then the others, then the
+  // link: three waits; 3M points 343 -> 254 us, 1M boxes 502 -> 292, 400k 233 -> 128, 50k 66 -> 52). The next one or three
+  // nodes in preorder fetched as well took longer (3M points 317, 388 us): then the reads of lanes that part ways bound it.
   while (i < nnodes) {
-    const float4 c = nodes[i].box;
-    const bool ov = !(c.x > b.z || c.z < b.x || c.y > b.w || c.w < b.y);
-    const uint32_t skip = (uint32_t)nodes[i].skip;
-    uint32_t next;
-    if (!ov) next = skip;
-    else {
-      const int32_t prim = nodes[i].prim;
+    const uint4* nd = reinterpret_cast<const uint4*>(nodes + i);
+    const float4 c = *reinterpret_cast<const float4*>(nd);
+    const uint4 link = nd[1];   // skip, prim, padding
+    const bool ov = !((int)(c.x > b.z) | (int)(c.z < b.x) | (int)(c.y > b.w) | (int)(c.w < b.y));
+    uint32_t next = link.x;
+    if (ov) {
+      const int32_t prim = (int32_t)link.y;
       if (prim < 0) next = i + 1;
-      else {
-        if (!upper || (uint32_t)prim >= q) {
-          if (WRITE) { out_a[o + cnt] = q; out_b[o + cnt] = (uint32_t)prim; }
-          else if (cnt < SLOT_K) slots[(uint64_t)t * SLOT_K + cnt] = (uint32_t)prim;
-          cnt++;
-        }
-        next = skip;
+      else if (!upper || (uint32_t)prim >= q) {
+        if (WRITE) { out_a[o + cnt] = q; out_b[o + cnt] = (uint32_t)prim; }
+        else if (cnt < SLOT_K) slots[(uint64_t)t * SLOT_K + cnt] = (uint32_t)prim;
+        cnt++;
       }
     }
-    if (next <= i) break;
-    i = next;
+    i = next > i ? next : nnodes;
   }
   if (!WRITE) {
     counts[t] = cnt;

@@ -12,7 +12,8 @@
 // reference reports NaN). Piece pairs fold to unique parent pairs with the minimum distance.
 //
 // Work classes as in the refinement: small pairs (both pieces <= 32 stored vertices) on 16-lane groups with 32-edge
-// LDS lists, larger pairs on a wave with 128-edge lists, overflowing pairs on a wave with lists in global memory.
+// LDS lists, larger pairs on a wave with 128-edge lists, overflowing pairs on a wave with lists of up to 448 edges in
+// LDS, and in global memory beyond. Geography distances are queued by the pair kernels and run in full waves.
 // All transcendental math is the portable set of gmath.h, so every threshold decision and distance has the bits of
 // the CPU restatement.
 #include "pairs.h"

@@ -228,11 +228,14 @@ Probes probes_of(const Layer& L, const float4* qbb = nullptr);
 // the device and the stream synchronised. Adds traverse_ms, batches and candidates to s; polls o.cancel.
 // on_members(list, n, mstart), when given, runs once before the walk with the probes that will be walked (list ==
 // nullptr: all n probes in id order) and may return the search boxes to use instead of pr.qbb (indexed by probe id;
-// by member position in for_each_candidate_multi, whose mstart gives the windows' member boundaries).
+// by member position in for_each_candidate_multi, whose mstart gives the windows' member boundaries). *long_runs, when
+// given, is set before every fn: whether the probe batch holds a probe of more than SLOT_K candidates (the search has
+// counted them, so it costs nothing to know).
+constexpr uint32_t SLOT_K = 16;   // candidates kept per probe by the counting walk
 using PairsFn = std::function<void(uint32_t* pa, uint32_t* pb, uint64_t np)>;
 using MembersFn = std::function<const float4*(const uint32_t* list, uint32_t n, const uint64_t* mstart)>;
 void for_each_candidate_batch(Context& c, const Probes& pr, const DBvh& t, bool upper, const gsj_join_opts& o, gsj_join_stats& s,
-                              const PairsFn& fn, const MembersFn& on_members = nullptr);
+                              const PairsFn& fn, const MembersFn& on_members = nullptr, bool* long_runs = nullptr);
 
 // Several windowed requests over the same probes in one candidate search (the batched served path). Window r's
 // members come after window r-1's, each in walk order, so request r's candidates are a contiguous run of every
@@ -247,6 +250,7 @@ struct SegBounds {
   uint32_t k = 0;
   const uint64_t* h = nullptr;   // host, k + 1 entries
   const uint64_t* d = nullptr;   // device copy
+  bool long_runs = false;        // see for_each_candidate_batch
 };
 using SegPairsFn = std::function<void(uint32_t* pa, uint32_t* pb, uint64_t np, const SegBounds& sb)>;
 bool probes_batchable(const Probes& pr);

@@ -115,8 +115,10 @@ __global__ void k_pip_emit(const DPolys R, const uint32_t* __restrict__ pa, cons
 // point's candidates are a run, so its rows are counted, the counts scanned in point order, and every run writes its
 // own: two passes over the candidates and a scan instead of a 64-bit sort of the rows (1.76M candidates of 3M points:
 // 813 -> 231 us, half of it the scattered rows). RUN_MAX: a run is searched once per parent, so a batch with a longer one
-// (counted in *over) keeps the sort.
-constexpr int RUN_MAX = 16;
+// keeps the sort. RUN_MAX is the search's slot count, so that the search itself tells (its long_runs) before either way
+// is begun (3M points in 20 layers of parcels on top of each other, 70M candidates: 68 ms a call; counted first, then
+// sorted, 175).
+constexpr int RUN_MAX = SLOT_K;
 // calls row(parent, where) for the distinct parents of the run's hits, ascending
 template <class Row>
 __device__ __forceinline__ void run_rows(const DPolys& R, const uint32_t* pb, const uint8_t* hit, uint64_t i, uint64_t e, const Row& row) {
@@ -136,23 +138,20 @@ __device__ __forceinline__ void run_rows(const DPolys& R, const uint32_t* pb, co
     last = next;
   }
 }
-// end of the run of candidates that starts at i (at most RUN_MAX; the rest is then left out), or i when one is under way
-__device__ __forceinline__ uint64_t run_end(const uint32_t* pa, uint64_t i, uint64_t np, bool& longer) {
+// end of the run of candidates that starts at i (at most RUN_MAX), or i when one is under way
+__device__ __forceinline__ uint64_t run_end(const uint32_t* pa, uint64_t i, uint64_t np) {
   const uint32_t q = pa[i];
   if (i > 0 && pa[i - 1] == q) return i;
   uint64_t e = i + 1;
   while (e < np && e < i + RUN_MAX && pa[e] == q) e++;
-  longer = e < np && e == i + RUN_MAX && pa[e] == q;
   return e;
 }
 __global__ void k_pip_count(const DPolys R, const uint32_t* __restrict__ pa, const uint32_t* __restrict__ pb, const uint8_t* __restrict__ hit, uint64_t np,
-                            uint32_t* __restrict__ cnt, uint32_t* __restrict__ over) {
+                            uint32_t* __restrict__ cnt) {
   const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= np) return;
-  bool longer = false;
-  const uint64_t e = run_end(pa, i, np, longer);
+  const uint64_t e = run_end(pa, i, np);
   if (e == i) return;
-  if (longer) atomicAdd(over, 1u);
   uint32_t n = 0;
   run_rows(R, pb, hit, i, e, [&](uint32_t, uint8_t) { n++; });
   cnt[pa[i]] = n;
@@ -161,8 +160,7 @@ __global__ void k_pip_rows(const DPolys R, const uint32_t* __restrict__ pa, cons
                            const uint64_t* __restrict__ off, uint32_t* __restrict__ orow, uint8_t* __restrict__ owhere) {
   const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= np) return;
-  bool longer = false;
-  const uint64_t e = run_end(pa, i, np, longer);
+  const uint64_t e = run_end(pa, i, np);
   if (e == i) return;
   const uint32_t q = pa[i];
   uint64_t o = off[q];
@@ -272,6 +270,7 @@ void points_join_run(Context& c, const Layer& PL, const Layer& RL, const gsj_joi
   gsj_join_stats s{};
   if (PL.n == 0 || RL.n == 0) { if (st) *st = s; return; }
   hipStream_t stream = c.stream;
+  bool long_runs = false;
   for_each_candidate_batch(c, probes_of(PL), RL.bvh, false, o, s, [&](uint32_t* pa, uint32_t* pb, uint64_t np) {
       WallTimer t2;
       uint8_t* hit = c.s_flag.as<uint8_t>(np + 16);
@@ -284,9 +283,9 @@ void points_join_run(Context& c, const Layer& PL, const Layer& RL, const gsj_joi
       uint64_t* hoffs = c.s_offs.as<uint64_t>(np + 16);
       uint32_t* orow = c.s_out_a.as<uint32_t>(2 * np + 16);
       uint8_t* owhere = c.s_out_flag.as<uint8_t>(np + 16);
-      const HostWords w = host_words(c, 0, 2);
+      const HostWords w = host_words(c, 0, 1);
       uint64_t nrows = 0;
-      bool sort = RL.poly.parent && !points_counted(PL.n, np);
+      const bool count = RL.poly.parent && !long_runs && points_counted(PL.n, np);
       if (!RL.poly.parent) {
         scan_loaded<uint64_t>(c, LoadAny{hit}, hoffs, np, ScanTotal{w.dev});
         hipLaunchKernelGGL(k_pip_emit, dim3(div_up(np, 256)), dim3(256), 0, stream, RL.poly, pa, pb, hit, hoffs, np, orow, owhere, nullptr, nullptr);
@@ -294,28 +293,24 @@ void points_join_run(Context& c, const Layer& PL, const Layer& RL, const gsj_joi
         w.fetch(c);
         GSJ_HIP(hipStreamSynchronize(stream));
         nrows = w.host[0];
-      } else if (!sort) {
-        uint32_t* cnt = c.s_seg.as<uint32_t>(PL.n + 17);
-        uint32_t* over = cnt + PL.n;
+      } else if (count) {
+        uint32_t* cnt = c.s_seg.as<uint32_t>(PL.n + 16);
         uint64_t* off = c.s_tmp2.as<uint64_t>(PL.n + 16);
-        hipLaunchKernelGGL(k_fill_zero, dim3(div_up(PL.n + 1, 256)), dim3(256), 0, stream, cnt, PL.n + 1);
+        hipLaunchKernelGGL(k_fill_zero, dim3(div_up(PL.n, 256)), dim3(256), 0, stream, cnt, PL.n);
         GSJ_LAUNCHED();
-        hipLaunchKernelGGL(k_pip_count, dim3(div_up(np, 256)), dim3(256), 0, stream, RL.poly, pa, pb, hit, np, cnt, over);
+        hipLaunchKernelGGL(k_pip_count, dim3(div_up(np, 256)), dim3(256), 0, stream, RL.poly, pa, pb, hit, np, cnt);
         GSJ_LAUNCHED();
-        scan_loaded<uint64_t>(c, LoadArray<uint32_t>{cnt}, off, PL.n, ScanTotal{w.dev, over});
+        scan_loaded<uint64_t>(c, LoadArray<uint32_t>{cnt}, off, PL.n, ScanTotal{w.dev});
         hipLaunchKernelGGL(k_pip_rows, dim3(div_up(np, 256)), dim3(256), 0, stream, RL.poly, pa, pb, hit, np, off, orow, owhere);
         GSJ_LAUNCHED();
         w.fetch(c);
         GSJ_HIP(hipStreamSynchronize(stream));
         nrows = w.host[0];
-        sort = w.host[1] != 0;
-      }
-      if (sort) {
+      } else {
         scan_loaded<uint64_t>(c, LoadAny{hit}, hoffs, np, ScanTotal{w.dev});
         w.fetch(c);
         GSJ_HIP(hipStreamSynchronize(stream));
         const uint64_t nh = w.host[0];
-        nrows = 0;
         if (nh) {
           uint64_t* keys = c.s_keys.as<uint64_t>(nh);
           uint64_t* keys2 = c.s_keys2.as<uint64_t>(nh);
@@ -346,7 +341,7 @@ void points_join_run(Context& c, const Layer& PL, const Layer& RL, const gsj_joi
       const RowPart parts[2] = {{orow, hrow, 8}, {owhere, hw, 1}};
       const bool stop = deliver_rows(c, parts, 2, nrows, s.copy_ms, [&](uint64_t r, uint64_t n) { return cb ? cb(user, hrow + 2 * r, hw + r, (size_t)n) : 0; });
       if (stop) throw Error(GSJ_E_CANCEL, "points join cancelled by the row callback");
-  });
+  }, nullptr, &long_runs);
   if (st) *st = s;
 }
 

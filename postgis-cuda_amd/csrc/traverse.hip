@@ -13,8 +13,6 @@ namespace gsj {
 
 namespace {
 
-constexpr uint32_t SLOT_K = 16;   // candidates kept per probe by the counting walk
-
 // WRITE false: count the probe's candidates into counts[t] and keep the first SLOT_K in slots[t * SLOT_K ..]
 // (probes with more are counted in *nover); WRITE true: the probes with counts[t] > SLOT_K write all theirs at offs[t]
 template <bool WRITE>
@@ -330,6 +328,7 @@ void walk_batches(Context& c, const Probes& pr, const DBvh& t, bool upper, const
       traverse_write(c, qbb, qidx, q0 + s0, s1 - s0, t, upper, counts + s0, offs, slots + (uint64_t)s0 * SLOT_K, any_over, pa, pb, box_by_pos);
       GSJ_HIP(hipEventRecord(c.ev[15], stream));
       SegBounds sb;
+      sb.long_runs = any_over;
       if (mstart) {
         hipLaunchKernelGGL(k_seg_bounds, dim3(1), dim3(64), 0, stream, mstart, k, (uint64_t)(q0 + s0), (uint64_t)(s1 - s0), offs, np, dlo);
         GSJ_LAUNCHED();
@@ -355,7 +354,7 @@ void walk_batches(Context& c, const Probes& pr, const DBvh& t, bool upper, const
 bool probes_batchable(const Probes& pr) { return pr.order && pr.tiles && !pr.h_parent; }
 
 void for_each_candidate_batch(Context& c, const Probes& pr, const DBvh& t, bool upper, const gsj_join_opts& o, gsj_join_stats& s,
-                              const PairsFn& fn, const MembersFn& on_members) {
+                              const PairsFn& fn, const MembersFn& on_members, bool* long_runs) {
   hipStream_t stream = c.stream;
   // probe positions 0 .. nQ: probe ids directly, through the walk order, or through the window's member list (in walk
   // order); a subdivided layer walks in id order (its parents' pieces are contiguous)
@@ -404,7 +403,10 @@ void for_each_candidate_batch(Context& c, const Probes& pr, const DBvh& t, bool 
     if (b) qbb = b;
   }
   walk_batches(c, pr, t, upper, o, s, qidx, nQ, hq, nullptr, 0, qbb, false,
-               [&](uint32_t* pa, uint32_t* pb, uint64_t np, const SegBounds&) { fn(pa, pb, np); });
+               [&](uint32_t* pa, uint32_t* pb, uint64_t np, const SegBounds& sb) {
+                 if (long_runs) *long_runs = sb.long_runs;
+                 fn(pa, pb, np);
+               });
 }
 
 void for_each_candidate_multi(Context& c, const Probes& pr, const DBvh& t, bool upper, const gsj_join_opts& o, const WindowSet& ws,

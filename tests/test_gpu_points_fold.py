@@ -1,5 +1,7 @@
 """Rows of points in subdivided layers: counted per point where the batch covers the points, sorted where it covers few of
 them or a point meets more pieces than a run holds. Against the oracle to the bit, in the oracle's order of keys."""
+import json
+
 import numpy as np
 import pytest
 
@@ -57,9 +59,29 @@ def test_points_mostly_elsewhere(ctx, far):
     _check(ctx, np.concatenate([out[: far // 2], xy, out[far // 2 :]]), gsj.subdivide(M, 8))
 
 
-# 1 to 40 layers on top of each other: up to, at and beyond the length of a run
+# 1 to 40 layers on top of each other: up to, at and beyond the length of a run (16 candidates)
 @pytest.mark.parametrize("k", [1, 4, 8, 15, 16, 17, 40])
 def test_points_in_stacked_pieces(ctx, k):
     M = _mesh(6, 9)
     got, _ = _check(ctx, _points(M, 3000, k), gsj.subdivide(_stack(M, k), 8))
     assert (np.diff(got.pairs[:, 0].astype(np.int64)) >= 0).all()
+
+
+def test_stacked_pieces_take_one_way(ctx):
+    # one point with more pieces than a run holds sends its batch to the sort; the counters and offsets that the other way
+    # keeps for every point of the layer (12 bytes each) are then not set up at all, let alone run through
+    M, n = _mesh(6, 9), 4 << 20
+    S, near = gsj.subdivide(_stack(M, 17), 8), _points(M, 300, 2)
+    xy = np.concatenate([np.random.default_rng(1).random((n, 2)) + [5.0, 0.0], near])
+    own = gsj.Context(0)
+    try:
+        pts, plain, stacked = own.points(xy), own.polys(M), own.polys(S)
+        own.points_in_polygons(pts, plain)   # the search's buffers; no subdivided layer, no fold
+        free = json.loads(own.status())["mem_free_mb"]
+        got = own.points_in_polygons(pts, stacked)
+        assert (free - json.loads(own.status())["mem_free_mb"]) * 2**20 < 12 * n
+        exp = O.points_join(O.Layer.points_layer(near), O.Layer.polys(S))
+        g, e = sorted_rows(got.pairs, got.where), sorted_rows(exp["pairs"] + np.array([n, 0], np.uint32), exp["where"])
+        assert len(e[0]) and np.array_equal(g[0], e[0]) and np.array_equal(g[1], e[1])
+    finally:
+        own.close()

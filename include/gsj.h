@@ -118,7 +118,11 @@ typedef struct {
 } gsj_join_opts;
 
 typedef struct {
-  double traverse_ms, refine_ms, compact_ms, copy_ms;   /* JoinStats, engine/engine.cuh:814 */
+  /* JoinStats, engine/engine.cuh:814: host times of a call's phases. Where the refinement and the compaction are waited
+   * for together (point joins, polygon joins of few candidates), refine_ms is the device's time for the refinement and
+   * compact_ms the rest up to the rows. Rows written straight into host memory count in compact_ms; copy_ms is the time
+   * spent sending and waiting for rows copied afterwards, not the callbacks' own. */
+  double traverse_ms, refine_ms, compact_ms, copy_ms;
   uint64_t candidates;     /* candidate pairs (refined pairs) */
   uint64_t hits;           /* result rows delivered (parent pairs) */
   uint64_t heavy;          /* pairs whose local edge lists exceeded on-chip capacity */

@@ -170,6 +170,14 @@ void radix_sort_pairs(Context& c, uint64_t*& keys, uint64_t*& keys_alt, uint32_t
 // OR and AND of all keys (for choosing digits); synchronises
 void key_bits(Context& c, const uint64_t* keys, uint64_t n, uint64_t& or_all, uint64_t& and_all);
 
+// A sub-batch whose refinement and compaction are enqueued together and waited for once took `wall` ms: the refinement's
+// share is the device's time for it, or the time of its launches where that is longer
+inline void split_wait(gsj_join_stats& s, double wall, double launch_ms, double device_ms) {
+  const double refine = std::min(wall, std::max(launch_ms, device_ms));
+  s.refine_ms += refine;
+  s.compact_ms += wall - refine;
+}
+
 // Rows from device memory to the callback, DELIVER_ROWS at a time: a chunk is copied while the callback works on the one
 // before it (3M points in parcels, 24 MB of rows: 2277 -> 1975 us a call, of a 1M self-join 9.85 -> 9.5 ms). Chunks of 512k
 // rows are within 1-4% of it, of 64k slower (2462 us: each costs two copies, an event and a wait). parts: the arrays of a
@@ -285,13 +293,14 @@ uint64_t refine_pairs(Context& c, const DPolys& P, const DPolys& R, const uint32
 // The same for at most STAGED_MAX pairs without a host wait (see refine.hip): refine_stages enqueues the classes, the
 // overflow pass and a report; after the caller's own wait, refine_stages_finish adds to the statistics and refines the
 // pairs left over (lists too long for LDS), returning whether there were any: what the caller computed from the outputs
-// has to be redone then (n_over: pairs that took an overflow pass). refine_staged: whether a launch of np pairs takes this way.
+// has to be redone then (n_over: pairs that took an overflow pass; span_ms: the device's time from the partition to the
+// report). refine_staged: whether a launch of np pairs takes this way.
 constexpr uint64_t STAGED_MAX = 32768;
 bool refine_staged(const Context& c, uint64_t np);
 void refine_stages(Context& c, const DPolys& P, const DPolys& R, const uint32_t* pa, const uint32_t* pb, uint64_t np, const RefineParams& rp,
                    const RefineOut& out);
 bool refine_stages_finish(Context& c, const DPolys& P, const DPolys& R, const uint32_t* pa, const uint32_t* pb, uint64_t np, const RefineParams& rp,
-                          const RefineOut& out, gsj_join_stats& s, uint64_t& n_over);
+                          const RefineOut& out, gsj_join_stats& s, uint64_t& n_over, double& span_ms);
 
 // ------------------------------------------------------------------------------------------- join driver
 struct JoinHooks {

@@ -396,13 +396,14 @@ void join_run(Context& c, const Layer& PL, const Layer& RL, const gsj_join_opts&
     ro.evb = rp.want_relate ? c.s_evb.as<uint32_t>(np + 16) : nullptr;
     rp.done = hooks && hooks->decide ? hooks->decide(pa, pb, np, ro) : nullptr;
     // no host waits between refinement, compaction and the row copy beyond the ones that read sizes back: the
-    // stream orders the work (refine_ms and compact_ms are host times up to those reads)
+    // stream orders the work (refine_ms and compact_ms are host times up to those reads; split_wait where there is one)
     const bool folds = !o.no_agg && (PL.poly.pfirst || RL.poly.pfirst);
     const bool direct = !hooks && np <= DIRECT_ROWS && (!c.dev_arena || !folds);
     const bool staged = direct && refine_staged(c, np);   // then nothing is read back before the rows are there
     if (staged) refine_stages(c, PL.poly, RL.poly, pa, pb, np, rp, ro);
     else s.heavy += refine_pairs(c, PL.poly, RL.poly, pa, pb, np, rp, ro, &s);
-    s.refine_ms += t2.ms();
+    const double launch_ms = t2.ms();
+    if (!staged) s.refine_ms += launch_ms;
     WallTimer t3;
     if (direct) {
       uint32_t* hrow = c.h_pairs.as<uint32_t>(2 * np);
@@ -426,12 +427,20 @@ void join_run(Context& c, const Layer& PL, const Layer& RL, const gsj_join_opts&
       };
       Compaction k = rows();
       uint64_t n_over = 0;
-      if (staged && refine_stages_finish(c, PL.poly, RL.poly, pa, pb, np, rp, ro, s, n_over)) k = rows();   // the pairs refined since change the rows
+      double span_ms = 0;
+      if (staged) {
+        WallTimer tf;
+        if (refine_stages_finish(c, PL.poly, RL.poly, pa, pb, np, rp, ro, s, n_over, span_ms)) {
+          span_ms += tf.ms();
+          k = rows();   // the pairs refined since change the rows
+        }
+      }
       s.heavy += n_over;
       const bool late = k.host_folds();
       nrows = compact_finish(c, k);
       if (late) GSJ_HIP(hipStreamSynchronize(stream));   // the rows folded after the wait
-      s.compact_ms += t3.ms();
+      if (staged) split_wait(s, t2.ms(), launch_ms, span_ms);
+      else s.compact_ms += t3.ms();
       s.hits += nrows;
       if (nrows && cb && cb(user, hrow, harea, hcode, (size_t)nrows)) throw Error(GSJ_E_CANCEL, "join cancelled by the row callback");
       return;

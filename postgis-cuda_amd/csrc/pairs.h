@@ -309,7 +309,7 @@ struct PairClasses {
   uint32_t* list;
   uint32_t* counts;
   OverflowCtl* ctl;
-  uint64_t* start;   // words for launches' start times
+  uint64_t* start;   // [0] the partition's start time (wall_clock64); the words behind it are for the launches that follow
 };
 // size_sort: within a class, pairs of similar size side by side, in buckets 2^(size_sort-1) times the class's base
 // width (0: candidate order, a probe's pairs together); done (or null): the candidates whose byte is set are in no class

@@ -278,8 +278,7 @@ void points_join_run(Context& c, const Layer& PL, const Layer& RL, const gsj_joi
       hipLaunchKernelGGL(k_pip, dim3(div_up(np, 256)), dim3(256), 0, stream, PL.pts, RL.poly, pa, pb, np, hit);
       GSJ_LAUNCHED();
       GSJ_HIP(hipEventRecord(c.ev[1], stream));
-      s.refine_ms += t2.ms();
-      WallTimer t3;
+      const double launch_ms = t2.ms();
       uint64_t* hoffs = c.s_offs.as<uint64_t>(np + 16);
       uint32_t* orow = c.s_out_a.as<uint32_t>(2 * np + 16);
       uint8_t* owhere = c.s_out_flag.as<uint8_t>(np + 16);
@@ -333,7 +332,7 @@ void points_join_run(Context& c, const Layer& PL, const Layer& RL, const gsj_joi
       s.k_small_ms += ms;
       s.n_small += np;
       s.launches++;
-      s.compact_ms += t3.ms();
+      split_wait(s, t2.ms(), launch_ms, ms);
       s.hits += nrows;
       if (!nrows) return;
       uint32_t* hrow = c.h_pairs.as<uint32_t>(2 * nrows);

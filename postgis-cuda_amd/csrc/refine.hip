@@ -402,7 +402,7 @@ constexpr uint8_t ST_HIT = 1, ST_RTOUCH = 2, ST_INA = 4, ST_INB = 8;
 struct StageReport {
   uint32_t counts[16];
   OverflowCtl ctl[2];   // the overflow queue's, the host's queue's
-  uint64_t start[4];    // wall_clock64 at the screens, the edges, the overflow pass and the report
+  uint64_t start[5];    // wall_clock64 at the partition, the screens, the edges, the overflow pass and the report
 };
 HostWords stage_words(Context& c) { return host_words(c, 32, sizeof(StageReport) / 8); }
 
@@ -1040,7 +1040,7 @@ struct StageArgs {
   RefineOut out;
   EdgeQueue q;
   int cap_large;
-  uint64_t* start;   // start times of the stages (wall_clock64)
+  uint64_t* start;   // start times of the partition and the stages (wall_clock64)
 };
 
 // first item of this block's group gib (of gpb) among a class's n items, when the classes before it took `used` blocks
@@ -1052,7 +1052,7 @@ __device__ __forceinline__ uint32_t stage_first(uint32_t& used, uint32_t n, uint
 
 __global__ void __launch_bounds__(64, 3) k_stage_screens(const StageArgs A) {
   extern __shared__ __align__(16) unsigned char smem[];
-  if (blockIdx.x == 0 && threadIdx.x == 0) A.start[0] = wall_clock64();
+  if (blockIdx.x == 0 && threadIdx.x == 0) A.start[1] = wall_clock64();
   const bool rel = A.rp.want_relate != 0;
   const uint32_t* n = A.counts;
   uint32_t used = 0;
@@ -1085,7 +1085,7 @@ __global__ void __launch_bounds__(64, 3) k_stage_screens(const StageArgs A) {
 
 __global__ void __launch_bounds__(64, 3) k_stage_edges(const StageArgs A) {
   extern __shared__ __align__(16) unsigned char smem[];
-  if (blockIdx.x == 0 && threadIdx.x == 0) A.start[1] = wall_clock64();
+  if (blockIdx.x == 0 && threadIdx.x == 0) A.start[2] = wall_clock64();
   const bool rel = A.rp.want_relate != 0;
   const uint32_t* n = A.counts;
   uint32_t used = 0;
@@ -1109,12 +1109,12 @@ __global__ void __launch_bounds__(64, 3) k_stage_edges(const StageArgs A) {
 }
 
 // class sizes, edge queue sizes, queue controls and stage start times into the host's words
-__global__ void k_stage_report(const uint32_t* __restrict__ counts, const OverflowCtl* __restrict__ ctl, uint64_t* start, StageReport* __restrict__ out) {
+__global__ void k_stage_report(const uint32_t* __restrict__ counts, const OverflowCtl* __restrict__ ctl, const uint64_t* __restrict__ start, StageReport* __restrict__ out) {
   const int t = threadIdx.x;
-  if (t == 0) { start[3] = wall_clock64(); out->start[3] = start[3]; }
+  if (t == 0) out->start[4] = wall_clock64();
   if (t < 16) out->counts[t] = counts[t];
   if (t < 2) out->ctl[t] = ctl[t];
-  if (t < 3) out->start[t] = start[t];
+  if (t < 4) out->start[t] = start[t];
 }
 
 // LDS of the two stages' single-wave blocks
@@ -1158,7 +1158,7 @@ void refine_stages(Context& c, const DPolys& P, const DPolys& R, const uint32_t*
   GSJ_LAUNCHED();
   // few pairs, eight waves each (see the host-sized launch below); longer lists go on to the host's queue
   hipLaunchKernelGGL((k_refine_overflow<512, true>), dim3((uint32_t)std::min<uint64_t>(np, cu)), dim3(512), list_bytes(OVF_LDS_CAP, rel), st, P, R, pa, pb,
-                     A.ovf, 0u, rp, out, (int)OVF_LDS_CAP, nullptr, A.ctl, ovf_main, A.ctl + 1, A.start + 2);
+                     A.ovf, 0u, rp, out, (int)OVF_LDS_CAP, nullptr, A.ctl, ovf_main, A.ctl + 1, A.start + 3);
   GSJ_LAUNCHED();
   const HostWords w = stage_words(c);
   hipLaunchKernelGGL(k_stage_report, dim3(1), dim3(64), 0, st, pc.counts, pc.ctl, A.start, reinterpret_cast<StageReport*>(w.dev));
@@ -1167,12 +1167,13 @@ void refine_stages(Context& c, const DPolys& P, const DPolys& R, const uint32_t*
 }
 
 bool refine_stages_finish(Context& c, const DPolys& P, const DPolys& R, const uint32_t* pa, const uint32_t* pb, uint64_t np, const RefineParams& rp,
-                          const RefineOut& out, gsj_join_stats& s, uint64_t& n_over) {
+                          const RefineOut& out, gsj_join_stats& s, uint64_t& n_over, double& span_ms) {
   const StageReport r = *reinterpret_cast<const StageReport*>(stage_words(c).host);
   const uint32_t handed = r.ctl[1].count;   // pairs whose lists exceed OVF_LDS_CAP
   n_over = r.ctl[0].count;                  // (they are counted in it too)
   auto ms = [&](int k) { return (double)(r.start[k + 1] - r.start[k]) / c.clock_khz; };
-  const double m0 = ms(0), m1 = ms(1), m2 = ms(2);
+  const double m0 = ms(1), m1 = ms(2), m2 = ms(3);
+  span_ms = (double)(r.start[4] - r.start[0]) / c.clock_khz;
   s.n_tiny += r.counts[CL_TINY]; s.n_small += r.counts[CL_SMALL]; s.n_medium += r.counts[CL_MEDIUM]; s.n_mixed += r.counts[CL_MIXED];
   s.n_large += r.counts[CL_LARGE];
   s.n_tiny_edge += r.counts[8 + CL_TINY]; s.n_small_edge += r.counts[8 + CL_SMALL]; s.n_medium_edge += r.counts[8 + CL_MEDIUM];
@@ -1200,7 +1201,8 @@ uint64_t refine_pairs(Context& c, const DPolys& P, const DPolys& R, const uint32
     GSJ_HIP(hipStreamSynchronize(st));
     gsj_join_stats none{};
     uint64_t n_over = 0;
-    (void)refine_stages_finish(c, P, R, pa, pb, np, rp, out, stats ? *stats : none, n_over);
+    double span_ms = 0;
+    (void)refine_stages_finish(c, P, R, pa, pb, np, rp, out, stats ? *stats : none, n_over, span_ms);
     return n_over;
   }
   const bool rel = rp.want_relate != 0;
@@ -1362,12 +1364,13 @@ constexpr int PART_T = 1024, PART_MAX = 16384, PART_ITEMS = PART_MAX / PART_T;
 __global__ void __launch_bounds__(PART_T) k_partition_small(const DPolys P, const DPolys R, const uint32_t* __restrict__ pa, const uint32_t* __restrict__ pb,
                                                             const uint8_t* __restrict__ done, uint32_t np, uint32_t mcap, int mixed, uint32_t tcap,
                                                             uint32_t size_sort, uint32_t* __restrict__ list, uint32_t* __restrict__ counts,
-                                                            OverflowCtl* ctl) {
+                                                            OverflowCtl* ctl, uint64_t* start) {
   constexpr int NC = PART_T / 64 * 2, PARTS = PART_T / 256, CPP = NC / PARTS;   // counter columns; a thread scans CPP of a key's
   __shared__ uint32_t hist[NC][256];
   __shared__ uint32_t psum[PARTS][256];
   __shared__ uint32_t kfirst[256];
   __shared__ uint32_t wtot[4];
+  const uint64_t began = wall_clock64();
   const int t = threadIdx.x, lane = t & 63, w = t >> 6, col = 2 * w + (lane & 1);
   const uint32_t per = (np + PART_T - 1) / PART_T;             // rounds of 64 candidates per wave
   const uint32_t base = (uint32_t)w * per * 64 + (uint32_t)lane;
@@ -1394,6 +1397,7 @@ __global__ void __launch_bounds__(PART_T) k_partition_small(const DPolys P, cons
   }
   for (int k = t; k < NC * 256; k += PART_T) (&hist[0][0])[k] = 0;
   if (t < 5) ctl[t] = OverflowCtl{0, 0, 0, 0};
+  if (t == 0) *start = began;
   __syncthreads();
 #pragma unroll
   for (int j = 0; j < PART_ITEMS; j++)
@@ -1444,11 +1448,12 @@ constexpr int TILE_T = 256, TILE_ITEMS = 16, TILE_PAIRS = TILE_T * TILE_ITEMS, T
 __global__ void __launch_bounds__(TILE_T) k_part_count(const DPolys P, const DPolys R, const uint32_t* __restrict__ pa, const uint32_t* __restrict__ pb,
                                                        const uint8_t* __restrict__ done, uint64_t np, uint32_t mcap, int mixed, uint32_t tcap,
                                                        uint32_t size_sort, uint8_t* __restrict__ keys, uint32_t ntiles, uint32_t* __restrict__ ghist,
-                                                       OverflowCtl* ctl) {
+                                                       OverflowCtl* ctl, uint64_t* start) {
   __shared__ uint32_t hist[TILE_COLS][256];
   const int t = threadIdx.x, col = (t >> 6) * 2 + (t & 1);
   const uint64_t base = (uint64_t)blockIdx.x * TILE_PAIRS;
   if (blockIdx.x == 0 && t < 5) ctl[t] = OverflowCtl{0, 0, 0, 0};
+  if (blockIdx.x == 0 && t == 0) *start = wall_clock64();
 #pragma unroll
   for (int c = 0; c < TILE_COLS; c++) hist[c][t] = 0;
   uint32_t a[TILE_ITEMS], b[TILE_ITEMS];
@@ -1529,7 +1534,7 @@ PairClasses partition_pairs(Context& c, const DPolys& P, const DPolys& R, const 
   pc.list = c.s_vals.as<uint32_t>(np + 16);
   if (np <= (uint64_t)PART_MAX) {
     hipLaunchKernelGGL(k_partition_small, dim3(1), dim3(PART_T), 0, st, P, R, pa, pb, done, (uint32_t)np, mcap, mixed ? 1 : 0, tcap, size_sort, pc.list,
-                       pc.counts, pc.ctl);
+                       pc.counts, pc.ctl, pc.start);
     GSJ_LAUNCHED();
     return pc;
   }
@@ -1537,7 +1542,7 @@ PairClasses partition_pairs(Context& c, const DPolys& P, const DPolys& R, const 
   uint8_t* keys = c.s_keys.as<uint8_t>(np + 16);
   uint32_t* ghist = c.s_tmp2.as<uint32_t>((uint64_t)256 * ntiles + 8);
   hipLaunchKernelGGL(k_part_count, dim3(ntiles), dim3(TILE_T), 0, st, P, R, pa, pb, done, np, mcap, mixed ? 1 : 0, tcap, size_sort, keys, ntiles, ghist,
-                     pc.ctl);
+                     pc.ctl, pc.start);
   GSJ_LAUNCHED();
   scan_loaded<uint32_t>(c, LoadArray<uint32_t>{ghist}, ghist, (uint64_t)256 * ntiles, ScanTotal{});
   hipLaunchKernelGGL(k_part_scatter, dim3(ntiles), dim3(TILE_T), 0, st, keys, np, ntiles, ghist, pc.list, pc.counts);

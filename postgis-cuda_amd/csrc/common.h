@@ -10,6 +10,7 @@
 #include <vector>
 #include <mutex>
 #include "../../include/gsj.h"
+#include "grid.h"
 
 namespace gsj {
 

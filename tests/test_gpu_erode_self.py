@@ -99,3 +99,20 @@ def test_a_mesh_of_every_size(ctx):
         exp = O.erode(OL, OL, ra, rb, same=True, upper=True)
         got = ctx.intersects_buffered(L, L, ra, rb, same=True, upper=True)
         assert np.array_equal(sorted_rows(got.pairs)[0], sorted_rows(exp["pairs"])[0])
+
+
+def test_more_pairs_than_one_round_of_blocks(ctx):
+    # 8200 boxes on one spot: 67.2M candidates, the last of them in the blocks' second round; every pair meets
+    n = 8200
+    box = _box(0, 0, 30, 20)
+    hs = gsj.HostSet(np.arange(n + 1, dtype=np.uint64), 5 * np.arange(n + 1, dtype=np.uint64), np.tile(box, (n, 1)))
+    own = gsj.Context(0)   # (its scratch goes with it)
+    try:
+        L = own.polys(hs)
+        got = own.intersects_buffered(L, L, 2.0, 1.0, same=True)
+        seen = np.zeros(n * n, bool)
+        seen[got.pairs[:, 0].astype(np.int64) * n + got.pairs[:, 1]] = True
+        assert got.stats["candidates"] == n * n == len(got.pairs) and seen.all()
+        assert len(own.intersects_buffered(L, L, 11.0, 1.0, same=True).pairs) == 0
+    finally:
+        own.close()

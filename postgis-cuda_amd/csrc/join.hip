@@ -70,7 +70,7 @@ __global__ void k_emit_hits(const DPolys P, const DPolys R, const uint32_t* __re
 }
 
 // A folded candidate's place: parent pair, then piece pair. parent A | parent B | piece of A | piece of B within their
-// parents, in the bits that the layers need (their pieces are numbered parent by parent). Where those exceed 64, `wide`:
+// parents, in the bits that the layers need (their pieces are numbered parent by parent). Where those exceed 63, `wide`:
 // the piece pair first, and the parent pair as a second key (b = 32, la = lb = 0).
 struct FoldKey {
   int b, la, lb;   // bits of parent B, of a piece of A, of a piece of B
@@ -141,7 +141,7 @@ __global__ void __launch_bounds__(FOLD_T) k_fold_small(const DPolys P, const DPo
   uint32_t N = 64;
   while (N < m) N <<= 1;
   for (uint32_t j = t; j < N; j += FOLD_T) {
-    K[j] = j < m ? keys[j] : ~0ull;
+    K[j] = j < m ? keys[j] : ~0ull;   // above every key (FOLD_KEY_BITS)
     V[j] = j < m ? vals[j] : 0u;
   }
   __syncthreads();
@@ -246,7 +246,7 @@ inline int bits_for(uint64_t maxval) { int b = 1; while (b < 64 && (maxval >> b)
 
 namespace {
 
-constexpr int FOLD_KEY_BITS = 64;   // a fold key's bits (lower to send a test's layers the wide way)
+constexpr int FOLD_KEY_BITS = 63;   // a packed fold key's bits: 64 ones are the block sort's padding, which has to come last
 
 // Compaction of one sub-batch's refined candidates into parent-pair rows at (orow, oarea, ocode: device memory, or pinned
 // host memory that the kernels write directly). compact_enqueue asks for no host wait; after the caller's, the row

@@ -53,3 +53,35 @@ def test_one_parent_of_many_pieces(ctx):
 def test_clusters_of_pieces(ctx, n, maxv):
     S = gsj.subdivide(_mesh(n, 3 * n), maxv)
     assert np.array_equal(ctx.cluster(ctx.polys(S))[0], O.cluster(O.Layer.polys(S))["root"])
+
+
+def _bits(v):
+    return max(1, int(v).bit_length())
+
+
+def _key_bits(P, R):
+    """bits of a folded candidate's key: both parents, and both pieces within their parents"""
+    return sum(_bits(S.parent[-1]) + _bits(np.bincount(S.parent - S.parent[0]).max() - 1) for S in (P, R))
+
+
+def _cells(k, last):
+    """one parent, of id `last`, cut into k x k cells of unequal sizes; the cuts are synthetic edges"""
+    rng = np.random.default_rng(k)
+    x, y = (np.concatenate([[0.0], np.cumsum(0.5 + rng.random(k))]) * 1e-4 - o for o in (95.0, -38.0))
+    i, j = (a.ravel() for a in np.meshgrid(np.arange(k), np.arange(k), indexing="ij"))
+    x0, x1, y0, y1 = x[i], x[i + 1], y[j], y[j + 1]
+    xy = np.stack([np.stack([x0, x1, x1, x0, x0], 1), np.stack([y0, y0, y1, y1, y0], 1)], 2)
+    syn = np.stack([j > 0, i < k - 1, j < k - 1, i > 0, np.zeros(k * k, bool)], 1)
+    n = k * k
+    return gsj.HostSet(np.arange(n + 1, dtype=np.uint64), 5 * np.arange(n + 1, dtype=np.uint64), xy.reshape(-1, 2),
+                       np.full(n, last, np.uint32), syn.reshape(-1).astype(np.uint8))
+
+
+# the last piece of the last parent with itself, where both ids have all their bits set: its key is the largest there is,
+# 64 bits of ones at 2^24 parents and 256 pieces
+@pytest.mark.parametrize("bits", [23, 24, 25])
+@pytest.mark.parametrize("what", ["want_area", "want_relate"])
+def test_the_largest_key(ctx, bits, what):
+    S = _cells(16, 2**bits - 1)
+    assert _key_bits(S, S) == 2 * bits + 16
+    _check(ctx, S, S, True, what, (False, True))

@@ -14,6 +14,16 @@ def _mesh(n, seed, **kw):
     return gsj.generate("parcels_mesh", nx=n, ny=n, w=1 / 1549, h=1 / 1549, seed=seed, **kw)
 
 
+FOLD_MAX = 4096   # the most candidates that one block folds
+
+
+def _folded(ctx, P, R, upper):
+    """the candidates that go to the fold: piece pairs that meet, of a parent of several pieces on either side"""
+    pairs = ctx.join(ctx.polys(P), ctx.polys(R), upper=upper, want_area=True, no_agg=True).pairs
+    several = [np.zeros(S.n, bool) if S.parent is None else np.bincount(S.parent - S.parent[0])[S.parent - S.parent[0]] > 1 for S in (P, R)]
+    return int((several[0][pairs[:, 0]] | several[1][pairs[:, 1]]).sum())
+
+
 def _check(ctx, P, R, upper, what, entries=(False,)):
     LP, LR = ctx.polys(P), ctx.polys(R)
     exp = O.join(O.Layer.polys(P), O.Layer.polys(R), upper=upper, **{what: True})
@@ -25,11 +35,13 @@ def _check(ctx, P, R, upper, what, entries=(False,)):
     return got
 
 
-# from a handful of folded candidates to about a hundred thousand; 34 x 34 at 8 vertices lies around the block's 4096
-@pytest.mark.parametrize("n,maxv", [(4, 8), (12, 16), (20, 8), (34, 8), (36, 8), (40, 32), (90, 8)])
+# from a handful of folded candidates to about a hundred thousand; 17 to 20 cells a side at 8 vertices lie around the
+# block's 4096
+@pytest.mark.parametrize("n,maxv", [(4, 8), (12, 16), (17, 8), (18, 8), (20, 8), (34, 8), (36, 8), (40, 32), (90, 8)])
 @pytest.mark.parametrize("what", ["want_area", "want_relate"])
 def test_self_join_of_pieces(ctx, n, maxv, what):
     S = gsj.subdivide(_mesh(n, n), maxv)
+    assert (_folded(ctx, S, S, True) <= FOLD_MAX) == (n < 18 or maxv > 8)
     _check(ctx, S, S, True, what, (False, True) if n <= 40 else (False,))
 
 
@@ -85,3 +97,28 @@ def test_the_largest_key(ctx, bits, what):
     S = _cells(16, 2**bits - 1)
     assert _key_bits(S, S) == 2 * bits + 16
     _check(ctx, S, S, True, what, (False, True))
+
+
+def _renumbered(S, step):
+    """the pieces of S under parent ids `step` apart"""
+    return gsj.HostSet(S.gro, S.rvo, S.xy, S.parent * np.uint32(step), S.syn)
+
+
+# keys up to and beyond 63 bits (from 64 on the candidates are sorted twice, by piece pair and by parent pair), few and many
+# candidates: regions of hundreds of pieces under ids millions apart, with themselves and with parcels of a few pieces
+@pytest.mark.parametrize("k,segs", [(2, 110), (2, 250), (3, 500)])
+@pytest.mark.parametrize("what", ["want_area", "want_relate"])
+def test_wide_keys(ctx, k, segs, what):
+    R = gsj.subdivide(gsj.generate("regions_grid", nx=30, ny=30, kx=k, ky=k, edge_segs=segs, seed=segs), 8)
+    P = gsj.subdivide(gsj.generate("parcels_grid", nx=30, ny=30, seed=segs, kmin=9, kmax=30), 8)
+    assert R.parent[-1] < P.parent[-1] and P.n > P.parent[-1] + 1
+    last = int(R.parent[-1])
+    for bits in (62, 64, 66):
+        half = (bits - _key_bits(_renumbered(R, 1), _renumbered(R, 1))) // 2 + _bits(last)
+        S = _renumbered(R, 2 ** (half - 1) // last + 1)
+        assert _key_bits(S, S) == bits
+        assert (_folded(ctx, S, S, True) > FOLD_MAX) == (segs > 110)
+        _check(ctx, S, S, True, what, (False, True) if segs == 110 else (False,))
+    narrow = max(q for q in range(9, 28) if _key_bits(_renumbered(P, 2 ** (q - 9)), _renumbered(R, 2**q)) <= 63)
+    for q in (narrow, narrow + 1):
+        _check(ctx, _renumbered(P, 2 ** (q - 9)), _renumbered(R, 2**q), False, what)

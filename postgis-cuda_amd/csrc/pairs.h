@@ -302,8 +302,9 @@ enum PairClass : int { CL_TINY = 0, CL_SMALL = 1, CL_MEDIUM = 2, CL_MIXED = 3, C
 // Candidate pairs split by work class, on the device: list[0 .. counts[0]) the tiny pairs (both polygons within tcap
 // / RCAP; none when tcap is 0), then counts[1] small pairs (both within VCAP / RCAP), counts[2] medium pairs (both
 // within mcap / RCAP; none when mcap is 0), counts[3] mixed pairs (with `mixed`: one polygon within VCAP vertices),
-// then the counts[4] others; within a class by mean vertex count, then candidate order; ctl cleared for the overflow
-// queue. counts[8 ..) is left zeroed for the callers' queues.
+// then the counts[4] others; within a class by mean vertex count, then about in candidate order (k_part_scatter; a
+// launch of one block, up to 16384 pairs, keeps it only between runs of up to 1024); ctl cleared for the overflow queue.
+// counts[8 .. 11) is left zeroed for the callers' queues, counts[11 .. 14) holds the first three classes' list positions.
 // Uses the context's s_keys, s_vals, s_tmp2 and s_misc scratch (the list lives in s_vals until its next use).
 struct PairClasses {
   uint32_t* list;
@@ -312,7 +313,7 @@ struct PairClasses {
   uint64_t* start;   // [0] the partition's start time (wall_clock64); the words behind it are for the launches that follow
 };
 // size_sort: within a class, pairs of similar size side by side, in buckets 2^(size_sort-1) times the class's base
-// width (0: candidate order, a probe's pairs together); done (or null): the candidates whose byte is set are in no class
+// width (0: about candidate order, a probe's pairs together); done (or null): the candidates whose byte is set are in no class
 // (they come last in the list)
 PairClasses partition_pairs(Context& c, const DPolys& P, const DPolys& R, const uint32_t* pa, const uint32_t* pb, uint64_t np, uint32_t mcap,
                             bool mixed, uint32_t tcap, uint32_t size_sort = 1, const uint8_t* done = nullptr);

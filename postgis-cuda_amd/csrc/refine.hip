@@ -1357,9 +1357,10 @@ __device__ __forceinline__ uint32_t class_key(uint32_t ia, uint32_t ib, uint32_t
 }
 // The keys, their sort and the class sizes in one block, for at most PART_MAX pairs: wave w takes the w-th run of the
 // candidates and counts its keys (256 of them) in LDS; once the counts are scanned over (key, wave), every candidate
-// knows its place: the order of the sort but for candidates that the same wave counted in the same instruction. Two
-// counters per wave and key, by the lane's parity, halve the same-address chains (a few keys hold most pairs).
-// 10.6k pairs: one launch of 14 us (24 us as a stable sort with ranks from ballots) instead of six launches.
+// knows its place. Two counters per wave and key, by the lane's parity, halve the same-address chains (a few keys hold
+// most pairs: 10.6k pairs 19 -> 15 us), so of one key and wave, a run of up to 1024 candidates, the even lanes' come first:
+// at this size the whole launch's pieces stay in cache, whatever the order.
+// 10.6k pairs: one launch of 15 us (24 us as a stable sort with ranks from ballots) instead of six launches.
 constexpr int PART_T = 1024, PART_MAX = 16384, PART_ITEMS = PART_MAX / PART_T;
 __global__ void __launch_bounds__(PART_T) k_partition_small(const DPolys P, const DPolys R, const uint32_t* __restrict__ pa, const uint32_t* __restrict__ pb,
                                                             const uint8_t* __restrict__ done, uint32_t np, uint32_t mcap, int mixed, uint32_t tcap,
@@ -1442,15 +1443,18 @@ __global__ void __launch_bounds__(PART_T) k_partition_small(const DPolys P, cons
 
 // The same for more pairs, as one 8-bit pass over tiles of TILE_PAIRS: the keys (a byte per candidate) and every tile's
 // counts, their scan in (key, tile) order, and the scatter, which also leaves the class sizes (a class starts where its
-// first key's first tile does) and clears what the callers' queues need at 0. 215k pairs: 45 us; the 64-bit radix pass
-// with its own kernels for keys, class sizes (a binary search: 15 us) and clearing took 105.
-constexpr int TILE_T = 256, TILE_ITEMS = 16, TILE_PAIRS = TILE_T * TILE_ITEMS, TILE_COLS = TILE_T / 64 * 2;
+// first key's first tile does) and clears what the callers' queues need at 0. One counter per wave and key: of one key
+// the list keeps the candidates' order, but for the 64 that a wave counts in one instruction, so that a probe's pairs
+// stay together (300k self dwithin, in candidate order: with two counters by the lane's parity the scatter takes as long
+// and the list kernels 1% longer). 215k pairs: 45 us; the 64-bit radix pass with its own kernels for keys, class sizes
+// (a binary search: 15 us) and clearing took 105.
+constexpr int TILE_T = 256, TILE_ITEMS = 16, TILE_PAIRS = TILE_T * TILE_ITEMS, TILE_COLS = TILE_T / 64;
 __global__ void __launch_bounds__(TILE_T) k_part_count(const DPolys P, const DPolys R, const uint32_t* __restrict__ pa, const uint32_t* __restrict__ pb,
                                                        const uint8_t* __restrict__ done, uint64_t np, uint32_t mcap, int mixed, uint32_t tcap,
                                                        uint32_t size_sort, uint8_t* __restrict__ keys, uint32_t ntiles, uint32_t* __restrict__ ghist,
                                                        OverflowCtl* ctl, uint64_t* start) {
   __shared__ uint32_t hist[TILE_COLS][256];
-  const int t = threadIdx.x, col = (t >> 6) * 2 + (t & 1);
+  const int t = threadIdx.x, col = t >> 6;
   const uint64_t base = (uint64_t)blockIdx.x * TILE_PAIRS;
   if (blockIdx.x == 0 && t < 5) ctl[t] = OverflowCtl{0, 0, 0, 0};
   if (blockIdx.x == 0 && t == 0) *start = wall_clock64();
@@ -1481,11 +1485,11 @@ __global__ void __launch_bounds__(TILE_T) k_part_count(const DPolys P, const DPo
   for (int c = 0; c < TILE_COLS; c++) sum += hist[c][t];
   ghist[(uint64_t)t * ntiles + blockIdx.x] = sum;
 }
-// wave w of a tile takes its w-th run of 64 TILE_ITEMS candidates, so that its list order follows the candidates'
+// wave w of a tile takes its w-th run of 64 TILE_ITEMS candidates, 64 at a time in order
 __global__ void __launch_bounds__(TILE_T) k_part_scatter(const uint8_t* __restrict__ keys, uint64_t np, uint32_t ntiles, const uint32_t* __restrict__ goff,
                                                          uint32_t* __restrict__ list, uint32_t* __restrict__ counts) {
   __shared__ uint32_t hist[TILE_COLS][256];
-  const int t = threadIdx.x, lane = t & 63, w = t >> 6, col = 2 * w + (t & 1);
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
   const uint64_t base = (uint64_t)blockIdx.x * TILE_PAIRS + (uint64_t)w * 64 * TILE_ITEMS + lane;
   uint32_t key[TILE_ITEMS], rank[TILE_ITEMS];
 #pragma unroll
@@ -1499,7 +1503,7 @@ __global__ void __launch_bounds__(TILE_T) k_part_scatter(const uint8_t* __restri
   __syncthreads();
 #pragma unroll
   for (int j = 0; j < TILE_ITEMS; j++)
-    if (key[j] < 256) rank[j] = atomicAdd(&hist[col][key[j]], 1u);
+    if (key[j] < 256) rank[j] = atomicAdd(&hist[w][key[j]], 1u);
   __syncthreads();
   uint32_t at = goff[(uint64_t)t * ntiles + blockIdx.x];
 #pragma unroll
@@ -1507,7 +1511,7 @@ __global__ void __launch_bounds__(TILE_T) k_part_scatter(const uint8_t* __restri
   __syncthreads();
 #pragma unroll
   for (int j = 0; j < TILE_ITEMS; j++)
-    if (key[j] < 256) list[hist[col][key[j]] + rank[j]] = (uint32_t)(base + j * 64);
+    if (key[j] < 256) list[hist[w][key[j]] + rank[j]] = (uint32_t)(base + j * 64);
 }
 
 // the overflow queue's control at ctl, the host-read queue's (ovf_lds 2) right after it, the promotion queue's 64 bytes on

@@ -408,7 +408,7 @@ def test_budget_admits_windowed_requests_by_their_windows(ctx):
     """Under a scratch budget a windowed request is estimated from the probes of the tiles its window meets, not from
     the whole layer: two small windows fit the budget together and run side by side; two windows covering the layer
     do not, so the second waits until the first has finished (each still runs: a request alone is always admitted)."""
-    import time
+    import threading
 
     hs = _mesh(150, 4)
     L = ctx.polys(hs)
@@ -418,24 +418,18 @@ def test_budget_admits_windowed_requests_by_their_windows(ctx):
     full = [(x0, y0, x1, y1)] * 2
     s = gsj.Scheduler(ctx, lanes=2, scratch_budget=16 << 20, batch=1)   # small windows ~5 MB each, full ~22 MB
 
-    def spans(wins):
-        t_sub, tickets = [], []
-        for w in wins:
-            t_sub.append(time.perf_counter())
-            tickets.append(s.submit(gsj.REQ_JOIN, L, L, want_relate=True, upper=True, window=w))
-        res = [s.wait(t) for t in tickets]
-        assert all(len(r.pairs) > 0 for r in res)
-        return [(t + r.stats["times"]["queue_ms"] / 1e3, t + (r.stats["times"]["queue_ms"] + r.stats["times"]["run_ms"]) / 1e3)
-                for t, r in zip(t_sub, res)]
+    def second_ends_first(wins, wait_s):
+        """whether the second request ends while the first still holds its lane and its scratch (its done callback waits for
+        the second's, up to wait_s): a request takes some 0.3 ms, too little to compare start and end times"""
+        second, seen = threading.Event(), []
+        tickets = [s.submit(gsj.REQ_JOIN, L, L, want_relate=True, upper=True, window=wins[0], on_done=lambda: seen.append(second.wait(wait_s))),
+                   s.submit(gsj.REQ_JOIN, L, L, want_relate=True, upper=True, window=wins[1], on_done=second.set)]
+        assert all(len(s.wait(t).pairs) > 0 for t in tickets)
+        return seen[0]
 
     try:
-        # side by side: admitted together, so overlapping unless the first ends before the second is even submitted
-        # (a request takes ~2 ms here); five tries
-        small_runs = [spans(small) for _ in range(5)]
-        assert any(b0 < a1 for (a0, a1), (b0, b1) in small_runs), small_runs
-        # one after the other, every time: admission holds the second until the first has released its scratch
-        for _ in range(3):
-            (a0, a1), (b0, b1) = spans(full)
-            assert b0 >= a1 - 2e-4, (a0, a1, b0, b1)
+        assert all(second_ends_first(small, 20.0) for _ in range(3))   # side by side
+        # one after the other: admission holds the second until the first has released its scratch
+        assert not any(second_ends_first(full, 0.2) for _ in range(3))
     finally:
         s.close()

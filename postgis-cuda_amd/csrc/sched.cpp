@@ -42,8 +42,8 @@ struct Req {
 // (pairs, flags, areas, evidence, partition lists, compaction keys) and, where distances are reported, 136 B more (two
 // queued items of 68 B, at most 2^25 of them), plus per-probe traversal counters. Measured beyond the search's own, a
 // candidate takes 23 to 35 B (points in polygons), 56 to 88 (distance joins; 212 to 259 with distances), 92 to 180 (joins
-// with areas or codes) and 103 (erosion; 350 subdivided), the larger of two figures with subdivided layers or codes; the
-// layers here have 4 candidates a probe where 8 are assumed. The probes are
+// with areas or codes) and 103 (erosion; 350 subdivided), the larger of two figures with subdivided layers or codes; a
+// parcel mesh has 4 candidates a probe where 8 are assumed. The probes are
 // the probe layer's, or for a window over a layer with tile boxes, the probes of the tiles meeting the window. Points in
 // polygons count their rows per point of the layer (12 B each).
 uint64_t estimate_scratch(const gsj_request& r) {

@@ -135,6 +135,9 @@ struct StreamTimer {
 
 inline uint32_t div_up(uint64_t a, uint64_t b) { return (uint32_t)((a + b - 1) / b); }
 
+inline dim3 item_blocks(uint64_t n, uint32_t lanes) { const ItemGrid g = item_grid(n, lanes); return dim3(g.x, g.y); }
+__device__ __forceinline__ uint64_t flat_block() { return (uint64_t)blockIdx.y * gridDim.x + blockIdx.x; }
+
 // MI355X dispatches the workgroups of a grid round-robin over its 8 XCDs, each with its own L2. This renumbers them
 // (a bijection on [0, gridDim.x)) so that each XCD runs one contiguous range of logical blocks: neighbouring work
 // items, which read the same polygons and tree nodes, then share an L2. For work of even cost per item (the tree

@@ -638,19 +638,19 @@ __device__ bool er_witness(const DPolys& P, uint32_t a, double ra_nom, double rb
 __global__ void __launch_bounds__(256) k_erode_witness(const DPolys P, const uint32_t* __restrict__ pairs, uint32_t np, const ErRadii rr,
                                                        uint8_t* __restrict__ flag, uint32_t* __restrict__ rest, ErCtl* rest_ctl) {
   constexpr int G = 16;
+  const uint64_t k = (flat_block() * blockDim.x + threadIdx.x) / G;
   const int lane = threadIdx.x % G;
-  for (uint64_t k = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) / G; k < np; k += (uint64_t)gridDim.x * blockDim.x / G) {
-    const uint32_t p = (uint32_t)k, a = pairs[2 * k];
-    bool hit = false;
-    if (a == pairs[2 * k + 1] && (P.ginfo[a] & 0xFFFFu) <= WITNESS_VERTS) {
-      double ra, rb;
-      radii_of(rr, p, ra, rb);
-      hit = er_witness<G>(P, a, ra, rb, lane);
-    }
-    if (lane == 0) {
-      flag[p] = hit ? 1 : 0;
-      if (!hit) rest[atomicAdd(&rest_ctl->n, 1u)] = p;
-    }
+  if (k >= np) return;   // (a group's lanes leave together)
+  const uint32_t p = (uint32_t)k, a = pairs[2 * k];
+  bool hit = false;
+  if (a == pairs[2 * k + 1] && (P.ginfo[a] & 0xFFFFu) <= WITNESS_VERTS) {
+    double ra, rb;
+    radii_of(rr, p, ra, rb);
+    hit = er_witness<G>(P, a, ra, rb, lane);
+  }
+  if (lane == 0) {
+    flag[p] = hit ? 1 : 0;
+    if (!hit) rest[atomicAdd(&rest_ctl->n, 1u)] = p;
   }
 }
 
@@ -828,39 +828,39 @@ __global__ void k_er_filter(const uint32_t* __restrict__ rows, const double* __r
 __global__ void __launch_bounds__(256) k_self_overlap(const DPolys P, const uint32_t* __restrict__ pa, const uint32_t* __restrict__ pb, uint64_t np,
                                                       const ErRadii rr, uint8_t* __restrict__ done, const RefineOut out) {
   constexpr int G = 16;
+  const uint64_t i = (flat_block() * blockDim.x + threadIdx.x) / G;
   const int lane = threadIdx.x % G;
-  for (uint64_t i = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) / G; i < np; i += (uint64_t)gridDim.x * blockDim.x / G) {
-    const uint32_t g = pa[i];
-    bool settled = false;
-    double area = 0;
-    if (g == pb[i]) {
-      double s = 0, sabs = 0;
-      const uint32_t r1 = P.gro[g + 1];
-      for (uint32_t r = P.gro[g]; r < r1; r++) {
-        const uint64_t e = P.rvo[r + 1];
-        for (uint64_t v = P.rvo[r] + lane; v + 1 < e; v += G) {
-          const double2 p = P.xy[v], q = P.xy[v + 1];
-          const double c = p.x * q.y - q.x * p.y;
-          s += c;
-          sabs += fabs(c);
-        }
+  if (i >= np) return;   // (a group's lanes leave together)
+  const uint32_t g = pa[i];
+  bool settled = false;
+  double area = 0;
+  if (g == pb[i]) {
+    double s = 0, sabs = 0;
+    const uint32_t r1 = P.gro[g + 1];
+    for (uint32_t r = P.gro[g]; r < r1; r++) {
+      const uint64_t e = P.rvo[r + 1];
+      for (uint64_t v = P.rvo[r] + lane; v + 1 < e; v += G) {
+        const double2 p = P.xy[v], q = P.xy[v + 1];
+        const double c = p.x * q.y - q.x * p.y;
+        s += c;
+        sabs += fabs(c);
       }
+    }
 #pragma unroll
-      for (int o = G / 2; o > 0; o >>= 1) { s += __shfl_xor(s, o, G); sabs += __shfl_xor(sabs, o, G); }
-      area = 0.5 * s;
-      double ra, rb;
-      radii_of(rr, i, ra, rb);
-      const double rmin = disk_radius(ra, rb);
-      const double y0 = P.origin[g].y;
-      double a_m2, need, t_m2;
-      area_bound(area, y0, y0 + P.ext[g].y, rmin, a_m2, need);
-      area_bound(0.5 * sabs, y0, y0 + P.ext[g].y, rmin, t_m2, need);
-      settled = rmin >= 0 && sabs > 0 && fabs(a_m2 - (rmin > 0 ? need : 0.0)) > 1e-6 * (need + t_m2);
-    }
-    if (lane == 0) {
-      done[i] = settled ? 1 : 0;
-      if (settled) { out.isect[i] = 1; out.area[i] = area; }
-    }
+    for (int o = G / 2; o > 0; o >>= 1) { s += __shfl_xor(s, o, G); sabs += __shfl_xor(sabs, o, G); }
+    area = 0.5 * s;
+    double ra, rb;
+    radii_of(rr, i, ra, rb);
+    const double rmin = disk_radius(ra, rb);
+    const double y0 = P.origin[g].y;
+    double a_m2, need, t_m2;
+    area_bound(area, y0, y0 + P.ext[g].y, rmin, a_m2, need);
+    area_bound(0.5 * sabs, y0, y0 + P.ext[g].y, rmin, t_m2, need);
+    settled = rmin >= 0 && sabs > 0 && fabs(a_m2 - (rmin > 0 ? need : 0.0)) > 1e-6 * (need + t_m2);
+  }
+  if (lane == 0) {
+    done[i] = settled ? 1 : 0;
+    if (settled) { out.isect[i] = 1; out.area[i] = area; }
   }
 }
 __global__ void k_compact_rows(const uint32_t* __restrict__ rows, const uint32_t* __restrict__ keep, const uint64_t* __restrict__ off, uint64_t n,
@@ -880,7 +880,7 @@ const uint8_t* decide_self(Context& c, const DPolys& P, const DPolys& R, bool sn
                            const RefineOut& out) {
   if (snap || P.xy != R.xy || P.pfirst || R.pfirst || !out.area) return nullptr;
   uint8_t* done = c.s_er_flag.as<uint8_t>(np + 16);
-  hipLaunchKernelGGL(k_self_overlap, dim3(stride_blocks(np, 16)), dim3(256), 0, c.stream, P, pa, pb, np, rr, done, out);
+  hipLaunchKernelGGL(k_self_overlap, item_blocks(np, 16), dim3(256), 0, c.stream, P, pa, pb, np, rr, done, out);
   GSJ_LAUNCHED();
   return done;
 }
@@ -927,7 +927,7 @@ uint64_t erode_pass2(Context& c, const DPolys& P, const DPolys& R, const uint32_
   const uint32_t g = (uint32_t)std::min<uint64_t>(div_up(ne, ER_WAVES), (uint64_t)c.cu_count * 32);
   const uint32_t* items = nullptr;
   if (same && !pfP && !pfR && P.xy == R.xy) {
-    hipLaunchKernelGGL(k_erode_witness, dim3(stride_blocks(ne, 16)), dim3(256), 0, stream, P, ep, (uint32_t)ne, rr, flag, list(3), ctl_pairs);
+    hipLaunchKernelGGL(k_erode_witness, item_blocks(ne, 16), dim3(256), 0, stream, P, ep, (uint32_t)ne, rr, flag, list(3), ctl_pairs);
     GSJ_LAUNCHED();
     items = list(3);
   }

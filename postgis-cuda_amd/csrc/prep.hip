@@ -25,27 +25,26 @@ inline int dd_hash_bits(uint64_t n) {
 }
 __global__ void k_dd_hash(const uint64_t* __restrict__ gro, const uint64_t* __restrict__ rvo, const double* __restrict__ xy, uint64_t n,
                           int bits, uint64_t* __restrict__ h, uint32_t* __restrict__ idx) {
+  const uint64_t g = (flat_block() * blockDim.x + threadIdx.x) >> 3;
+  if (g >= n) return;
   const uint32_t lane = threadIdx.x & 7;
+  const uint64_t r0 = gro[g], r1 = gro[g + 1], w0 = 2 * rvo[r0], nw = 2 * rvo[r1] - w0;
   auto mix = [](uint64_t v) {
     v *= 0xBF58476D1CE4E5B9ull;
     v ^= v >> 32;
     return v * 0x94D049BB133111EBull;
   };
-  for (uint64_t g = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 3; g < n; g += (uint64_t)gridDim.x * blockDim.x >> 3) {
-    const uint64_t r0 = gro[g], r1 = gro[g + 1], w0 = 2 * rvo[r0], nw = 2 * rvo[r1] - w0;
-    const unsigned long long* w = reinterpret_cast<const unsigned long long*>(xy) + w0;
-    uint64_t v = 0;
-    for (uint64_t r = r0 + lane; r < r1; r += 8) v += mix((rvo[r + 1] - rvo[r]) ^ (r - r0 + 1) * 0xD6E8FEB86659FD93ull);
+  const unsigned long long* w = reinterpret_cast<const unsigned long long*>(xy) + w0;
+  uint64_t v = 0;
+  for (uint64_t r = r0 + lane; r < r1; r += 8) v += mix((rvo[r + 1] - rvo[r]) ^ (r - r0 + 1) * 0xD6E8FEB86659FD93ull);
 #pragma unroll 4
-    for (uint64_t k = lane; k < nw; k += 8) v += mix(w[k] ^ (k + 1) * 0x9E3779B97F4A7C15ull);
+  for (uint64_t k = lane; k < nw; k += 8) v += mix(w[k] ^ (k + 1) * 0x9E3779B97F4A7C15ull);
 #pragma unroll
-    for (int s = 4; s > 0; s >>= 1) v += __shfl_xor((unsigned long long)v, s, 8);
-    v ^= v >> 29;
-    if (lane == 0) {
-      h[g] = v >> (64 - bits);
-      idx[g] = (uint32_t)g;
-    }
-  }
+  for (int s = 4; s > 0; s >>= 1) v += __shfl_xor((unsigned long long)v, s, 8);
+  v ^= v >> 29;
+  if (lane) return;
+  h[g] = v >> (64 - bits);
+  idx[g] = (uint32_t)g;
 }
 
 __device__ bool dd_same(const uint64_t* gro, const uint64_t* rvo, const double* xy, uint64_t a, uint64_t b) {
@@ -125,10 +124,10 @@ __global__ void k_dd_rings(const uint64_t* __restrict__ gro, const uint64_t* __r
 // (eight lanes per ring: their copies are runs of cache lines)
 __global__ void k_dd_copy(const uint64_t* __restrict__ rvo, const double2* __restrict__ xy, const uint64_t* __restrict__ src,
                           const uint64_t* __restrict__ urvo, uint64_t nur, double2* __restrict__ uxy) {
-  for (uint64_t k = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 3; k < nur; k += (uint64_t)gridDim.x * blockDim.x >> 3) {
-    const uint64_t r = src[k], a = rvo[r], m = rvo[r + 1] - a, o = urvo[k];
-    for (uint64_t j = threadIdx.x & 7; j < m; j += 8) uxy[o + j] = xy[a + j];
-  }
+  const uint64_t k = (flat_block() * blockDim.x + threadIdx.x) >> 3;
+  if (k >= nur) return;
+  const uint64_t r = src[k], a = rvo[r], m = rvo[r + 1] - a, o = urvo[k];
+  for (uint64_t j = threadIdx.x & 7; j < m; j += 8) uxy[o + j] = xy[a + j];
 }
 
 template <class T>
@@ -161,7 +160,7 @@ HostSet dedup_device(Context& c, const uint64_t* gro, const uint64_t* rvo, const
   uint32_t* ord = b_idx.as<uint32_t>(n);
   uint32_t* ord2 = b_idx2.as<uint32_t>(n);
   const int bits = dd_hash_bits(n);
-  hipLaunchKernelGGL(k_dd_hash, dim3(stride_blocks(n, 8)), dim3(256), 0, st, dgro, drvo, dxy, n, bits, h, ord);
+  hipLaunchKernelGGL(k_dd_hash, item_blocks(n, 8), dim3(256), 0, st, dgro, drvo, dxy, n, bits, h, ord);
   GSJ_LAUNCHED();
   radix_sort_pairs(c, h, h2, ord, ord2, n, 0, bits);   // stable: a hash group in index order
   uint32_t* head = b_head.as<uint32_t>(n + 16);
@@ -204,7 +203,7 @@ HostSet dedup_device(Context& c, const uint64_t* gro, const uint64_t* rvo, const
   GSJ_LAUNCHED();
   const uint64_t unv = scan_u32_to_u64(c, nvert, urvo, nur);
   double2* uxy = b_uxy.as<double2>(unv + 1);
-  hipLaunchKernelGGL(k_dd_copy, dim3(stride_blocks(nur, 8)), dim3(256), 0, st, drvo, reinterpret_cast<const double2*>(dxy), src, urvo, nur, uxy);
+  hipLaunchKernelGGL(k_dd_copy, item_blocks(nur, 8), dim3(256), 0, st, drvo, reinterpret_cast<const double2*>(dxy), src, urvo, nur, uxy);
   GSJ_LAUNCHED();
   u.gro.resize(un + 1);
   u.rvo.resize(nur + 1);
@@ -445,14 +444,13 @@ __global__ void k_sd_out_rings(const uint32_t* __restrict__ order, const uint32_
 }
 __global__ void k_sd_out_copy(const uint32_t* __restrict__ rlev, const uint32_t* __restrict__ rsrc, const uint64_t* __restrict__ orvo, uint64_t nr,
                               SdLevelPtrs lv, double2* __restrict__ oxy, uint8_t* __restrict__ osyn) {
-  // eight lanes per ring
-  for (uint64_t k = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 3; k < nr; k += (uint64_t)gridDim.x * blockDim.x >> 3) {
-    const uint32_t l = rlev[k], r = rsrc[k];
-    const uint64_t a = lv.rg_off[l][r], n = lv.rg_n[l][r], o = orvo[k];
-    for (uint64_t j = threadIdx.x & 7; j < n; j += 8) {
-      oxy[o + j] = lv.pool[l][a + j];
-      osyn[o + j] = lv.syn[l] ? lv.syn[l][a + j] : 0;
-    }
+  const uint64_t k = (flat_block() * blockDim.x + threadIdx.x) >> 3;   // eight lanes per ring
+  if (k >= nr) return;
+  const uint32_t l = rlev[k], r = rsrc[k];
+  const uint64_t a = lv.rg_off[l][r], n = lv.rg_n[l][r], o = orvo[k];
+  for (uint64_t j = threadIdx.x & 7; j < n; j += 8) {
+    oxy[o + j] = lv.pool[l][a + j];
+    osyn[o + j] = lv.syn[l] ? lv.syn[l][a + j] : 0;
   }
 }
 __global__ void k_sd_parent(const uint64_t* __restrict__ key, uint64_t np, uint32_t* __restrict__ parent) {
@@ -608,7 +606,7 @@ HostSet subdivide_device(Context& c, const uint64_t* gro, const uint64_t* rvo, c
   double2* oxy = b_oxy.as<double2>(onv + 1);
   uint8_t* osyn = b_osyn.as<uint8_t>(onv + 1);
   uint32_t* par = b_par.as<uint32_t>(npieces + 1);
-  if (onrings) hipLaunchKernelGGL(k_sd_out_copy, dim3(stride_blocks(onrings, 8)), dim3(256), 0, st, rlev, rsrc, orvo, onrings, lv, oxy, osyn);
+  if (onrings) hipLaunchKernelGGL(k_sd_out_copy, item_blocks(onrings, 8), dim3(256), 0, st, rlev, rsrc, orvo, onrings, lv, oxy, osyn);
   hipLaunchKernelGGL(k_sd_parent, dim3(div_up(npieces, 256)), dim3(256), 0, st, key, npieces, par);
   GSJ_LAUNCHED();
   o.gro.resize(npieces + 1);

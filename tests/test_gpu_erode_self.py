@@ -101,8 +101,8 @@ def test_a_mesh_of_every_size(ctx):
         assert np.array_equal(sorted_rows(got.pairs)[0], sorted_rows(exp["pairs"])[0])
 
 
-def test_more_pairs_than_one_round_of_blocks(ctx):
-    # 8200 boxes on one spot: 67.2M candidates, the last of them in the blocks' second round; every pair meets
+def test_more_pairs_than_one_row_of_blocks(ctx):
+    # 8200 boxes on one spot: 67.2M candidates, the last of them in the grid's second row; every pair meets
     n = 8200
     box = _box(0, 0, 30, 20)
     hs = gsj.HostSet(np.arange(n + 1, dtype=np.uint64), 5 * np.arange(n + 1, dtype=np.uint64), np.tile(box, (n, 1)))

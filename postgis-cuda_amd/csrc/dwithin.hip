@@ -190,7 +190,7 @@ __device__ __forceinline__ uint64_t near_mask(const Ed* L, int base, int n, doub
 }
 
 // The geography distances of the reported rows, put off to a kernel of their own. A pair's distance is the minimum of
-// the geography distances of the edge pairs that could hold it: a few of them per pair, each thousands of FP64
+// the geography distances of the edge pairs that could hold it: a few of them per pair, each some 2200 FP64
 // operations. Evaluated where they are found, one or two lanes of a group worked while its others waited; queued, they
 // fill whole waves (k_geog_items), and the pair kernels are left with the frame tests (300k parcels, 5 m self dwithin
 // with distances: the vertex-list classes 17.9 -> 3.0 ms, the items 0.34, the request 20.3 -> 5.1). The minimum does not depend on the
